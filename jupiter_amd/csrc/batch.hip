@@ -10,12 +10,13 @@
 // query's uint64 slot.  Clique roots with out-degree up to the hub threshold
 // (64 or 128, a tuning knob) run inside the wave (one- or two-word bitmap rows
 // in LDS); the few wider roots of a query run afterwards in the block-per-root
-// tier kernels, into the same slot, and 4-cycle (P1) queries run afterwards as
-// wedge launches (one wave per root), also into their slots.  All launches of a batch can be captured
+// tier kernels, into the same slot, and every 4-cycle (P1) query of the batch
+// runs in one sequence of wedge launches, also into its slot.  All launches of a batch can be captured
 // once in a HIP graph (prepared batches) and replayed.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstring>
 #include <numeric>
 #include <vector>
 
@@ -172,8 +173,7 @@ struct BatchBufs {
   int64_t sscr_stride = 1;
   uint64_t* gscr = nullptr;             // global-row tier scratch (nullptr: the context's)
   size_t gscr_words = 0;
-  int32_t* p1cnt = nullptr;             // zeroed wedge counters of the 4-cycle launches
-  size_t p1cnt_ints = 0;
+  void* p1 = nullptr;                   // scratch of the 4-cycle launches
 };
 
 __global__ void k_zero_u64(uint64_t* p, int n) {
@@ -196,18 +196,26 @@ static int batch_grid(jgpm_ctx_s* c) {
   return std::min(want, c->batch_occ) * c->num_cu;
 }
 
+// 64-bit words of the batch table for n queries: the chunk prefix (n + 1),
+// then for the 4-cycle queries (at most n) their descriptors and the prefixes
+// of their edge tiles and roots.
+constexpr size_t P1Q_WORDS = sizeof(jk::P1Q) / sizeof(int64_t);
+static_assert(sizeof(jk::P1Q) % sizeof(int64_t) == 0, "4-cycle descriptors are copied as 64-bit words");
+static size_t table_words(int n) { return (size_t)(n + 1) + (size_t)n * P1Q_WORDS + 2 * (size_t)(n + 1); }
+
 // Host side of a batch: the query table (work items sized by the tuning),
-// its chunk prefix and the list-scratch stride.  May build a graph's lazy
-// auxiliary arrays on st (kernels and allocations), so it is never captured.
+// its chunk prefix, the 4-cycle queries' descriptors and prefixes (pa.nq of
+// them, behind the chunk prefix in cs; pa holds their totals) and the
+// list-scratch stride.  May build a graph's lazy auxiliary arrays on st
+// (kernels and allocations), so it is never captured.
 static int plan_batch(jgpm_ctx_s* c, const jgpm_query* q, int n, std::vector<jk::BQ>& hq, std::vector<int64_t>& cs,
-                      int32_t& max_sym, size_t& p1_ints, hipStream_t st) {
-  // cs holds two prefixes of n + 1 entries: the persistent kernel's chunks,
-  // then the roots of the 4-cycle queries (one batched wedge launch)
+                      int32_t& max_sym, jk::P1Args& pa, hipStream_t st) {
+  std::vector<jk::P1Q> p1;
+  pa = jk::P1Args{};
   const int rchunk = std::max(1, c->tune.batch_root_chunk);
   const int echunk = std::max(1, c->tune.batch_edge_chunk);
   hq.assign(n, jk::BQ{});
   max_sym = 1;
-  p1_ints = 0;
   for (int i = 0; i < n; ++i) {
     jgpm_graph_s* g = q[i].graph;
     const int kind = batch_kind(q[i].pattern);
@@ -223,19 +231,19 @@ static int plan_batch(jgpm_ctx_s* c, const jgpm_query* q, int n, std::vector<jk:
       b.chunk = rchunk;
     } else if (kind == 101) {
       // 4-cycles run as wedge launches after the persistent kernel (no chunks here)
-      p1_ints = std::max(p1_ints, p1_counter_ints(c, (int32_t)g->sym.nv));
-      const bool whole = rb == 0 && re == g->sym.nv;
-      if (whole) {
-        int rc = ensure_rank_csr(g, st);
-        if (rc) return rc;
-      }
-      // a whole-graph count runs on the degree-ordered relabelling (same
-      // total, hubs ranked last), as the single-query launch does
-      b.rp = whole && g->rsym.ci ? g->rsym.rp : g->sym.rp;
-      b.ci = whole && g->rsym.ci ? g->rsym.ci : g->sym.ci;
-      b.base = rb;
       b.ntasks = 0;
       b.chunk = 1;
+      if (re <= rb) continue;
+      jk::P1Q w;
+      int rc = p1_query(g, rb, re, st, w);
+      if (rc) return rc;
+      w.slot = i;
+      w.eoff = pa.edges;
+      w.roff = pa.roots;
+      pa.edges += w.ne;
+      pa.roots += w.nr;
+      pa.max_nv = std::max(pa.max_nv, g->sym.nv);
+      p1.push_back(w);
     } else {
       const int p = kind - 100;
       // diamonds read the per-edge triangle array, as the single-query path does
@@ -252,25 +260,37 @@ static int plan_batch(jgpm_ctx_s* c, const jgpm_query* q, int n, std::vector<jk:
       max_sym = std::max(max_sym, g->sym_mmin);
     }
   }
-  cs.assign(2 * (size_t)(n + 1), 0);
+  pa.nq = (int)p1.size();
+  cs.assign((size_t)(n + 1) + p1.size() * P1Q_WORDS + 2 * (p1.size() + 1), 0);
   for (int i = 0; i < n; ++i) cs[i + 1] = cs[i] + (hq[i].ntasks + hq[i].chunk - 1) / hq[i].chunk;
-  int64_t* p1cs = cs.data() + n + 1;
-  for (int i = 0; i < n; ++i) {
-    int64_t r = 0;
-    if (hq[i].kind == 101) {
-      const jgpm_graph_s* g = q[i].graph;
-      r = (q[i].root_end < 0 ? g->sym.nv : q[i].root_end) - q[i].root_begin;
-    }
-    p1cs[i + 1] = p1cs[i] + r;
+  int64_t* w = cs.data() + n + 1;
+  if (!p1.empty()) std::memcpy(w, p1.data(), p1.size() * sizeof(jk::P1Q));
+  int64_t* tcs = w + p1.size() * P1Q_WORDS;
+  int64_t* rcs = tcs + p1.size() + 1;
+  for (size_t k = 0; k < p1.size(); ++k) {
+    tcs[k + 1] = tcs[k] + (p1[k].ne + 255) / 256;
+    rcs[k + 1] = rcs[k] + p1[k].nr;
   }
+  pa.tiles = tcs[p1.size()];
   return JGPM_OK;
+}
+
+// The 4-cycle launches' arguments once the table and the scratch have device
+// addresses.
+static void bind_p1(jk::P1Args& pa, int n, const BatchBufs& b) {
+  const int64_t* w = b.bcs + n + 1;
+  pa.q = reinterpret_cast<const jk::P1Q*>(w);
+  pa.tcs = w + (size_t)pa.nq * P1Q_WORDS;
+  pa.rcs = pa.tcs + pa.nq + 1;
+  pa.out = b.bcnt;
+  jk::p1_bind_scratch(pa, b.p1);
 }
 
 // Every launch of one batch, and nothing else (no allocation, host copy or
 // memset), so that the sequence can be captured: counter fills, the
 // persistent kernel, then the hub launches of each clique query into its slot.
 static int launch_batch(jgpm_ctx_s* c, const jgpm_query* q, int n, const std::vector<jk::BQ>& hq, const BatchBufs& b,
-                        int grid, hipStream_t st) {
+                        const jk::P1Args& pa, int grid, hipStream_t st) {
   hipLaunchKernelGGL(k_zero_u64, dim3((n + 255) / 256), dim3(256), 0, st, b.bcnt, n);
   hipLaunchKernelGGL(k_zero_u32, dim3((jk::NUM_TIERS * n + 255) / 256), dim3(256), 0, st, b.bq32, jk::NUM_TIERS * n);
   hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, reinterpret_cast<uint64_t*>(b.qctr), 1);
@@ -290,36 +310,12 @@ static int launch_batch(jgpm_ctx_s* c, const jgpm_query* q, int n, const std::ve
   prof_end(c, st);
   if (hipGetLastError() != hipSuccess) return JGPM_E_HIP;
   const int first_tier = hub <= 64 ? jk::TIER_LDS2 : jk::TIER_LDS4;
-  // every 4-cycle query in one wedge launch over their flattened roots
-  {
-    int first = -1;
-    int64_t total = 0;
-    int32_t max_nv = 1;
-    for (int i = 0; i < n; ++i)
-      if (hq[i].kind == 101) {
-        if (first < 0) first = i;
-        const jgpm_graph_s* g = q[i].graph;
-        total += (q[i].root_end < 0 ? g->sym.nv : q[i].root_end) - q[i].root_begin;
-        max_nv = std::max(max_nv, (int32_t)g->sym.nv);
-      }
-    if (total > 0) {
-      const int64_t waves = std::min<int64_t>((int64_t)c->num_cu * 32, (int64_t)(b.p1cnt_ints / (size_t)max_nv));
-      const int grid = (int)std::min<int64_t>(waves / jk::P1_WPB, (total + jk::P1_WPB - 1) / jk::P1_WPB);
-      if (!b.p1cnt || grid < 1) return JGPM_E_STATE;  // counters not sized for these graphs
-      jk::P1BatchArgs pa{};
-      pa.q = b.bq;
-      pa.p1cs = b.bcs + (n + 1);
-      pa.nq = n;
-      pa.total = total;
-      pa.qctr = b.bq32 + (size_t)jk::NUM_TIERS * first;  // zeroed above, unused by the wedge query otherwise
-      pa.cnt = b.p1cnt;
-      pa.cnt_stride = max_nv;
-      pa.counts = b.bcnt;
-      prof_begin(c, st, "batch_p1_wedge");
-      hipError_t e = jk::launch_p1_batch(pa, grid, st);
-      prof_end(c, st);
-      if (e != hipSuccess) return JGPM_E_HIP;
-    }
+  // every 4-cycle query in one sequence of wedge launches
+  if (pa.nq > 0) {
+    prof_begin(c, st, "batch_p1_wedge");
+    hipError_t e = jk::launch_p1(pa, c->num_cu, st);
+    prof_end(c, st);
+    if (e != hipSuccess) return JGPM_E_HIP;
   }
   for (int i = 0; i < n; ++i) {
     if (hq[i].kind >= 100) continue;
@@ -346,7 +342,7 @@ static int ensure_batch_buffers(jgpm_ctx_s* c, int n) {
   c->bcap = 0;
   int cap = std::max(64, n);
   if (hipMalloc(&c->d_bq, sizeof(jk::BQ) * cap) != hipSuccess ||
-      hipMalloc(&c->d_bcs, sizeof(int64_t) * 2 * (cap + 1)) != hipSuccess ||
+      hipMalloc(&c->d_bcs, sizeof(int64_t) * table_words(cap)) != hipSuccess ||
       hipMalloc(&c->d_bcnt, sizeof(uint64_t) * cap) != hipSuccess ||
       hipMalloc(&c->d_bq32, sizeof(unsigned) * jk::NUM_TIERS * cap) != hipSuccess)
     return JGPM_E_NOMEM;
@@ -362,10 +358,10 @@ int enqueue_batch(jgpm_ctx_s* c, const jgpm_query* q, int n, std::vector<jk::BQ>
   int rc = ensure_batch_buffers(c, n);
   if (rc) return rc;
   int32_t max_sym = 1;
-  size_t p1_ints = 0;
-  rc = plan_batch(c, q, n, hq, cs, max_sym, p1_ints, st);
+  jk::P1Args pa;
+  rc = plan_batch(c, q, n, hq, cs, max_sym, pa, st);
   if (rc) return rc;
-  if (p1_ints && (rc = ensure_p1_counters(c, p1_ints, st))) return rc;
+  if (pa.nq && (rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(pa.roots, pa.edges), st))) return rc;
   const int grid = batch_grid(c);
   const size_t need = (size_t)grid * jk::BWPB * jk::symd::NLIST * (size_t)max_sym;
   if (c->sscr_ints < need) {
@@ -377,19 +373,19 @@ int enqueue_batch(jgpm_ctx_s* c, const jgpm_query* q, int n, std::vector<jk::BQ>
     c->sscr_ints = need;
   }
   if (hipMemcpyAsync(c->d_bq, hq.data(), sizeof(jk::BQ) * n, hipMemcpyHostToDevice, st) != hipSuccess ||
-      hipMemcpyAsync(c->d_bcs, cs.data(), sizeof(int64_t) * 2 * (n + 1), hipMemcpyHostToDevice, st) != hipSuccess)
+      hipMemcpyAsync(c->d_bcs, cs.data(), sizeof(int64_t) * cs.size(), hipMemcpyHostToDevice, st) != hipSuccess)
     return JGPM_E_HIP;
   BatchBufs b;
   b.bq = static_cast<jk::BQ*>(c->d_bq);
   b.bcs = c->d_bcs;
   b.bcnt = c->d_bcnt;
-  b.p1cnt = c->d_p1cnt;
-  b.p1cnt_ints = c->p1cnt_ints;
+  b.p1 = c->d_p1;
   b.bq32 = c->d_bq32;
   b.qctr = c->d_q64 + (CTX_SLOTS - 2);
   b.sscr = c->d_sscr;
   b.sscr_stride = max_sym;
-  return launch_batch(c, q, n, hq, b, grid, st);
+  if (pa.nq) bind_p1(pa, n, b);
+  return launch_batch(c, q, n, hq, b, pa, grid, st);
 }
 
 int enqueue_batch_q(jgpm_ctx_s* c, const jgpm_query* q, int n, hipStream_t st) {
@@ -502,7 +498,7 @@ struct jgpm_batch_s {
 static void batch_release(jgpm_batch_s* B) {
   if (B->exec) (void)hipGraphExecDestroy(B->exec);
   if (B->graph) (void)hipGraphDestroy(B->graph);
-  void* bufs[] = {B->b.bq, B->b.bcs, B->b.bcnt, B->b.bq32, B->b.qctr, B->b.sscr, B->b.gscr, B->b.p1cnt};
+  void* bufs[] = {B->b.bq, B->b.bcs, B->b.bcnt, B->b.bq32, B->b.qctr, B->b.sscr, B->b.gscr, B->b.p1};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   for (const jgpm_query& x : B->q) x.graph->nbatch--;
@@ -533,8 +529,8 @@ extern "C" int jgpm_batch_create(jgpm_ctx_t ctx, const jgpm_query* q, int n, jgp
   };
   if (hipSetDevice(ctx->dev) != hipSuccess) return fail(JGPM_E_HIP);
   int32_t max_sym = 1;
-  size_t p1_ints = 0;
-  st = plan_batch(ctx, B->q.data(), n, B->hq, B->cs, max_sym, p1_ints, ctx->st);
+  jk::P1Args pa;
+  st = plan_batch(ctx, B->q.data(), n, B->hq, B->cs, max_sym, pa, ctx->st);
   if (st) return fail(st);
   B->grid = batch_grid(ctx);
   // global-row scratch only when a clique query has roots in that tier
@@ -550,20 +546,18 @@ extern "C" int jgpm_batch_create(jgpm_ctx_t ctx, const jgpm_query* q, int n, jgp
   const size_t sscr = (size_t)B->grid * jk::BWPB * jk::symd::NLIST * (size_t)max_sym;
   if (glb) B->b.gscr_words = jk::tier_scratch_words(jk::TIER_GLB32) * (size_t)glb_tier_grid(ctx);
   if (hipMalloc(&B->b.bq, sizeof(jk::BQ) * n) != hipSuccess ||
-      hipMalloc(&B->b.bcs, sizeof(int64_t) * 2 * (n + 1)) != hipSuccess ||
+      hipMalloc(&B->b.bcs, sizeof(int64_t) * B->cs.size()) != hipSuccess ||
       hipMalloc(&B->b.bcnt, sizeof(uint64_t) * n) != hipSuccess ||
       hipMalloc(&B->b.bq32, sizeof(unsigned) * jk::NUM_TIERS * n) != hipSuccess ||
       hipMalloc(&B->b.qctr, 64) != hipSuccess || hipMalloc(&B->b.sscr, sscr * sizeof(int32_t)) != hipSuccess ||
       (glb && hipMalloc(&B->b.gscr, B->b.gscr_words * sizeof(uint64_t)) != hipSuccess) ||
-      (p1_ints && hipMalloc(&B->b.p1cnt, p1_ints * sizeof(int32_t)) != hipSuccess))
+      // the batch's own 4-cycle scratch (a later context allocation cannot
+      // move it under the captured launches)
+      (pa.nq && hipMalloc(&B->b.p1, jk::p1_scratch_bytes(pa.roots, pa.edges)) != hipSuccess))
     return fail(JGPM_E_NOMEM);
-  // the batch's own wedge counters (a later context allocation cannot move
-  // them under the captured launches): zeroed once, left zero by every replay
-  B->b.p1cnt_ints = p1_ints;
-  if (p1_ints && hipMemsetAsync(B->b.p1cnt, 0, p1_ints * sizeof(int32_t), ctx->st) != hipSuccess)
-    return fail(JGPM_E_HIP);
+  if (pa.nq) bind_p1(pa, n, B->b);
   if (hipMemcpyAsync(B->b.bq, B->hq.data(), sizeof(jk::BQ) * n, hipMemcpyHostToDevice, ctx->st) != hipSuccess ||
-      hipMemcpyAsync(B->b.bcs, B->cs.data(), sizeof(int64_t) * 2 * (n + 1), hipMemcpyHostToDevice, ctx->st) !=
+      hipMemcpyAsync(B->b.bcs, B->cs.data(), sizeof(int64_t) * B->cs.size(), hipMemcpyHostToDevice, ctx->st) !=
           hipSuccess ||
       hipStreamSynchronize(ctx->st) != hipSuccess)
     return fail(JGPM_E_HIP);
@@ -577,7 +571,7 @@ extern "C" int jgpm_batch_create(jgpm_ctx_t ctx, const jgpm_query* q, int n, jgp
     ctx->capturing = false;
     return fail(JGPM_E_HIP);
   }
-  st = launch_batch(ctx, B->q.data(), n, B->hq, B->b, B->grid, ctx->st);
+  st = launch_batch(ctx, B->q.data(), n, B->hq, B->b, pa, B->grid, ctx->st);
   const hipError_t ce = hipStreamEndCapture(ctx->st, &B->graph);
   ctx->prof_on = prof;
   ctx->capturing = false;

@@ -61,58 +61,56 @@ static bool heavy_split_on(const jgpm_ctx_s* c, int p) {
 
 bool query_needs_tri(const jgpm_ctx_s* c, int p) { return p == 2 || pattern_uses_tri(p) || heavy_split_on(c, p); }
 
-// Waves of the 4-cycle wedge kernel on a graph of nv vertices: one dense
-// counter array of nv ints each, within 2 GiB, at most 32 waves per CU.
-static int64_t p1_waves(jgpm_ctx_s* c, int32_t nv) {
-  const int64_t budget = (int64_t)1 << 29;  // ints
-  const int64_t cap = (int64_t)c->num_cu * 32;
-  return std::max<int64_t>(jk::P1_WPB, std::min<int64_t>(cap, budget / std::max<int32_t>(nv, 1)));
-}
-
-size_t p1_counter_ints(jgpm_ctx_s* c, int32_t nv) { return (size_t)p1_waves(c, nv) * (size_t)std::max<int32_t>(nv, 1); }
-
-int ensure_p1_counters(jgpm_ctx_s* c, size_t need, hipStream_t st) {
-  if (c->p1cnt_ints >= need) return JGPM_OK;
+int ensure_p1_scratch(jgpm_ctx_s* c, size_t bytes, hipStream_t st) {
+  if (c->p1_bytes >= bytes) return JGPM_OK;
   if (c->capturing) return JGPM_E_STATE;
-  if (c->d_p1cnt) {
+  if (c->d_p1) {
     if (hipStreamSynchronize(st) != hipSuccess) return JGPM_E_HIP;
-    (void)hipFree(c->d_p1cnt);
-    c->d_p1cnt = nullptr;
-    c->p1cnt_ints = 0;
+    (void)hipFree(c->d_p1);
+    c->d_p1 = nullptr;
+    c->p1_bytes = 0;
   }
-  if (hipMalloc(&c->d_p1cnt, need * sizeof(int32_t)) != hipSuccess) return JGPM_E_NOMEM;
-  // zero once: every launch leaves the counters it touched at zero again
-  if (hipMemsetAsync(c->d_p1cnt, 0, need * sizeof(int32_t), st) != hipSuccess) return JGPM_E_HIP;
-  c->p1cnt_ints = need;
+  if (hipMalloc(&c->d_p1, bytes) != hipSuccess) return JGPM_E_NOMEM;
+  c->p1_bytes = bytes;
   return JGPM_OK;
 }
 
-int launch_p1(jgpm_graph_s* g, int64_t rb, int64_t re, uint64_t* out, unsigned* qctr, int32_t* cnt, size_t cnt_ints,
-              hipStream_t st) {
-  jgpm_ctx_s* c = exec_ctx(g);
-  const int32_t nv = (int32_t)g->sym.nv;
+int p1_query(jgpm_graph_s* g, int64_t rb, int64_t re, hipStream_t st, jk::P1Q& q) {
+  q = jk::P1Q{};
+  // a whole-graph count runs on the degree-ordered relabelling: the same
+  // identity in another vertex order gives the same total, and the hubs,
+  // ranked last, are no wedge's middle vertex
+  const bool whole = rb == 0 && re == g->sym.nv;
+  int rc = whole ? ensure_rank_csr(g, st) : ensure_sym_aux(g, false, false, st);
+  if (rc) return rc;
+  q.rp = whole ? g->rsym.rp : g->sym.rp;
+  q.ci = whole ? g->rsym.ci : g->sym.ci;
+  q.src = whole ? g->d_rsrc : g->d_src;
+  q.e0 = whole ? 0 : g->sym_rp_h[rb];
+  q.ne = whole ? g->sym.nnz : g->sym_rp_h[re] - q.e0;
+  q.rb = rb;
+  q.nr = re - rb;
+  q.xmin = whole ? g->rank_min2 : 0;
+  return JGPM_OK;
+}
+
+static int enqueue_p1(jgpm_graph_s* g, int64_t rb, int64_t re, int slot, hipStream_t st) {
   if (re <= rb) return JGPM_OK;
-  const int64_t waves = std::min<int64_t>(p1_waves(c, nv), (int64_t)(cnt_ints / std::max<int32_t>(nv, 1)));
-  const int grid = (int)std::min<int64_t>(waves / jk::P1_WPB, (re - rb + jk::P1_WPB - 1) / jk::P1_WPB);
-  if (!cnt || grid < 1) return JGPM_E_STATE;  // counters not sized for this graph
-  // a whole-graph count runs on the degree-ordered relabelling when it is
-  // built: the same identity in another vertex order gives the same total,
-  // and the hubs, ranked last, are no wedge's middle vertex
-  const bool ranked = rb == 0 && re == nv && g->rsym.ci;
+  jgpm_ctx_s* c = exec_ctx(g);
   jk::P1Args a{};
-  a.rp = ranked ? g->rsym.rp : g->sym.rp;
-  a.ci = ranked ? g->rsym.ci : g->sym.ci;
-  a.rb = rb;
-  a.re = re;
-  a.nv = nv;
-  // on the relabelling the hubs rank last: deal them first, so the widest
-  // roots do not run alone at the end of the launch
-  a.desc = ranked ? 1 : 0;
-  a.qctr = qctr;
-  a.cnt = cnt;
-  a.out = out;
+  int rc = p1_query(g, rb, re, st, a.one);
+  if (rc) return rc;
+  a.one.slot = slot;
+  a.nq = 1;
+  a.max_nv = g->sym.nv;
+  a.tiles = (a.one.ne + 255) / 256;
+  a.roots = a.one.nr;
+  a.edges = a.one.ne;
+  a.out = c->d_out;
+  if ((rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(a.roots, a.edges), st))) return rc;
+  jk::p1_bind_scratch(a, c->d_p1);
   prof_begin(c, st, "sym_p1_wedge");
-  hipError_t e = jk::launch_p1_wedge(a, grid, st);
+  hipError_t e = jk::launch_p1(a, c->num_cu, st);
   prof_end(c, st);
   return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
 }
@@ -120,12 +118,7 @@ int launch_p1(jgpm_graph_s* g, int64_t rb, int64_t re, uint64_t* out, unsigned* 
 int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStream_t st) {
   if (!g->has_sym) return JGPM_E_GRAPHKIND;
   jgpm_ctx_s* c = exec_ctx(g);
-  if (p == 1) {
-    int rc = ensure_p1_counters(c, p1_counter_ints(c, (int32_t)g->sym.nv), st);
-    if (rc) return rc;
-    if (rb == 0 && re == g->sym.nv && (rc = ensure_rank_csr(g, st))) return rc;
-    return launch_p1(g, rb, re, c->d_out + slot, c->d_q + slot, c->d_p1cnt, c->p1cnt_ints, st);
-  }
+  if (p == 1) return enqueue_p1(g, rb, re, slot, st);
   if (p == 2) {
     // diamonds from the per-edge triangle array: the array's one pass of
     // intersections (k_edge_tri) costs about what one P2 pass costs, and
@@ -299,7 +292,8 @@ int prepare_pattern(jgpm_graph_s* g, int pattern, int64_t rb, int64_t re) {
   if (clique_k(pattern)) {
     if (g->has_dag) rc = ensure_huge_ids(g);
   } else if (pattern == JGPM_P1) {
-    if (g->has_sym && rb == 0 && re == g->sym.nv) rc = ensure_rank_csr(g, c->st);
+    jk::P1Q q;
+    if (g->has_sym && re > rb) rc = p1_query(g, rb, re, c->st, q);
   } else if (pattern >= JGPM_P2 && pattern <= JGPM_P12) {
     if (g->has_sym) rc = ensure_sym_aux(g, query_needs_tri(c, pattern), pattern == JGPM_P3, c->st);
   }

@@ -298,9 +298,12 @@ __global__ void k_rank_deg(const int64_t* rp, const int32_t* ord, int32_t nv, in
   for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv; v += (int64_t)gridDim.x * blockDim.x)
     deg[ord[v]] = rp[v + 1] - rp[v];
 }
-__global__ void k_low_bits(const uint64_t* keys, int64_t ne, uint64_t mask, int32_t* ci) {
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += (int64_t)gridDim.x * blockDim.x)
+__global__ void k_split_keys(const uint64_t* keys, int64_t ne, int B, int32_t* src, int32_t* ci) {
+  const uint64_t mask = (1ull << B) - 1;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += (int64_t)gridDim.x * blockDim.x) {
+    src[e] = (int32_t)(keys[e] >> B);
     ci[e] = (int32_t)(keys[e] & mask);
+  }
 }
 
 }  // namespace
@@ -437,12 +440,15 @@ int ensure_rank_csr(jgpm_graph_s* g, hipStream_t st) {
     (void)hipFree(r.rp);
     return JGPM_E_NOMEM;
   }
+  int32_t* rsrc = nullptr;
   auto fail = [&](int code) {
     (void)hipStreamSynchronize(st);
     (void)hipFree(r.rp);
     (void)hipFree(r.ci);
+    if (rsrc) (void)hipFree(rsrc);
     return code;
   };
+  if (hipMalloc(&rsrc, sizeof(int32_t) * std::max<int64_t>(ne, 1)) != hipSuccess) return fail(JGPM_E_NOMEM);
   int64_t* deg = S.get<int64_t>((size_t)nv + 1);
   if (!deg) return fail(JGPM_E_NOMEM);
   hipLaunchKernelGGL(k_rank_deg, dim3(grid_for(nv)), dim3(256), 0, st, g->sym.rp, g->d_ord, nv, deg);
@@ -459,11 +465,14 @@ int ensure_rank_csr(jgpm_graph_s* g, hipStream_t st) {
     void* tmp = S.get<char>(tb);
     if (!tmp) return fail(JGPM_E_NOMEM);
     if (hipcub::DeviceRadixSort::SortKeys(tmp, tb, db, (int)ne, 0, 2 * B, st) != hipSuccess) return fail(JGPM_E_HIP);
-    hipLaunchKernelGGL(k_low_bits, dim3(grid_for(ne)), dim3(256), 0, st, db.Current(), ne, (1ull << B) - 1, r.ci);
+    hipLaunchKernelGGL(k_split_keys, dim3(grid_for(ne)), dim3(256), 0, st, db.Current(), ne, B, rsrc, r.ci);
   }
   if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return fail(JGPM_E_HIP);
   g->rsym = r;
-  g->bytes += 8 * ((int64_t)nv + 1) + 4 * ne;
+  g->d_rsrc = rsrc;
+  g->rank_min2 = 0;  // the vertices with at most one neighbour hold the first ranks
+  for (int32_t v = 0; v < nv; ++v) g->rank_min2 += g->sym_rp_h[v + 1] - g->sym_rp_h[v] <= 1;
+  g->bytes += 8 * ((int64_t)nv + 1) + 8 * ne;
   return JGPM_OK;
 }
 

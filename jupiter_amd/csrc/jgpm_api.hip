@@ -299,7 +299,7 @@ extern "C" int jgpm_shutdown(jgpm_ctx_t c) {
   if (c->d_sscr) (void)hipFree(c->d_sscr);
   if (c->d_hlist) (void)hipFree(c->d_hlist);
   if (c->d_hctr) (void)hipFree(c->d_hctr);
-  if (c->d_p1cnt) (void)hipFree(c->d_p1cnt);
+  if (c->d_p1) (void)hipFree(c->d_p1);
   if (c->d_bq) (void)hipFree(c->d_bq);
   if (c->d_bcs) (void)hipFree(c->d_bcs);
   if (c->d_bcnt) (void)hipFree(c->d_bcnt);
@@ -408,6 +408,7 @@ extern "C" int jgpm_graph_free(jgpm_graph_t g) {
   if (g->d_ord) (void)hipFree(g->d_ord);
   if (g->huge_d) (void)hipFree(g->huge_d);
   free_csr(g->rsym);
+  if (g->d_rsrc) (void)hipFree(g->d_rsrc);
   delete g;
   return JGPM_OK;
 }

@@ -36,8 +36,8 @@ struct jgpm_ctx_s {
   int32_t* d_hlist = nullptr;  // heavy-edge lists of P5/P7/P9/P11/P12 (3 x hcap ints)
   int64_t hcap = 0;
   unsigned long long* d_hctr = nullptr;  // their append and pop counters (6)
-  int32_t* d_p1cnt = nullptr;  // wedge counters of the 4-cycle kernel (all zero between launches)
-  size_t p1cnt_ints = 0;
+  void* d_p1 = nullptr;        // scratch of the 4-cycle launches (per-root and per-edge arrays)
+  size_t p1_bytes = 0;
   // batched / served launches: query table, chunk prefix, per-query counts
   void* d_bq = nullptr;
   int64_t* d_bcs = nullptr;
@@ -76,6 +76,8 @@ struct jgpm_graph_s {
   int32_t* d_tri = nullptr;                    // triangles per symmetric edge (lazy)
   int64_t* d_nsum = nullptr;                   // neighbour-degree sums (lazy)
   DevCSR rsym;                                 // symmetric CSR relabelled by d_ord (lazy, 4-cycle totals)
+  int32_t* d_rsrc = nullptr;                   // ... and the source of each of its edges
+  int32_t rank_min2 = 0;                       // vertices with at most one neighbour: the first ranks
   int64_t bytes = 0;
   int nbatch = 0;                              // prepared batches that reference this graph
 };
@@ -110,22 +112,19 @@ int zero_u64(uint64_t* p, int n, hipStream_t st);
 // Address of this device's static scratch array of jgpm_count_noalloc
 // (noalloc.hip), taken once per device with `dev` current.
 int noalloc_setup(int dev, uint64_t** out);
-// 4-cycle (P1) wedge kernel.  p1_counter_ints: the zeroed counter ints a
-// graph of nv vertices needs; ensure_p1_counters grows the context's (it
-// allocates, never while capturing); launch_p1 only launches, into *out, with
-// the zeroed 32-bit queue counter qctr and counters cnt[0..cnt_ints) that are
-// all zero (and are left so).
-size_t p1_counter_ints(jgpm_ctx_s* c, int32_t nv);
-// g->rsym: vertex v becomes d_ord[v] (degree order), lists re-sorted.  Built
-// once per graph (allocates; never while capturing).
+// The 4-cycle (P1) query of a root range: builds what it reads of the graph
+// on first use (COO sources, or for a whole graph the degree-order
+// relabelling; allocates, never while capturing) and describes it.
+int p1_query(jgpm_graph_s* g, int64_t rb, int64_t re, hipStream_t st, jk::P1Q& q);
+// Grows the context's 4-cycle scratch (allocates, never while capturing).
+int ensure_p1_scratch(jgpm_ctx_s* c, size_t bytes, hipStream_t st);
+// g->rsym: vertex v becomes d_ord[v] (degree order), lists re-sorted, and its
+// edge sources.  Built once per graph (allocates; never while capturing).
 int ensure_rank_csr(jgpm_graph_s* g, hipStream_t st);
 // A checked symmetric CSR in host memory -> resident graph; the degree DAG is
 // built on the device (ingest.hip).  dag_only keeps only the DAG.
 int graph_from_host_sym(jgpm_ctx_s* c, const int64_t* rowptr, const int32_t* colidx, int32_t nv, int64_t nnz,
                         bool dag_only, jgpm_graph_t* out);
-int ensure_p1_counters(jgpm_ctx_s* c, size_t need, hipStream_t st);
-int launch_p1(jgpm_graph_s* g, int64_t rb, int64_t re, uint64_t* out, unsigned* qctr, int32_t* cnt, size_t cnt_ints,
-              hipStream_t st);
 int ensure_scratch(jgpm_ctx_s* c, size_t words);
 int clique_k(int pattern);
 int enqueue_clique(jgpm_graph_s* g, int k, bool bytes, int64_t rb, int64_t re, int out_slot, hipStream_t st,

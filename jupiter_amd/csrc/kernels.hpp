@@ -101,34 +101,37 @@ int sym_heavy_stream();
 int sym_heavy_mid(int p);  // |S| up to this: the narrow launch (more blocks per CU)
 hipError_t launch_sym_heavy(int p, const SymArgs& a, int shape, int grid, hipStream_t st);
 
-// 4-cycles (P1) by wedges: one wave per root of [rb, re), counters in a
-// per-wave dense array of nv ints (cnt + wave * nv), zero before and after.
-struct P1Args {
+// 4-cycles (P1) by wedges (p1_wedge.hip): every root range of one or more
+// queries in one sequence of launches.
+struct P1Q {
   const int64_t* rp;
   const int32_t* ci;
-  int64_t rb, re;
-  int32_t nv;
-  int32_t desc;  // deal the roots from re - 1 down (degree-ordered graphs: widest roots first)
-  unsigned* qctr;
-  int32_t* cnt;
+  const int32_t* src;    // source of every directed edge
+  int64_t e0, ne;        // directed edges of the root range
+  int64_t rb, nr;        // first root, number of roots
+  int64_t eoff, roff;    // the query's first entry in the per-edge and per-root scratch
+  int32_t xmin;          // ids below have at most one neighbour (0: unknown)
+  int32_t slot;          // its accumulator is out[slot]
+};
+struct P1Args {
+  P1Q one;               // the query, when q is null
+  const P1Q* q;          // device table of nq queries
+  int nq;
+  int32_t max_nv;        // largest vertex count of the queries
+  const int64_t* tcs;    // prefix of the queries' 256-edge tiles (nq + 1)
+  const int64_t* rcs;    // prefix of the queries' roots (nq + 1)
+  int64_t tiles, roots, edges;  // totals
+  unsigned long long* ctr;      // scratch: list and task counters (8)
+  uint64_t* W;                  // per root its wedges
+  int32_t* m0;                  // per root its neighbours below it
+  int2* list;                   // roots (root, query) as wave tasks from the front, block tasks from the back
+  int2* split;                  // roots taken by several blocks
+  int32_t* len;                 // per edge (v0, v) the neighbours of v below v0
   uint64_t* out;
 };
-constexpr int P1_WPB = 4;
-hipError_t launch_p1_wedge(const P1Args& a, int grid, hipStream_t st);
-// Every 4-cycle query of a batch (BQ kind 101: rp/ci, first root `base`) in
-// one launch over the flattened roots; p1cs[i] = roots of the 4-cycle
-// queries before query i (nq + 1 entries), counts[i] the query's slot.
-struct P1BatchArgs {
-  const BQ* q;
-  const int64_t* p1cs;
-  int nq;
-  int64_t total;
-  unsigned* qctr;        // zero before the launch
-  int32_t* cnt;          // per wave cnt_stride ints, zero before and after
-  int64_t cnt_stride;    // >= the largest vertex count of the queries
-  uint64_t* counts;
-};
-hipError_t launch_p1_batch(const P1BatchArgs& a, int grid, hipStream_t st);
+size_t p1_scratch_bytes(int64_t roots, int64_t edges);
+void p1_bind_scratch(P1Args& a, void* p);  // a.roots and a.edges set
+hipError_t launch_p1(const P1Args& a, int num_cu, hipStream_t st);
 
 // One wave per root vertex v_0 of [rb, re) on the symmetric CSR.
 struct PlanArgs {

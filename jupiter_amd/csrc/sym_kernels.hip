@@ -28,8 +28,8 @@
 //       (s - 1 - [v3 in S])(t(v0,v3) - 1 - [v3 in S]) - (|S ∩ N(v3)| - 1)
 //   P11 sum_{S'} (a b c - q (a + b + c) + 2 q), a = s-1, b = t(v0,v2)-1, c = t(v1,v2)-1   (v0 < v1)
 //   P12 (s - 3) sum_S C(q(v2), 2)                                 (v0 < v1)
-// P1 runs as per-root wedge counting (p1_wedge_kernel below), which sums the
-// reference nest's per-edge values exactly.
+// P1 runs as per-root wedge counting (p1_wedge.hip), which sums the reference
+// nest's per-edge values exactly.
 //
 // Set operations are wave-wide: the shorter list is the lookup side, each
 // lane binary-searches its element in the longer list (staged in LDS when it
@@ -379,262 +379,6 @@ __global__ void __launch_bounds__(64 * WAVES) sym_heavy_kernel(SymArgs a) {
     }
   }
   if (tid == 0 && acc) atomicAdd((unsigned long long*)a.out, (unsigned long long)acc);
-}
-
-// ---------------------------------------------------------------------------
-// P1 (4-cycles) by wedges.  The reference's per-edge value (edges (v0, v1),
-// v1 < v0: sum over v2 in N(v0), v2 < v1, of |N(v1) ∩ N(v2) ∩ [0, v0)|;
-// src/message_passing_gpu_kernels.cuh:104-186) summed over a root's edges is
-//   sum over x < v0 of C(c_x, 2),  c_x = |{v in N(v0) : v < v0, x in N(v)}|:
-// every pair v2 < v1 of the c_x such v with the common neighbour x is one
-// term.  So a root needs one pass over its wedges (v0, v, x) with v, x < v0,
-// not an intersection per pair.  One wave per root; the wedges of 64
-// neighbours v at a time form one flattened stream (consecutive lanes read
-// consecutive elements).  The root's wedge count W picks where the c_x live:
-//  * W <= P1_HS / 2: the wave's LDS hash table, its first 2^t slots with
-//    2^t >= 2W: open addressing on 64-bit slots (key x in the high half,
-//    count in the low half; a slot is claimed by compare-and-swap and counted
-//    by a 64-bit add), summed and emptied in one sweep of those 2^t slots;
-//  * larger W up to a bound: a hash table of the same form over the first
-//    words of the wave's global counter region (keys x + 1, so that zero is
-//    the empty slot), claimed and counted by atomics, emptied by atomicExch;
-//  * otherwise the region as dense counters: a first pass adds 1 to c_x, a
-//    second takes every counter back to zero with atomicExch and adds C(c, 2)
-//    for the value it took (a repeated x takes 0 after its first exchange).
-constexpr uint64_t P1_EMPTY = 0xffffffff00000000ull;  // key -1, count 0
-
-// Calls f(x) for every wedge endpoint x of root v0 (its m0 neighbours below
-// v0 start at ci[b0]), 64 neighbours at a time.
-template <class F>
-__device__ void p1_wedges(const int64_t* rp, const int32_t* ci, int64_t b0, int m0, int32_t v0, int32_t* off,
-                          int64_t* lbase, F f, int len0 = -1, int64_t base0 = 0) {
-  const int ln = lane();
-  for (int jb = 0; jb < m0; jb += 64) {
-    const int j = jb + ln;
-    int len = 0;
-    int64_t base = 0;
-    if (jb == 0 && len0 >= 0) {
-      // the first 64 neighbours' segments, found by the caller
-      len = len0;
-      base = base0;
-    } else if (j < m0) {
-      const int32_t v = ci[b0 + j];
-      base = rp[v];
-      len = lb(ci + base, (int)(rp[v + 1] - base), v0);  // x < v0
-    }
-    int incl = len;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(incl, o);
-      if (ln >= o) incl += y;
-    }
-    const int T = __shfl(incl, 63);
-    off[ln] = incl - len;
-    lbase[ln] = base - (incl - len);  // element f of v's segment is ci[lbase + f]
-    if (ln == 63) off[64] = T;
-    __syncwarp();
-    int i = 0;
-    for (int fe = ln; fe < T; fe += 64) {
-      i = seg_advance(off, 64, i, fe);
-      f(ci[lbase[i] + fe]);
-    }
-    __syncwarp();
-  }
-}
-
-// The 4-cycle count of root v0: sum over x < v0 of C(c_x, 2), the c_x in the
-// wave's LDS table `tab` (roots with at most P1_HS / 2 wedges), else in a hash
-// table laid over the wave's global counter region `cnt` (cnt_len ints, zero
-// before, left zero), or in the region as dense counters when the table does
-// not fit it.  Wave-uniform result.
-template <int LOG>
-__device__ uint64_t p1_root(const int64_t* rp, const int32_t* ci, int32_t v0, uint64_t* tab, int32_t* off,
-                            int64_t* lbase, int32_t* cnt, int64_t cnt_len) {
-  constexpr int P1_HS = 1 << LOG;
-  constexpr int P1_LOG_HS = LOG;
-  const int ln = lane();
-  const int64_t b0 = rp[v0];
-  const int m0 = lb(ci + b0, (int)(rp[v0 + 1] - b0), v0);  // neighbours below v0
-  // wedge count of the root, to pick the table; the first 64 neighbours'
-  // segments are kept for the wedge passes (most roots have no more), so
-  // their binary searches are not repeated
-  int64_t w = 0;
-  int len0 = 0;
-  int64_t base0 = 0;
-  for (int j = ln; j < m0; j += 64) {
-    const int32_t v = ci[b0 + j];
-    const int64_t base = rp[v];
-    const int len = lb(ci + base, (int)(rp[v + 1] - base), v0);
-    if (j == ln) {
-      len0 = len;
-      base0 = base;
-    }
-    w += len;
-  }
-  w = wsum64(w);
-  uint64_t acc = 0;
-  if (w < 2) return 0;  // no pair of wedges shares an endpoint
-  if (w <= P1_HS / 2) {
-    // only the first 2^lt slots (load <= 1/2) are used, so the sweep below
-    // costs the root's own wedge count, not the whole table
-    int lt = 6;
-    while (lt < P1_LOG_HS && ((int64_t)1 << lt) < 2 * w) ++lt;
-    const int used = 1 << lt;
-    p1_wedges(rp, ci, b0, m0, v0, off, lbase, [&](int32_t x) {
-      const uint64_t key = (uint64_t)(uint32_t)x << 32;
-      int h = (int)(((uint32_t)x * 2654435761u) >> (32 - lt));
-      for (;;) {
-        uint64_t cur = tab[h];
-        if ((cur & P1_EMPTY) == key) {
-          atomicAdd((unsigned long long*)&tab[h], 1ull);
-          break;
-        }
-        if (cur == P1_EMPTY) {
-          cur = atomicCAS((unsigned long long*)&tab[h], P1_EMPTY, key | 1ull);
-          if (cur == P1_EMPTY) break;
-          if ((cur & P1_EMPTY) == key) {  // claimed by another lane for the same x
-            atomicAdd((unsigned long long*)&tab[h], 1ull);
-            break;
-          }
-        }
-        h = (h + 1) & (used - 1);
-      }
-    }, len0, base0);
-    __syncwarp();
-    for (int k = ln; k < used; k += 64) {
-      const uint64_t v = tab[k];
-      if (v != P1_EMPTY) {
-        const uint64_t c = (uint32_t)v;
-        acc += c * (c - 1) / 2;
-        tab[k] = P1_EMPTY;
-      }
-    }
-    __syncwarp();
-  } else {
-    // a hash table of 2^lt 64-bit slots (load <= 1/2) laid over the wave's
-    // counter region when it is small and fits: key x + 1 in the high half (0 = empty, so
-    // the region's all-zero state is an empty table), count in the low half.
-    // Its slots are a compact block of the region, where the dense counters
-    // below scatter over all nv of them.  Every access is an atomic, so no
-    // stale cached line is read, and the sweep leaves the region zero.
-    int lt = P1_LOG_HS + 1;
-    while (((int64_t)1 << lt) < 2 * w) ++lt;
-    const int64_t used = (int64_t)1 << lt;
-    const uintptr_t a0 = (reinterpret_cast<uintptr_t>(cnt) + 7) & ~(uintptr_t)7;
-    uint64_t* gt = reinterpret_cast<uint64_t*>(a0);
-    const int64_t slots = ((reinterpret_cast<uintptr_t>(cnt + cnt_len) - a0) / 8);
-    // beyond 2^15 slots (256 KiB) the table no longer stays in cache and its
-    // probes cost more than the dense counters' (R-MAT 20, vertex order: half
-    // the roots 1.02 s with dense counters, 1.50 s with unbounded tables)
-    if (lt <= 15 && used <= slots) {
-      p1_wedges(rp, ci, b0, m0, v0, off, lbase, [&](int32_t x) {
-        const uint64_t key = (uint64_t)(uint32_t)(x + 1) << 32;
-        uint64_t h = ((uint64_t)((uint32_t)x * 2654435761u) << lt) >> 32;  // top lt bits of the product
-        for (;;) {
-          const uint64_t cur = atomicCAS((unsigned long long*)&gt[h], 0ull, (unsigned long long)(key | 1ull));
-          if (cur == 0ull) break;
-          if ((cur >> 32) == (key >> 32)) {
-            atomicAdd((unsigned long long*)&gt[h], 1ull);
-            break;
-          }
-          h = (h + 1) & (uint64_t)(used - 1);
-        }
-      }, len0, base0);
-      __threadfence();
-      for (int64_t k = ln; k < used; k += 64) {
-        const uint64_t v = atomicExch((unsigned long long*)&gt[k], 0ull);
-        const uint64_t c = (uint32_t)v;
-        acc += c * (c - 1) / 2;
-      }
-      __threadfence();
-    } else {
-      p1_wedges(rp, ci, b0, m0, v0, off, lbase, [&](int32_t x) { atomicAdd(&cnt[x], 1); }, len0, base0);
-      __threadfence();  // the increments are performed before they are taken back
-      p1_wedges(rp, ci, b0, m0, v0, off, lbase, [&](int32_t x) {
-        const uint64_t c = (uint32_t)atomicExch(&cnt[x], 0);
-        acc += c * (c - 1) / 2;
-      }, len0, base0);
-      __threadfence();
-    }
-  }
-  return wave_sum_u64(acc);
-}
-
-template <int LOG>
-__global__ void __launch_bounds__(64 * P1_WPB) p1_wedge_kernel(P1Args a) {
-  constexpr int P1_HS = 1 << LOG;
-  __shared__ uint64_t s_tab[P1_WPB][P1_HS];
-  __shared__ int32_t s_off[P1_WPB][65];
-  __shared__ int64_t s_lb[P1_WPB][64];
-  const int wv = threadIdx.x >> 6;
-  const int ln = lane();
-  uint64_t* tab = s_tab[wv];
-  int32_t* cnt = a.cnt + ((int64_t)blockIdx.x * P1_WPB + wv) * a.nv;
-  for (int k = ln; k < P1_HS; k += 64) tab[k] = P1_EMPTY;
-  __syncwarp();
-  uint64_t acc = 0;
-  for (;;) {
-    int64_t t = 0;
-    if (ln == 0) t = (int64_t)atomicAdd(a.qctr, 1u);
-    t = __shfl(t, 0);
-    if (a.rb + t >= a.re) break;
-    const int64_t r = a.desc ? a.re - 1 - t : a.rb + t;
-    acc += p1_root<LOG>(a.rp, a.ci, (int32_t)r, tab, s_off[wv], s_lb[wv], cnt, a.nv);
-  }
-  if (ln == 0 && acc) atomicAdd((unsigned long long*)a.out, (unsigned long long)acc);
-}
-
-// The 4-cycle queries of a batch in one launch: the roots of every query
-// with kind 101 form one flattened task range (prefix p1cs over the query
-// table); a wave takes one root at a time, finds its query by binary search
-// over the prefix, and adds the root's count to the query's slot.
-template <int LOG>
-__global__ void __launch_bounds__(64 * P1_WPB) p1_batch_kernel(P1BatchArgs a) {
-  constexpr int P1_HS = 1 << LOG;
-  __shared__ uint64_t s_tab[P1_WPB][P1_HS];
-  __shared__ int32_t s_off[P1_WPB][65];
-  __shared__ int64_t s_lb[P1_WPB][64];
-  const int wv = threadIdx.x >> 6;
-  const int ln = lane();
-  uint64_t* tab = s_tab[wv];
-  int32_t* cnt = a.cnt + ((int64_t)blockIdx.x * P1_WPB + wv) * a.cnt_stride;
-  for (int k = ln; k < P1_HS; k += 64) tab[k] = P1_EMPTY;
-  __syncwarp();
-  for (;;) {
-    int64_t t = 0;
-    if (ln == 0) t = (int64_t)atomicAdd(a.qctr, 1u);
-    t = __shfl(t, 0);
-    if (t >= a.total) break;
-    int lo = 0, hi = a.nq;  // last query i with p1cs[i] <= t
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (a.p1cs[mid] <= t) lo = mid; else hi = mid;
-    }
-    // (ascending within a query: dealing a relabelled query's hubs first
-    // measured slower here, 276 -> 284 ms for 256 queries, the batch's other
-    // queries already filling the launch's tail)
-    const BQ& Q = a.q[lo];
-    const uint64_t c =
-        p1_root<LOG>(Q.rp, Q.ci, (int32_t)(Q.base + (t - a.p1cs[lo])), tab, s_off[wv], s_lb[wv], cnt, a.cnt_stride);
-    if (ln == 0 && c) atomicAdd((unsigned long long*)(a.counts + lo), (unsigned long long)c);
-  }
-}
-
-// log2 of the per-wave LDS table slots: 4096 (32 KiB per wave) measured
-// fastest against 2048 and 1024 on a batch of 256 Erdos-Renyi / Barabasi-
-// Albert 4-cycle queries (323 vs 420 vs 516 ms), though the smaller tables
-// give more waves per CU (R-MAT 18/20 and the 3.8M Chung-Lu graph: within
-// 0-28%, the Chung-Lu graph faster with 1024).
-constexpr int P1_TABLE_LOG2 = 12;
-
-hipError_t launch_p1_batch(const P1BatchArgs& a, int grid, hipStream_t st) {
-  hipLaunchKernelGGL(p1_batch_kernel<P1_TABLE_LOG2>, dim3(grid), dim3(64 * P1_WPB), 0, st, a);
-  return hipGetLastError();
-}
-
-hipError_t launch_p1_wedge(const P1Args& a, int grid, hipStream_t st) {
-  hipLaunchKernelGGL(p1_wedge_kernel<P1_TABLE_LOG2>, dim3(grid), dim3(64 * P1_WPB), 0, st, a);
-  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
