@@ -67,6 +67,19 @@ __device__ __forceinline__ int seg_advance(const int* a, int n, int i, int f) {
   return lo;
 }
 
+// Takes n items from a shared work counter for the whole wave (every lane
+// gets the counter's old value).  The wave barriers keep the compiler from
+// joining the lane-0 branch to a lane-0 branch before or after it: the other
+// lanes would then run ahead of lane 0 and read no counter value.
+template <class T>
+__device__ __forceinline__ T wave_take(T* ctr, T n) {
+  __builtin_amdgcn_wave_barrier();
+  T t = 0;
+  if (lane_id() == 0) t = atomicAdd(ctr, n);
+  __builtin_amdgcn_wave_barrier();
+  return __shfl(t, 0);
+}
+
 // first index p in [0, n) with a[p] >= y (n if none)
 template <class T>
 __device__ __forceinline__ int lower_bound_dev(const T* a, int n, int y) {

@@ -20,6 +20,53 @@ jgpm_ctx_s* exec_ctx(const jgpm_graph_s* g) { return t_exec ? t_exec : g->ctx; }
 ExecScope::ExecScope(jgpm_ctx_s* c) : prev(t_exec) { t_exec = c; }
 ExecScope::~ExecScope() { t_exec = prev; }
 
+// Hub bitmaps of the triangle launches: the highest-degree vertices whose
+// bitmaps fit this (R-MAT 18: its 4,096 widest vertices).
+constexpr int64_t TRI_HUB_BYTES = (int64_t)128 << 20;
+
+// Arguments of the triangle launches on g, their scratch on the executing
+// context (the hub bitmaps still to be made by launch_hub_bitmaps).
+static int tri_args(jgpm_graph_s* g, hipStream_t st, jk::TriArgs& a) {
+  jgpm_ctx_s* c = exec_ctx(g);
+  const int32_t nv = g->sym.nv;
+  a = jk::TriArgs{};
+  a.rp = g->sym.rp;
+  a.ci = g->sym.ci;
+  a.drp = g->dag.rp;
+  a.dci = g->dag.ci;
+  a.ord = g->d_ord;
+  a.dtri = g->d_dtri;
+  a.nv = nv;
+  a.wide = g->sym.max_deg > 64;
+  // a wave works its vertices off one after another: no more per wave than
+  // it takes to fill the device (32 waves per CU)
+  a.vchunk = std::max(1, std::min(64, nv / (64 * c->num_cu)));
+  a.hwords = (((int64_t)nv + 31) / 32 + 3) & ~(int64_t)3;
+  a.nhub = (int32_t)std::min<int64_t>(g->hubs, TRI_HUB_BYTES / (4 * a.hwords));
+  a.lstride = std::max(1, g->dag.max_deg);
+  const size_t hub_b = 4 * (size_t)a.hwords * (size_t)a.nhub;
+  const size_t list_b = (sizeof(int32_t) * 3 * (size_t)nv + 15) & ~(size_t)15;
+  const size_t lscr_b = a.wide ? sizeof(int32_t) * 3 * (size_t)a.lstride * (size_t)(jk::TRI_SMALL_PER_CU * c->num_cu) : 0;
+  const size_t need = 64 + hub_b + list_b + lscr_b;
+  if (c->te_bytes < need) {
+    if (c->capturing) return JGPM_E_STATE;
+    if (c->d_te) {
+      if (hipStreamSynchronize(st) != hipSuccess) return JGPM_E_HIP;
+      (void)hipFree(c->d_te);
+      c->d_te = nullptr;
+      c->te_bytes = 0;
+    }
+    if (hipMalloc(&c->d_te, need) != hipSuccess) return JGPM_E_NOMEM;
+    c->te_bytes = need;
+  }
+  unsigned char* b = static_cast<unsigned char*>(c->d_te);
+  a.ctr = reinterpret_cast<unsigned long long*>(b);
+  a.hub = reinterpret_cast<const uint32_t*>(b + 64);
+  a.list = reinterpret_cast<int32_t*>(b + 64 + hub_b);
+  a.lscr = reinterpret_cast<int32_t*>(b + 64 + hub_b + list_b);
+  return JGPM_OK;
+}
+
 // Lazily built per-graph arrays of the symmetric kernels.
 int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t st) {
   jgpm_ctx_s* c = exec_ctx(g);
@@ -32,13 +79,15 @@ int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t s
   if (need_tri && !g->d_tri) {
     if (hipMalloc(&g->d_tri, sizeof(int32_t) * std::max<int64_t>(ne, 1)) != hipSuccess) return JGPM_E_NOMEM;
     g->bytes += 4 * ne;
-    // its own queue counter, zeroed here: the builder runs from single
-    // queries, batch plans and the serving scheduler alike, and not every
-    // caller resets the context's counters first
-    unsigned long long* q = c->d_q64 + (CTX_SLOTS - 1);
-    if (zero_u64(reinterpret_cast<uint64_t*>(q), 1, st)) return JGPM_E_HIP;
+    const int64_t nd = g->dag.nnz;
+    if (hipMalloc(&g->d_dtri, sizeof(int32_t) * std::max<int64_t>(nd, 1)) != hipSuccess) return JGPM_E_NOMEM;
+    g->bytes += 4 * nd;
+    jk::TriArgs a;
+    int rc = tri_args(g, st, a);
+    if (rc) return rc;
     prof_begin(c, st, "edge_triangles");
-    hipError_t e = jk::launch_aux_tri(g->sym.rp, g->sym.ci, g->d_src, ne, g->d_tri, q, grid_for(c, 4), st);
+    hipError_t e = jk::launch_hub_bitmaps(a, c->num_cu, st);
+    if (e == hipSuccess) e = jk::launch_tri_build(a, g->d_dtri, g->d_src, ne, g->d_tri, c->num_cu, st);
     prof_end(c, st);
     if (e != hipSuccess) return JGPM_E_HIP;
   }
@@ -53,8 +102,50 @@ int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t s
 
 bool pattern_uses_tri(int p) { return p == 3 || p == 4 || p == 7 || p == 10 || p == 11; }
 
-// The single-query launches of P5, P7, P9, P11 and P12 read the triangle
-// array to send their heavy edges to the block-per-edge kernel.
+// P5, P7, P9, P11 and P12 over a root range that holds at least 1 / this of
+// the directed edges run as sums over all triangles, the terms of other roots
+// left out; smaller ranges run per edge.  P5 and P7 have work at every edge
+// of the range, the others only towards larger ids (R-MAT 18, the last
+// quarter of the ids with 1/17 of the edges: P5 16.7 ms per edge, 10.1 over
+// triangles; P7 10.5 and 10.1; P9 0.85 and 8.8, P12 1.7 and 10.1).
+static int64_t tri_sum_share(int p) { return p == 5 || p == 7 ? 32 : 8; }
+
+static int enqueue_tri_sum(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStream_t st) {
+  jgpm_ctx_s* c = exec_ctx(g);
+  int rc = ensure_sym_aux(g, true, false, st);
+  if (rc) return rc;
+  jk::TriArgs a;
+  if ((rc = tri_args(g, st, a))) return rc;
+  a.rb = rb;
+  a.re = re;
+  a.out = c->d_out + slot;
+  // roots whose rows do not fit LDS: one slice of the row scratch per block
+  if (g->tri_rows < 0) {
+    g->tri_rows = 0;
+    if (jk::tri_rows_global(g->sym.max_deg, g->dag.max_deg))
+      for (int32_t v = 0; v < g->sym.nv; ++v) {
+        const int64_t d = g->sym_rp_h[v + 1] - g->sym_rp_h[v], dp = g->dag_rp_h[v + 1] - g->dag_rp_h[v];
+        if (jk::tri_rows_global(d, dp)) g->tri_rows = std::max(g->tri_rows, jk::tri_row_words(d, dp));
+      }
+  }
+  int gblocks = 0;
+  if (g->tri_rows > 0) {
+    a.rstride = g->tri_rows;
+    gblocks = (int)std::max<int64_t>(1, std::min<int64_t>(c->num_cu, ((int64_t)1 << 27) / a.rstride));  // 1 GiB
+    if ((rc = ensure_scratch(c, (size_t)a.rstride * (size_t)gblocks))) return rc;
+    a.rows = c->d_scr;
+  }
+  static const char* const kName[13] = {"", "", "", "", "", "sym_p5_tri", "", "sym_p7_tri", "", "sym_p9_tri", "",
+                                        "sym_p11_tri", "sym_p12_tri"};
+  prof_begin(c, st, kName[p]);
+  hipError_t e = jk::launch_hub_bitmaps(a, c->num_cu, st);
+  if (e == hipSuccess) e = jk::launch_tri_sum(p, a, c->num_cu, gblocks, st);
+  prof_end(c, st);
+  return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
+}
+
+// The per-edge launches of P5, P7, P9, P11 and P12 read the triangle array
+// to send their heavy edges to the block-per-edge kernel.
 static bool heavy_split_on(const jgpm_ctx_s* c, int p) {
   return jk::sym_heavy_pattern(p) && c->tune.sym_heavy_min < jk::sym_heavy_nmax();
 }
@@ -136,8 +227,9 @@ int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStr
     prof_end(c, st);
     return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
   }
-  // The triangle array is shared by later queries; its counter slot is
-  // reset per query by ctx_reset_counters before it is used here.
+  const int64_t ne_q = g->sym_rp_h[re] - g->sym_rp_h[rb];
+  if (jk::sym_heavy_pattern(p) && ne_q > 0 && ne_q >= g->sym.nnz / tri_sum_share(p))
+    return enqueue_tri_sum(g, p, rb, re, slot, st);
   int rc = ensure_sym_aux(g, query_needs_tri(c, p), p == 3, st);
   if (rc) return rc;
   // the heavy-edge split needs its three edge lists, each as long as the

@@ -146,7 +146,10 @@ int set_degree_order(jgpm_graph_s* g, const std::vector<int64_t>& sym_rp, int32_
   std::vector<int32_t> ord((size_t)std::max(nv, 1));
   std::vector<int64_t> pos((size_t)max_deg + 2, 0);
   for (int32_t v = 0; v < nv; ++v) pos[sym_rp[v + 1] - sym_rp[v] + 1]++;
-  for (int32_t k = 0; k <= max_deg; ++k) pos[k + 1] += pos[k];
+  for (int32_t k = 0; k <= max_deg; ++k) {
+    if (k >= HUB_MIN_DEG) g->hubs += (int32_t)pos[k + 1];
+    pos[k + 1] += pos[k];
+  }
   for (int32_t v = 0; v < nv; ++v) ord[v] = (int32_t)pos[sym_rp[v + 1] - sym_rp[v]]++;
   if (hipMalloc(&g->d_ord, sizeof(int32_t) * std::max(nv, 1)) != hipSuccess) return JGPM_E_NOMEM;
   if (hipMemcpy(g->d_ord, ord.data(), sizeof(int32_t) * nv, hipMemcpyHostToDevice) != hipSuccess) return JGPM_E_HIP;
@@ -300,6 +303,7 @@ extern "C" int jgpm_shutdown(jgpm_ctx_t c) {
   if (c->d_hlist) (void)hipFree(c->d_hlist);
   if (c->d_hctr) (void)hipFree(c->d_hctr);
   if (c->d_p1) (void)hipFree(c->d_p1);
+  if (c->d_te) (void)hipFree(c->d_te);
   if (c->d_bq) (void)hipFree(c->d_bq);
   if (c->d_bcs) (void)hipFree(c->d_bcs);
   if (c->d_bcnt) (void)hipFree(c->d_bcnt);
@@ -404,6 +408,7 @@ extern "C" int jgpm_graph_free(jgpm_graph_t g) {
     if (g->tier_d[t]) (void)hipFree(g->tier_d[t]);
   if (g->d_src) (void)hipFree(g->d_src);
   if (g->d_tri) (void)hipFree(g->d_tri);
+  if (g->d_dtri) (void)hipFree(g->d_dtri);
   if (g->d_nsum) (void)hipFree(g->d_nsum);
   if (g->d_ord) (void)hipFree(g->d_ord);
   if (g->huge_d) (void)hipFree(g->huge_d);

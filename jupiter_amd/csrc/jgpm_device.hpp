@@ -9,6 +9,10 @@
 #include "jgpm_internal.hpp"
 #include "kernels.hpp"
 
+// Vertices with fewer neighbours are no hubs of the triangle launches: their
+// lists are searched in a few steps.
+constexpr int HUB_MIN_DEG = 32;
+
 // Accumulator / queue-counter slots per context (one query uses a few).
 constexpr int CTX_SLOTS = 64;
 
@@ -36,6 +40,8 @@ struct jgpm_ctx_s {
   int32_t* d_hlist = nullptr;  // heavy-edge lists of P5/P7/P9/P11/P12 (3 x hcap ints)
   int64_t hcap = 0;
   unsigned long long* d_hctr = nullptr;  // their append and pop counters (6)
+  void* d_te = nullptr;        // scratch of the triangle launches (lists, hub bitmaps)
+  size_t te_bytes = 0;
   void* d_p1 = nullptr;        // scratch of the 4-cycle launches (per-root and per-edge arrays)
   size_t p1_bytes = 0;
   // batched / served launches: query table, chunk prefix, per-query counts
@@ -74,6 +80,9 @@ struct jgpm_graph_s {
   int32_t sym_mmin = 1;                        // max over edges of min(d(u), d(v)): longest S = N(u) ∩ N(v)
   int32_t* d_src = nullptr;                    // COO source per symmetric edge (lazy)
   int32_t* d_tri = nullptr;                    // triangles per symmetric edge (lazy)
+  int32_t* d_dtri = nullptr;                   // ... and per DAG edge (built with d_tri)
+  int32_t hubs = 0;                            // vertices of at least HUB_MIN_DEG neighbours
+  int64_t tri_rows = -1;                       // widest rows of the triangle sums beyond LDS, words (-1: not known yet)
   int64_t* d_nsum = nullptr;                   // neighbour-degree sums (lazy)
   DevCSR rsym;                                 // symmetric CSR relabelled by d_ord (lazy, 4-cycle totals)
   int32_t* d_rsrc = nullptr;                   // ... and the source of each of its edges

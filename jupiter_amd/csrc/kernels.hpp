@@ -146,11 +146,45 @@ struct PlanArgs {
 };
 constexpr int PLAN_WPB = 4;
 hipError_t launch_plan(const PlanArgs& a, int grid, hipStream_t st);
+// Per-edge triangle counts, and the patterns that are sums over triangles
+// (tri_engine.hip).
+struct TriArgs {
+  const int64_t* rp;     // symmetric CSR
+  const int32_t* ci;
+  const int64_t* drp;    // degree DAG
+  const int32_t* dci;
+  const int32_t* ord;    // position of every vertex in the degree order
+  const int32_t* dtri;   // triangles per DAG edge (sums only)
+  int32_t nv;
+  int32_t vchunk;        // vertices a wave takes at a time (1 .. 64)
+  int32_t wide;          // some vertex has more neighbours than a wave task takes
+  int32_t nhub;          // hubs: the last nhub vertices of the degree order
+  const uint32_t* hub;   // their neighbours as bitmaps over the vertices
+  int64_t hwords;        // words per bitmap (a multiple of 4)
+  int64_t rb, re;        // root range
+  unsigned long long* ctr;      // scratch: list and task counters (8)
+  int32_t* list;                // 3 lists of nv roots
+  int32_t* lscr;                // 3 arrays of lstride ints per block
+  int64_t lstride;              // >= the DAG's maximum out-degree
+  uint64_t* rows;               // rows of roots too wide for LDS, rstride words per block
+  int64_t rstride;
+  uint64_t* out;
+};
+constexpr int TRI_SMALL_PER_CU = 6;  // blocks per CU of the narrow block tier
+int64_t tri_row_words(int64_t d, int64_t dp);  // words of the rows of a root (degree d, out-degree dp)
+bool tri_rows_global(int64_t d, int64_t dp);   // ... which do not fit LDS
+// the hubs' bitmaps, then with them:
+hipError_t launch_hub_bitmaps(const TriArgs& a, int num_cu, hipStream_t st);
+// triangles of every DAG edge and of every symmetric edge (src: their sources)
+hipError_t launch_tri_build(const TriArgs& a, int32_t* dtri, const int32_t* src, int64_t ne, int32_t* tri, int num_cu,
+                            hipStream_t st);
+// P5, P7, P9, P11 or P12 over [rb, re); gblocks blocks for the roots whose
+// rows are in a.rows (0: none)
+hipError_t launch_tri_sum(int p, const TriArgs& a, int num_cu, int gblocks, hipStream_t st);
+
 int sym_waves_per_block();
 int sym_lists_per_wave();
 hipError_t launch_aux_src(const int64_t* rp, int32_t nv, int32_t* src, int grid, hipStream_t st);
-hipError_t launch_aux_tri(const int64_t* rp, const int32_t* ci, const int32_t* src, int64_t ne, int32_t* tri,
-                          unsigned long long* qctr, int grid, hipStream_t st);
 hipError_t launch_aux_nsum(const int64_t* rp, const int32_t* ci, int32_t nv, int64_t* nsum, int grid, hipStream_t st);
 // mode 0: sum C(d,3) (3-stars); mode 1: sum t_v (d_v - 2) (tailed triangles)
 hipError_t launch_vertex_sums(const int64_t* rp, const int32_t* tri, int64_t rb, int64_t re, int mode,

@@ -35,7 +35,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "clique_dev.hpp"  // seg_advance, wave_sum_u64
+#include "clique_dev.hpp"  // seg_advance, wave_sum_u64, wave_take
 #include "kernels.hpp"
 #include "sym_dev.hpp"
 
@@ -140,9 +140,7 @@ __global__ void __launch_bounds__(256) k_p1_classify(P1Args a) {
   for (int c = 0; c < 3; ++c) {
     const uint64_t m = __ballot(cls == c);
     if (!m) continue;
-    unsigned long long base = 0;
-    if (ln == 0) base = atomicAdd(a.ctr + c, (unsigned long long)__popcll(m));
-    base = __shfl(base, 0);
+    const unsigned long long base = wave_take(a.ctr + c, (unsigned long long)__popcll(m));
     if (cls == c) {
       const int64_t k = (int64_t)base + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                                                       __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
@@ -360,9 +358,7 @@ __global__ void __launch_bounds__(64 * P1_WAVES) p1_kernel(P1Args a) {
       __syncthreads();
       const int32_t lo32 = (int32_t)lo;
       for (;;) {
-        int jb = 0;
-        if (ln == 0) jb = atomicAdd(&s_next, cs);
-        jb = __shfl(jb, 0);
+        const int jb = wave_take(&s_next, cs);
         if (jb >= m0) break;
         const int j = jb + ln;
         int len = 0;
@@ -412,9 +408,7 @@ __global__ void __launch_bounds__(64 * P1_WAVES) p1_kernel(P1Args a) {
   const int64_t nwave = (int64_t)a.ctr[C_WAVE];
   constexpr int CHUNK = 4;
   for (;;) {
-    unsigned long long t0 = 0;
-    if (ln == 0) t0 = atomicAdd(a.ctr + C_POPW, (unsigned long long)CHUNK);
-    const int64_t tb = (int64_t)__shfl(t0, 0);
+    const int64_t tb = (int64_t)wave_take(a.ctr + C_POPW, (unsigned long long)CHUNK);
     if (tb >= nwave) break;
     for (int64_t t = tb; t < min(nwave, tb + CHUNK); ++t) {
       const int2 it = a.list[t];

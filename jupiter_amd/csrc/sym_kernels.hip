@@ -393,36 +393,6 @@ __global__ void k_fill_src(const int64_t* rp, int32_t nv, int32_t* src) {
     for (int64_t e = rp[v] + lane(); e < rp[v + 1]; e += 64) src[e] = (int32_t)v;
 }
 
-// tri[e] = |N(u) ∩ N(v)| for every directed edge e = (u, v): one wave per edge.
-__global__ void __launch_bounds__(256) k_edge_tri(const int64_t* rp, const int32_t* ci, const int32_t* src,
-                                                  int64_t ne, int32_t* tri, unsigned long long* qctr) {
-  __shared__ int32_t s_stage[4][STAGE];
-  Wave w{s_stage[threadIdx.x >> 6]};
-  const int ln = lane();
-  for (;;) {
-    int64_t t = 0;
-    if (ln == 0) t = (int64_t)atomicAdd(qctr, 64ull);
-    const int64_t base = __shfl(t, 0);
-    if (base >= ne) break;
-    const int64_t end = min(ne, base + 64);
-    for (int64_t e = base; e < end; ++e) {
-      // |N(u) ∩ N(v)| is the same for both directions: intersect once, from
-      // the smaller end, and write it to (v, u) too (found by a wave-wide
-      // lower bound in N(v))
-      const int32_t u = src[e], v = ci[e];
-      if (v < u) continue;
-      const int64_t bv = rp[v];
-      const int dv = (int)(rp[v + 1] - bv);
-      int64_t c = w_icount(w, ci + rp[u], (int)(rp[u + 1] - rp[u]), ci + bv, dv, INT32_MAX);
-      const int pr = w_lb(ci + bv, dv, u);
-      if (ln == 0) {
-        tri[e] = (int32_t)c;
-        tri[bv + pr] = (int32_t)c;
-      }
-    }
-  }
-}
-
 // nsum[v] = sum of the degrees of v's neighbours.
 __global__ void k_nsum(const int64_t* rp, const int32_t* ci, int32_t nv, int64_t* nsum) {
   const int64_t wid = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -557,11 +527,6 @@ int sym_lists_per_wave() { return NLIST; }
 
 hipError_t launch_aux_src(const int64_t* rp, int32_t nv, int32_t* src, int grid, hipStream_t st) {
   hipLaunchKernelGGL(k_fill_src, dim3(grid), dim3(256), 0, st, rp, nv, src);
-  return hipGetLastError();
-}
-hipError_t launch_aux_tri(const int64_t* rp, const int32_t* ci, const int32_t* src, int64_t ne, int32_t* tri,
-                          unsigned long long* qctr, int grid, hipStream_t st) {
-  hipLaunchKernelGGL(k_edge_tri, dim3(grid), dim3(256), 0, st, rp, ci, src, ne, tri, qctr);
   return hipGetLastError();
 }
 hipError_t launch_aux_nsum(const int64_t* rp, const int32_t* ci, int32_t nv, int64_t* nsum, int grid, hipStream_t st) {
