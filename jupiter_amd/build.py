@@ -24,7 +24,7 @@ COMMON = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]
-LIB_SOURCES = ["host_graph.cpp", "clique_kernels.hip", "sym_kernels.hip", "p1_wedge.hip", "tri_engine.hip", "jgpm_api.hip", "dispatch.hip",
+LIB_SOURCES = ["host_graph.cpp", "clique_kernels.hip", "sym_kernels.hip", "wedge.hip", "tri_engine.hip", "jgpm_api.hip", "dispatch.hip",
                "batch.hip", "serve.hip", "ingest.hip", "plan.cpp", "plan_kernels.hip", "noalloc.hip", "clique_huge.hip",
                # the reference-shaped C++ host API (Graph, VertexSet, Pattern, SubgraphSolver)
                "Graph.cc", "VertexSet.cc", "Pattern.cc", "solver.cc"]

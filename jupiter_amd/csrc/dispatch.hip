@@ -20,6 +20,25 @@ jgpm_ctx_s* exec_ctx(const jgpm_graph_s* g) { return t_exec ? t_exec : g->ctx; }
 ExecScope::ExecScope(jgpm_ctx_s* c) : prev(t_exec) { t_exec = c; }
 ExecScope::~ExecScope() { t_exec = prev; }
 
+// Grows one of the context's scratch buffers to `need` bytes (allocates, never
+// while capturing); its contents are lost.
+static int grow(jgpm_ctx_s* c, void*& p, size_t& have, size_t need, hipStream_t st) {
+  if (have >= need) return JGPM_OK;
+  if (c->capturing) return JGPM_E_STATE;
+  if (p) {
+    if (hipStreamSynchronize(st) != hipSuccess) return JGPM_E_HIP;
+    (void)hipFree(p);
+    p = nullptr;
+    have = 0;
+  }
+  if (hipMalloc(&p, need) != hipSuccess) {
+    (void)hipGetLastError();
+    return JGPM_E_NOMEM;
+  }
+  have = need;
+  return JGPM_OK;
+}
+
 // Hub bitmaps of the triangle launches: the highest-degree vertices whose
 // bitmaps fit this (R-MAT 18: its 4,096 widest vertices).
 constexpr int64_t TRI_HUB_BYTES = (int64_t)128 << 20;
@@ -48,17 +67,7 @@ static int tri_args(jgpm_graph_s* g, hipStream_t st, jk::TriArgs& a) {
   const size_t list_b = (sizeof(int32_t) * 3 * (size_t)nv + 15) & ~(size_t)15;
   const size_t lscr_b = a.wide ? sizeof(int32_t) * 3 * (size_t)a.lstride * (size_t)(jk::TRI_SMALL_PER_CU * c->num_cu) : 0;
   const size_t need = 64 + hub_b + list_b + lscr_b;
-  if (c->te_bytes < need) {
-    if (c->capturing) return JGPM_E_STATE;
-    if (c->d_te) {
-      if (hipStreamSynchronize(st) != hipSuccess) return JGPM_E_HIP;
-      (void)hipFree(c->d_te);
-      c->d_te = nullptr;
-      c->te_bytes = 0;
-    }
-    if (hipMalloc(&c->d_te, need) != hipSuccess) return JGPM_E_NOMEM;
-    c->te_bytes = need;
-  }
+  if (int rc = grow(c, c->d_te, c->te_bytes, need, st)) return rc;
   unsigned char* b = static_cast<unsigned char*>(c->d_te);
   a.ctr = reinterpret_cast<unsigned long long*>(b);
   a.hub = reinterpret_cast<const uint32_t*>(b + 64);
@@ -77,19 +86,29 @@ int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t s
     if (jk::launch_aux_src(g->sym.rp, g->sym.nv, g->d_src, grid_for(c, 4), st) != hipSuccess) return JGPM_E_HIP;
   }
   if (need_tri && !g->d_tri) {
-    if (hipMalloc(&g->d_tri, sizeof(int32_t) * std::max<int64_t>(ne, 1)) != hipSuccess) return JGPM_E_NOMEM;
-    g->bytes += 4 * ne;
     const int64_t nd = g->dag.nnz;
-    if (hipMalloc(&g->d_dtri, sizeof(int32_t) * std::max<int64_t>(nd, 1)) != hipSuccess) return JGPM_E_NOMEM;
-    g->bytes += 4 * nd;
     jk::TriArgs a;
     int rc = tri_args(g, st, a);
     if (rc) return rc;
+    int32_t *tri = nullptr, *dtri = nullptr;
+    if (hipMalloc(&tri, sizeof(int32_t) * std::max<int64_t>(ne, 1)) != hipSuccess ||
+        hipMalloc(&dtri, sizeof(int32_t) * std::max<int64_t>(nd, 1)) != hipSuccess) {
+      if (tri) (void)hipFree(tri);
+      return JGPM_E_NOMEM;
+    }
     prof_begin(c, st, "edge_triangles");
     hipError_t e = jk::launch_hub_bitmaps(a, c->num_cu, st);
-    if (e == hipSuccess) e = jk::launch_tri_build(a, g->d_dtri, g->d_src, ne, g->d_tri, c->num_cu, st);
+    if (e == hipSuccess) e = jk::launch_tri_build(a, dtri, g->d_src, ne, tri, c->num_cu, st);
     prof_end(c, st);
-    if (e != hipSuccess) return JGPM_E_HIP;
+    if (e != hipSuccess) {
+      (void)hipStreamSynchronize(st);
+      (void)hipFree(tri);
+      (void)hipFree(dtri);
+      return JGPM_E_HIP;
+    }
+    g->d_tri = tri;
+    g->d_dtri = dtri;
+    g->bytes += 4 * ne + 4 * nd;
   }
   if (need_nsum && !g->d_nsum) {
     if (hipMalloc(&g->d_nsum, sizeof(int64_t) * (g->sym.nv + 1)) != hipSuccess) return JGPM_E_NOMEM;
@@ -135,11 +154,169 @@ static int enqueue_tri_sum(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int s
     if ((rc = ensure_scratch(c, (size_t)a.rstride * (size_t)gblocks))) return rc;
     a.rows = c->d_scr;
   }
-  static const char* const kName[13] = {"", "", "", "", "", "sym_p5_tri", "", "sym_p7_tri", "", "sym_p9_tri", "",
-                                        "sym_p11_tri", "sym_p12_tri"};
+  static const char* const kName[13] = {"", "", "", "", "sym_p4_tri", "sym_p5_tri", "", "sym_p7_tri", "", "sym_p9_tri",
+                                        "sym_p10_tri", "sym_p11_tri", "sym_p12_tri"};
   prof_begin(c, st, kName[p]);
   hipError_t e = jk::launch_hub_bitmaps(a, c->num_cu, st);
   if (e == hipSuccess) e = jk::launch_tri_sum(p, a, c->num_cu, gblocks, st);
+  prof_end(c, st);
+  return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
+}
+
+int ensure_tri_prefix(jgpm_graph_s* g, hipStream_t st) {
+  if (!g->tri_pre_h.empty()) return JGPM_OK;
+  jgpm_ctx_s* c = exec_ctx(g);
+  if (c->capturing) return JGPM_E_STATE;
+  int rc = ensure_sym_aux(g, true, false, st);
+  if (rc) return rc;
+  const int32_t nv = g->sym.nv;
+  int64_t* d = nullptr;
+  if (hipMalloc(&d, sizeof(int64_t) * std::max(nv, 1)) != hipSuccess) return JGPM_E_NOMEM;
+  std::vector<int64_t> pre((size_t)nv + 1, 0);
+  bool ok = jk::launch_root_tri(g->sym.rp, g->d_tri, nv, d, c->num_cu, st) == hipSuccess &&
+            hipMemcpyAsync(pre.data() + 1, d, sizeof(int64_t) * (size_t)nv, hipMemcpyDeviceToHost, st) == hipSuccess;
+  ok = (hipStreamSynchronize(st) == hipSuccess) && ok;
+  (void)hipFree(d);
+  if (!ok) return JGPM_E_HIP;
+  int64_t most = 0;
+  for (int32_t v = 0; v < nv; ++v) {
+    most = std::max(most, pre[v + 1]);
+    pre[v + 1] += pre[v];
+  }
+  g->tri_max = most;
+  g->tri_pre_h.swap(pre);
+  return JGPM_OK;
+}
+
+// P6, P8 and P10 count wedges on the graph of induced neighbourhoods, which
+// has a vertex per directed edge of the roots and 2 t entries per edge.  It is
+// built per query, for as many roots at a time as EGO_CAP entries hold.
+constexpr int64_t EGO_CAP = (int64_t)1 << 28;
+
+// Whether the range runs on the induced neighbourhoods: every root fits the
+// cap, for P10, whose triangle part covers all triangles, the range is not a
+// sliver of the graph, and there are triangles enough to pay for the launches
+// (Erdos-Renyi, 1,000 vertices, 640 triangles: P8 114 us per edge, 194 on the
+// induced graph; Barabasi-Albert, 1,000 vertices: 1,040 and 221; R-MAT 12
+// 384,000 and 357).
+static bool ego_route(jgpm_graph_s* g, int p, int64_t rb, int64_t re) {
+  if (p != 6 && p != 8 && p != 10) return false;
+  const int64_t ne = g->sym_rp_h[re] - g->sym_rp_h[rb];
+  if (g->tri_pre_h[re] - g->tri_pre_h[rb] < 16384 && g->tri_max < 256) return false;
+  return g->tri_max <= EGO_CAP && g->sym.max_deg < EGO_CAP && (p != 10 || ne >= g->sym.nnz / 1024);
+}
+
+static int enqueue_ego(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStream_t st) {
+  jgpm_ctx_s* c = exec_ctx(g);
+  uint64_t* const out = c->d_out + slot;
+  const int64_t *rp = g->sym_rp_h.data(), *pre = g->tri_pre_h.data();
+  // chunks of whole roots, and the scratch of the largest
+  std::vector<int64_t> cut{rb};
+  int64_t most_e = 0, most_n = 0;
+  for (int64_t r = rb; r < re;) {
+    int64_t r2 = std::upper_bound(pre + r + 1, pre + re + 1, pre[r] + EGO_CAP) - pre - 1;
+    r2 = std::min(r2, (int64_t)(std::upper_bound(rp + r + 1, rp + re + 1, rp[r] + EGO_CAP) - rp - 1));
+    r2 = std::max(r2, r + 1);
+    most_e = std::max(most_e, pre[r2] - pre[r]);
+    most_n = std::max(most_n, rp[r2] - rp[r]);
+    cut.push_back(r = r2);
+  }
+  const size_t rp_b = sizeof(int64_t) * (size_t)(most_n + 1), tiles_b = sizeof(int64_t) * (size_t)jk::ego_tiles(most_n);
+  const size_t ent_b = sizeof(int32_t) * (size_t)most_e;
+  int rc = grow(c, c->d_ego, c->ego_bytes, rp_b + tiles_b + 2 * ent_b + 64, st);
+  if (!rc) rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(most_n, most_e), st);
+  jk::TriArgs ta;
+  if (!rc) rc = tri_args(g, st, ta);
+  if (!rc && p == 10) rc = enqueue_tri_sum(g, 10, rb, re, slot, st);
+  if (rc) return rc;  // (nothing is launched when there was no room)
+  static const char* const kName[11] = {"", "", "", "", "", "", "sym_p6_wedge", "", "sym_p8_wedge", "", "sym_p10_wedge"};
+  prof_begin(c, st, kName[p]);
+  hipError_t e = jk::launch_hub_bitmaps(ta, c->num_cu, st);
+  for (size_t k = 0; k + 1 < cut.size() && e == hipSuccess; ++k) {
+    jk::EgoArgs ea{};
+    ea.src = g->d_src;
+    ea.tri = g->d_tri;
+    ea.e0 = rp[cut[k]];
+    ea.n = rp[cut[k + 1]] - ea.e0;
+    const int64_t ents = pre[cut[k + 1]] - pre[cut[k]];
+    if (ents == 0) continue;
+    unsigned char* b = static_cast<unsigned char*>(c->d_ego);
+    ea.rp = reinterpret_cast<int64_t*>(b);
+    ea.tiles = reinterpret_cast<int64_t*>(b + rp_b);
+    ea.ci = reinterpret_cast<int32_t*>(b + rp_b + tiles_b);
+    ea.row = reinterpret_cast<int32_t*>(b + rp_b + tiles_b + ent_b);
+    e = jk::launch_ego_build(ta, ea, c->num_cu, st);
+    jk::P1Args a{};
+    a.one.rp = ea.rp;
+    a.one.ci = ea.ci;
+    a.one.src = ea.row;
+    a.one.ne = ents;
+    a.one.nr = ea.n;
+    a.one.slot = slot;
+    a.one.csrc = g->d_src + ea.e0;
+    a.one.crp = g->sym.rp;
+    a.one.cbase = ea.e0;
+    if (p == 6) {
+      a.one.vid = g->sym.ci + ea.e0;
+      a.one.lrp = g->sym.rp;
+      a.one.lci = g->sym.ci;
+      a.one.xend = g->sym.nv;
+    }
+    if (p == 10) a.one.scale = -4;
+    a.nq = 1;
+    a.max_nv = (int32_t)ea.n;
+    a.tiles = (ents + 255) / 256;
+    a.roots = ea.n;
+    a.edges = ents;
+    a.out = c->d_out;
+    jk::p1_bind_scratch(a, c->d_p1);
+    if (e == hipSuccess) e = jk::launch_wedge(p == 6 ? jk::WEDGE_P6 : jk::WEDGE_P1, a, c->num_cu, st);
+    if (e == hipSuccess && p == 10) e = jk::launch_p10_rows(ea, out, c->num_cu, st);
+    if (e == hipSuccess && p == 6)
+      e = jk::launch_edge_base(g->sym.rp, g->sym.ci, g->d_src, g->d_tri, ea.e0, ea.e0 + ea.n, 2, out, c->num_cu, st);
+  }
+  prof_end(c, st);
+  return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
+}
+
+// P4 over a root range that is not a sliver of the graph (the triangle part
+// of a partial range covers all triangles): wedges from every root of the
+// range.
+static bool p4_route(const jgpm_graph_s* g, int64_t rb, int64_t re) {
+  return g->sym_rp_h[re] - g->sym_rp_h[rb] >= g->sym.nnz / 1024;
+}
+
+static int enqueue_p4(jgpm_graph_s* g, int64_t rb, int64_t re, int slot, hipStream_t st) {
+  jgpm_ctx_s* c = exec_ctx(g);
+  int rc = ensure_sym_aux(g, true, false, st);
+  if (rc) return rc;
+  const bool whole = rb == 0 && re == g->sym.nv;
+  const int64_t e0 = g->sym_rp_h[rb], e1 = g->sym_rp_h[re];
+  jk::P1Args a{};
+  a.one.rp = g->sym.rp;
+  a.one.ci = g->sym.ci;
+  a.one.src = g->d_src;
+  a.one.e0 = e0;
+  a.one.ne = e1 - e0;
+  a.one.rb = rb;
+  a.one.nr = re - rb;
+  a.one.slot = slot;
+  a.one.weight = g->d_tri;
+  a.one.xend = g->sym.nv;
+  a.nq = 1;
+  a.max_nv = g->sym.nv;
+  a.tiles = (a.one.ne + 255) / 256;
+  a.roots = a.one.nr;
+  a.edges = a.one.ne;
+  a.out = c->d_out;
+  if ((rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(a.roots, a.edges), st))) return rc;
+  if (!whole && (rc = enqueue_tri_sum(g, 4, rb, re, slot, st))) return rc;  // (nothing is launched when there was no room)
+  jk::p1_bind_scratch(a, c->d_p1);
+  prof_begin(c, st, "sym_p4_wedge");
+  hipError_t e = jk::launch_wedge(jk::WEDGE_P4, a, c->num_cu, st);
+  if (e == hipSuccess)
+    e = jk::launch_edge_base(g->sym.rp, g->sym.ci, g->d_src, g->d_tri, e0, e1, whole ? 1 : 0, c->d_out + slot, c->num_cu,
+                             st);
   prof_end(c, st);
   return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
 }
@@ -152,19 +329,7 @@ static bool heavy_split_on(const jgpm_ctx_s* c, int p) {
 
 bool query_needs_tri(const jgpm_ctx_s* c, int p) { return p == 2 || pattern_uses_tri(p) || heavy_split_on(c, p); }
 
-int ensure_p1_scratch(jgpm_ctx_s* c, size_t bytes, hipStream_t st) {
-  if (c->p1_bytes >= bytes) return JGPM_OK;
-  if (c->capturing) return JGPM_E_STATE;
-  if (c->d_p1) {
-    if (hipStreamSynchronize(st) != hipSuccess) return JGPM_E_HIP;
-    (void)hipFree(c->d_p1);
-    c->d_p1 = nullptr;
-    c->p1_bytes = 0;
-  }
-  if (hipMalloc(&c->d_p1, bytes) != hipSuccess) return JGPM_E_NOMEM;
-  c->p1_bytes = bytes;
-  return JGPM_OK;
-}
+int ensure_p1_scratch(jgpm_ctx_s* c, size_t bytes, hipStream_t st) { return grow(c, c->d_p1, c->p1_bytes, bytes, st); }
 
 int p1_query(jgpm_graph_s* g, int64_t rb, int64_t re, hipStream_t st, jk::P1Q& q) {
   q = jk::P1Q{};
@@ -227,9 +392,22 @@ int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStr
     prof_end(c, st);
     return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
   }
+  // patterns that run over triangles or wedges of the whole range; where
+  // there is no room for their scratch (nothing launched), per edge
   const int64_t ne_q = g->sym_rp_h[re] - g->sym_rp_h[rb];
-  if (jk::sym_heavy_pattern(p) && ne_q > 0 && ne_q >= g->sym.nnz / tri_sum_share(p))
-    return enqueue_tri_sum(g, p, rb, re, slot, st);
+  if (ne_q > 0) {
+    int rr = JGPM_E_NOMEM;
+    if (jk::sym_heavy_pattern(p) && ne_q >= g->sym.nnz / tri_sum_share(p)) {
+      rr = enqueue_tri_sum(g, p, rb, re, slot, st);
+    } else if (p == 4 && p4_route(g, rb, re)) {
+      rr = enqueue_p4(g, rb, re, slot, st);
+    } else if (p == 6 || p == 8 || p == 10) {
+      rr = ensure_tri_prefix(g, st);
+      if (!rr) rr = ego_route(g, p, rb, re) ? enqueue_ego(g, p, rb, re, slot, st) : JGPM_E_NOMEM;
+    }
+    if (rr != JGPM_E_NOMEM) return rr;
+    (void)hipGetLastError();
+  }
   int rc = ensure_sym_aux(g, query_needs_tri(c, p), p == 3, st);
   if (rc) return rc;
   // the heavy-edge split needs its three edge lists, each as long as the
@@ -388,6 +566,8 @@ int prepare_pattern(jgpm_graph_s* g, int pattern, int64_t rb, int64_t re) {
     if (g->has_sym && re > rb) rc = p1_query(g, rb, re, c->st, q);
   } else if (pattern >= JGPM_P2 && pattern <= JGPM_P12) {
     if (g->has_sym) rc = ensure_sym_aux(g, query_needs_tri(c, pattern), pattern == JGPM_P3, c->st);
+    if (g->has_sym && !rc && (pattern == JGPM_P6 || pattern == JGPM_P8 || pattern == JGPM_P10))
+      rc = ensure_tri_prefix(g, c->st);
   }
   if (hipStreamSynchronize(c->st) != hipSuccess && !rc) rc = JGPM_E_HIP;
   return rc;

@@ -304,6 +304,7 @@ extern "C" int jgpm_shutdown(jgpm_ctx_t c) {
   if (c->d_hctr) (void)hipFree(c->d_hctr);
   if (c->d_p1) (void)hipFree(c->d_p1);
   if (c->d_te) (void)hipFree(c->d_te);
+  if (c->d_ego) (void)hipFree(c->d_ego);
   if (c->d_bq) (void)hipFree(c->d_bq);
   if (c->d_bcs) (void)hipFree(c->d_bcs);
   if (c->d_bcnt) (void)hipFree(c->d_bcnt);

@@ -40,6 +40,8 @@ struct jgpm_ctx_s {
   int32_t* d_hlist = nullptr;  // heavy-edge lists of P5/P7/P9/P11/P12 (3 x hcap ints)
   int64_t hcap = 0;
   unsigned long long* d_hctr = nullptr;  // their append and pop counters (6)
+  void* d_ego = nullptr;       // the graph of induced neighbourhoods of P6, P8, P10
+  size_t ego_bytes = 0;
   void* d_te = nullptr;        // scratch of the triangle launches (lists, hub bitmaps)
   size_t te_bytes = 0;
   void* d_p1 = nullptr;        // scratch of the 4-cycle launches (per-root and per-edge arrays)
@@ -81,6 +83,8 @@ struct jgpm_graph_s {
   int32_t* d_src = nullptr;                    // COO source per symmetric edge (lazy)
   int32_t* d_tri = nullptr;                    // triangles per symmetric edge (lazy)
   int32_t* d_dtri = nullptr;                   // ... and per DAG edge (built with d_tri)
+  std::vector<int64_t> tri_pre_h;              // prefix of d_tri over the vertices (P6, P8, P10; empty: not known yet)
+  int64_t tri_max = 0;                         // ... and its largest vertex
   int32_t hubs = 0;                            // vertices of at least HUB_MIN_DEG neighbours
   int64_t tri_rows = -1;                       // widest rows of the triangle sums beyond LDS, words (-1: not known yet)
   int64_t* d_nsum = nullptr;                   // neighbour-degree sums (lazy)
@@ -144,6 +148,8 @@ int glb_tier_grid(const jgpm_ctx_s* c);
 // Root tier lists of the DAG (host row pointers) and the degree order.
 int build_tiers(jgpm_graph_s* g, const int64_t* rp, int32_t nv);
 int set_degree_order(jgpm_graph_s* g, const std::vector<int64_t>& sym_rp, int32_t max_deg);
+// g->tri_pre_h (waits for the stream once per graph).
+int ensure_tri_prefix(jgpm_graph_s* g, hipStream_t st);
 int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t st);
 // Batched persistent launch over queries the kernel supports (TC, P1..P16);
 // counts land in c->d_bcnt[0..n).  hq / cs are host staging that must stay

@@ -101,8 +101,9 @@ int sym_heavy_stream();
 int sym_heavy_mid(int p);  // |S| up to this: the narrow launch (more blocks per CU)
 hipError_t launch_sym_heavy(int p, const SymArgs& a, int shape, int grid, hipStream_t st);
 
-// 4-cycles (P1) by wedges (p1_wedge.hip): every root range of one or more
-// queries in one sequence of launches.
+// Patterns counted by wedges (wedge.hip).  4-cycles (P1): every root range of
+// one or more queries in one sequence of launches.
+enum { WEDGE_P1 = 0, WEDGE_P4 = 1, WEDGE_P6 = 2 };
 struct P1Q {
   const int64_t* rp;
   const int32_t* ci;
@@ -112,6 +113,17 @@ struct P1Q {
   int64_t eoff, roff;    // the query's first entry in the per-edge and per-root scratch
   int32_t xmin;          // ids below have at most one neighbour (0: unknown)
   int32_t slot;          // its accumulator is out[slot]
+  // single queries only:
+  int64_t scale = 1;     // what the count is multiplied by
+  const int32_t* csrc = nullptr;  // P8, P6 (roots are directed edges): the edges' sources ...
+  const int64_t* crp = nullptr;   // ... and row pointers: a P8 root's ids start at crp[csrc[root]] - cbase
+  int64_t cbase = 0;
+  const int32_t* vid = nullptr;   // P6: the edges' ends
+  const int64_t* lrp = nullptr;   // P6: the lists
+  const int32_t* lci = nullptr;
+  const int32_t* weight = nullptr;  // P4: per edge its triangles
+  int32_t xend = 0;      // P4, P6: ids end here
+  int32_t pad = 0;
 };
 struct P1Args {
   P1Q one;               // the query, when q is null
@@ -132,6 +144,7 @@ struct P1Args {
 size_t p1_scratch_bytes(int64_t roots, int64_t edges);
 void p1_bind_scratch(P1Args& a, void* p);  // a.roots and a.edges set
 hipError_t launch_p1(const P1Args& a, int num_cu, hipStream_t st);
+hipError_t launch_wedge(int mode, const P1Args& a, int num_cu, hipStream_t st);  // one query
 
 // One wave per root vertex v_0 of [rb, re) on the symmetric CSR.
 struct PlanArgs {
@@ -178,9 +191,29 @@ hipError_t launch_hub_bitmaps(const TriArgs& a, int num_cu, hipStream_t st);
 // triangles of every DAG edge and of every symmetric edge (src: their sources)
 hipError_t launch_tri_build(const TriArgs& a, int32_t* dtri, const int32_t* src, int64_t ne, int32_t* tri, int num_cu,
                             hipStream_t st);
-// P5, P7, P9, P11 or P12 over [rb, re); gblocks blocks for the roots whose
+// P5, P7, P9, P11 or P12, or the triangle parts of P4 and P10, over [rb, re); gblocks blocks for the roots whose
 // rows are in a.rows (0: none)
 hipError_t launch_tri_sum(int p, const TriArgs& a, int num_cu, int gblocks, hipStream_t st);
+
+// The graph of induced neighbourhoods over the directed edges [e0, e0 + n)
+// (whole roots): a vertex per edge (v0, u), joined to (v0, y) for every common
+// neighbour y of v0 and u; vertices are numbered from 0.
+struct EgoArgs {
+  const int32_t* src;   // the edges' sources, triangle counts (whole graph)
+  const int32_t* tri;
+  int64_t e0, n;
+  int64_t* tiles;       // scratch, ego_tiles(n)
+  int64_t* rp;          // out: n + 1 row pointers
+  int32_t* ci;          // out: entries, ascending in each row
+  int32_t* row;         // out: their rows
+};
+int64_t ego_tiles(int64_t n);
+hipError_t launch_ego_build(const TriArgs& a, const EgoArgs& g, int num_cu, hipStream_t st);  // with the hub bitmaps
+hipError_t launch_p10_rows(const EgoArgs& g, uint64_t* out, int num_cu, hipStream_t st);
+// closed per-edge parts: P4 (mode 0: root range, 1: whole graph), P6 (mode 2)
+hipError_t launch_edge_base(const int64_t* rp, const int32_t* ci, const int32_t* src, const int32_t* tri, int64_t e0,
+                            int64_t e1, int mode, uint64_t* out, int num_cu, hipStream_t st);
+hipError_t launch_root_tri(const int64_t* rp, const int32_t* tri, int32_t nv, int64_t* sum, int num_cu, hipStream_t st);
 
 int sym_waves_per_block();
 int sym_lists_per_wave();

@@ -244,7 +244,7 @@ __device__ int64_t edge_value(const Ctx& g, Wave& w, int32_t v0, int32_t v1, int
   int32_t* T = L[3];
   int32_t* pT = L[4];
   const int ln = lane();
-  static_assert(P >= 2 && P <= 12, "P1 runs as wedge counting (p1_wedge.hip)");
+  static_assert(P >= 2 && P <= 12, "P1 runs as wedge counting (wedge.hip)");
   if constexpr (P == 2) {
     if (v1 >= v0) return 0;
     return C2(w_icount(w, N0, d0, N1, d1, INT32_MAX));

@@ -28,7 +28,7 @@
 //       (s - 1 - [v3 in S])(t(v0,v3) - 1 - [v3 in S]) - (|S ∩ N(v3)| - 1)
 //   P11 sum_{S'} (a b c - q (a + b + c) + 2 q), a = s-1, b = t(v0,v2)-1, c = t(v1,v2)-1   (v0 < v1)
 //   P12 (s - 3) sum_S C(q(v2), 2)                                 (v0 < v1)
-// P1 runs as per-root wedge counting (p1_wedge.hip), which sums the reference
+// P1 runs as per-root wedge counting (wedge.hip), which sums the reference
 // nest's per-edge values exactly.
 //
 // Set operations are wave-wide: the shorter list is the lookup side, each

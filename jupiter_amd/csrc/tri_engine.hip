@@ -1,5 +1,6 @@
-// tri_engine.hip — per-edge triangle counts, and the patterns that are sums
-// over triangles: P5, P7, P9, P11 and P12 (and the 4-clique part of P10).
+// tri_engine.hip — per-edge triangle counts, the patterns that are sums over
+// triangles (P5, P7, P9, P11 and P12, and parts of P4 and P10), and the graph
+// of induced neighbourhoods that P6, P8 and P10 count wedges on.
 //
 // With t(u, v) = |N(u) ∩ N(v)| and q(T) = |N(a) ∩ N(x) ∩ N(y)| of a triangle
 // T = {a, x, y}, the per-edge values of sym_kernels.hip's header, summed over
@@ -250,6 +251,8 @@ __global__ void __launch_bounds__(256) k_tri_scatter(TriArgs a, const int32_t* d
 
 template <int P>
 constexpr bool needs_t() { return P != 9; }
+template <int P>
+constexpr bool is_twice() { return P == 5 || P == 10; }  // sums twice the value
 
 // one triangle's terms whose owner lies in [rb, re); ids a, x, y; txy etc.
 // the triangle counts of its edges (unused for P9)
@@ -257,7 +260,15 @@ template <int P>
 __device__ __forceinline__ int64_t tri_term(const TriArgs& g, int32_t a, int32_t x, int32_t y, int64_t tax, int64_t tay,
                                             int64_t txy, int64_t q) {
   auto in = [&](int32_t v) { return (int64_t)(v >= g.rb && v < g.re); };
-  if constexpr (P == 5) {  // twice the value: halved at the end
+  if constexpr (P == 4) {
+    // the part of P4 over triangles: less, for each edge as the (v0, v1) of
+    // the nest, the (t - 1) of the triangle's two other edges
+    return -(in(max(a, x)) * (tay + txy - 2) + in(max(a, y)) * (tax + txy - 2) + in(max(x, y)) * (tax + tay - 2));
+  } else if constexpr (P == 10) {
+    // sum over the edges (v0, x) of k (3 - 2 t), k the 4-cliques on the edge:
+    // half of the q of the edge's triangles
+    return q * ((in(a) + in(x)) * (3 - 2 * tax) + (in(a) + in(y)) * (3 - 2 * tay) + (in(x) + in(y)) * (3 - 2 * txy));
+  } else if constexpr (P == 5) {  // twice the value: halved at the end
     return q * (in(max(a, x)) * (tax - 2) + in(max(a, y)) * (tay - 2) + in(max(x, y)) * (txy - 2));
   } else if constexpr (P == 7) {
     return in(a) * ((tax - 1) * (tay - 1) - q) + in(x) * ((tax - 1) * (txy - 1) - q) +
@@ -279,14 +290,14 @@ __device__ __forceinline__ int32_t dag_t(const TriArgs& a, int32_t x, int32_t y,
   return a.dtri[b + lb(a.dci + b, (int)(a.drp[s + 1] - b), z)];
 }
 
-// Adds a wave's sum to the result.  P5's sums count every value twice: the
-// half is added, and an odd sum pairs up with another through a flag (the
-// total is even).
+// Adds a wave's sum to the result.  P5's and P10's sums count every value
+// twice: the half is added, and an odd sum pairs up with another through a
+// flag (the total is even).
 template <int P>
 __device__ __forceinline__ void tri_add(const TriArgs& a, uint64_t acc) {
   acc = wave_sum_u64(acc);
   if (lane() != 0 || !acc) return;
-  if constexpr (P == 5) {
+  if constexpr (is_twice<P>()) {
     const uint64_t half = (uint64_t)((int64_t)acc >> 1);
     const uint64_t odd = (acc & 1) ? atomicXor(a.ctr + 6, 1ull) : 0;
     atomicAdd((unsigned long long*)a.out, (unsigned long long)(half + odd));
@@ -547,6 +558,178 @@ unsigned wave_grid(const TriArgs& a, int num_cu) {
   return (unsigned)(blocks < num_cu * 8 ? blocks : num_cu * 8);
 }
 
+// ---------------------------------------------------------------------------
+// The graph of induced neighbourhoods: a vertex per directed edge (v0, u) of
+// the edges [e0, e0 + n), numbered from 0, joined to (v0, y) for every common
+// neighbour y of v0 and u.  Row (v0, u) has t(v0, u) entries; the rows of one
+// v0 are the graph that N(v0) induces.
+
+// exclusive prefix of tri over the rows: tile sums, their prefix, the rows
+constexpr int SCAN_TILE = 2048;
+
+__device__ __forceinline__ int64_t block_excl(int64_t v, int64_t* part, int64_t& total) {
+  const int ln = lane(), wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  int64_t x = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int64_t y = (int64_t)__shfl_up((unsigned long long)x, o);
+    if (ln >= o) x += y;
+  }
+  __syncthreads();
+  if (ln == 63) part[wv] = x;
+  __syncthreads();
+  int64_t base = 0;
+  total = 0;
+  for (int k = 0; k < nw; ++k) {
+    if (k < wv) base += part[k];
+    total += part[k];
+  }
+  return base + x - v;
+}
+
+__global__ void __launch_bounds__(256) k_scan_tiles(const int32_t* tri, int64_t n, int64_t* tiles) {
+  __shared__ int64_t part[4];
+  const int64_t b = (int64_t)blockIdx.x * SCAN_TILE + threadIdx.x * 8;
+  int64_t s = 0, total;
+  for (int k = 0; k < 8; ++k) s += b + k < n ? tri[b + k] : 0;
+  block_excl(s, part, total);
+  if (threadIdx.x == 0) tiles[blockIdx.x] = total;
+}
+
+__global__ void __launch_bounds__(1024) k_scan_tops(int64_t* tiles, int64_t nt) {
+  __shared__ int64_t part[16];
+  int64_t run = 0;
+  for (int64_t b = 0; b < nt; b += 1024) {
+    const int64_t i = b + threadIdx.x;
+    int64_t total;
+    const int64_t x = block_excl(i < nt ? tiles[i] : 0, part, total);
+    if (i < nt) tiles[i] = run + x;
+    run += total;
+  }
+}
+
+__global__ void __launch_bounds__(256) k_scan_rows(const int32_t* tri, int64_t n, const int64_t* tiles, int64_t* rp) {
+  __shared__ int64_t part[4];
+  const int64_t b = (int64_t)blockIdx.x * SCAN_TILE + threadIdx.x * 8;
+  int64_t s = 0, total;
+  int32_t t[8];
+  for (int k = 0; k < 8; ++k) {
+    t[k] = b + k < n ? tri[b + k] : 0;
+    s += t[k];
+  }
+  int64_t run = tiles[blockIdx.x] + block_excl(s, part, total);
+  for (int k = 0; k < 8; ++k) {
+    if (b + k < n) rp[b + k] = run;
+    run += t[k];
+    if (b + k == n - 1) rp[n] = run;
+  }
+}
+
+// A wave per row: the members of M = N(v0) that N(u) holds, in order.  Tests
+// M's members against u when u is a hub or its list is not much shorter than
+// M, else searches u's list in M.
+__global__ void __launch_bounds__(256) k_ego_fill(TriArgs a, EgoArgs g) {
+  const Adj A(a);
+  const int ln = lane();
+  const int64_t nw = (int64_t)gridDim.x * 4;
+  for (int64_t k = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); k < g.n; k += nw) {
+    const int64_t e = g.e0 + k;
+    if (g.tri[e] == 0) continue;
+    const int32_t v0 = uni(g.src[e]), u = uni(a.ci[e]);
+    const int64_t b = a.rp[v0], ub = a.rp[u];
+    const int d = (int)(a.rp[v0 + 1] - b), du = (int)(a.rp[u + 1] - ub);
+    const int32_t* M = a.ci + b;
+    const int32_t* N = a.ci + ub;
+    const uint32_t* bm = A.bitmap(u);
+    const bool over_m = bm ? d <= 16 * du : d <= 2 * du;
+    const int32_t base = (int32_t)(b - g.e0);
+    int64_t at = g.rp[k];
+    const int n = over_m ? d : du;
+    for (int i0 = 0; i0 < n; i0 += 64) {
+      const int i = i0 + ln;
+      bool f = false;
+      int p = i;
+      if (i < n) {
+        if (over_m) {
+          f = bm ? bit(bm, M[i]) : in_list(N, du, M[i]);
+        } else {
+          const int32_t y = N[i];
+          p = lb(M, d, y);
+          f = p < d && M[p] == y;
+        }
+      }
+      const uint64_t mk = __ballot(f);
+      if (f) {
+        const int64_t o = at + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mk >> 32),
+                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)mk, 0u));
+        g.ci[o] = base + p;
+        g.row[o] = (int32_t)k;
+      }
+      at += __popcll(mk);
+    }
+  }
+}
+
+// P10's part over the rows: for (v0, u), the pairs x, y of its entries with
+// (t(v0, x) - 1)(t(v0, y) - 1).  A wave per row.
+__global__ void __launch_bounds__(256) k_p10_rows(EgoArgs g, uint64_t* out) {
+  const int ln = lane();
+  const int64_t nw = (int64_t)gridDim.x * 4;
+  uint64_t acc = 0;
+  for (int64_t k = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); k < g.n; k += nw) {
+    const int64_t b = g.rp[k], e = g.rp[k + 1];
+    if (e - b < 2) continue;
+    uint64_t s = 0, s2 = 0;
+    for (int64_t i = b + ln; i < e; i += 64) {
+      const uint64_t x = (uint64_t)(g.tri[g.e0 + g.ci[i]] - 1);
+      s += x;
+      s2 += x * x;
+    }
+    s = wave_sum_u64(s);
+    s2 = wave_sum_u64(s2);
+    acc += (uint64_t)(((unsigned __int128)s * s - s2) >> 1);
+  }
+  if (ln == 0 && acc) atomicAdd((unsigned long long*)out, (unsigned long long)acc);
+}
+
+// The closed parts of P4 and P6 per edge (v0, v1), v1 < v0, with s common
+// neighbours: P4 (mode 0) -s (d0 + d1 - 1), and for a whole graph (mode 1) the
+// triangle part too, which then sums to -2 s (s - 1); P6 (mode 2) -2 C(s, 2).
+__global__ void __launch_bounds__(256) k_edge_base(const int64_t* rp, const int32_t* ci, const int32_t* src,
+                                                   const int32_t* tri, int64_t e0, int64_t e1, int mode, uint64_t* out) {
+  uint64_t acc = 0;
+  for (int64_t e = e0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < e1; e += (int64_t)gridDim.x * blockDim.x) {
+    const int32_t v0 = src[e], v1 = ci[e];
+    const int64_t s = tri[e];
+    if (v1 >= v0 || s == 0) continue;
+    if (mode == 2) {
+      acc -= (uint64_t)(s * (s - 1));
+    } else {
+      const int64_t d = (rp[v0 + 1] - rp[v0]) + (rp[v1 + 1] - rp[v1]);
+      acc -= (uint64_t)(s * (d - 1)) + (mode == 1 ? (uint64_t)(2 * s * (s - 1)) : 0ull);
+    }
+  }
+  acc = wave_sum_u64(acc);
+  if (lane() == 0 && acc) atomicAdd((unsigned long long*)out, (unsigned long long)acc);
+}
+
+// sum of tri over each vertex's edges
+__global__ void __launch_bounds__(256) k_root_tri(const int64_t* rp, const int32_t* tri, int32_t nv, int64_t* sum) {
+  const int64_t nw = (int64_t)gridDim.x * 4;
+  for (int64_t v = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); v < nv; v += nw) {
+    int64_t s = 0;
+    for (int64_t e = rp[v] + lane(); e < rp[v + 1]; e += 64) s += tri[e];
+    s = symd::wsum64(s);
+    if (lane() == 0) sum[v] = s;
+  }
+}
+
+// grid of a kernel with a wave per item, 4 waves per block
+unsigned item_grid(int64_t items, int num_cu) {
+  const int64_t blocks = (items + 3) / 4;
+  return (unsigned)(blocks < (int64_t)num_cu * 8 ? (blocks > 0 ? blocks : 1) : (int64_t)num_cu * 8);
+}
+
 template <int P>
 hipError_t launch_sum(const TriArgs& a, int num_cu, int gblocks, hipStream_t st) {
   hipLaunchKernelGGL(k_tri_reset, dim3(1), dim3(64), 0, st, a.ctr);
@@ -586,8 +769,42 @@ hipError_t launch_tri_build(const TriArgs& a, int32_t* dtri, const int32_t* src,
   return hipGetLastError();
 }
 
+int64_t ego_tiles(int64_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE; }
+
+hipError_t launch_ego_build(const TriArgs& a, const EgoArgs& g, int num_cu, hipStream_t st) {
+  if (g.n <= 0) return hipSuccess;
+  const int64_t nt = ego_tiles(g.n);
+  const int32_t* tri = g.tri + g.e0;
+  hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)nt), dim3(256), 0, st, tri, g.n, g.tiles);
+  hipLaunchKernelGGL(k_scan_tops, dim3(1), dim3(1024), 0, st, g.tiles, nt);
+  hipLaunchKernelGGL(k_scan_rows, dim3((unsigned)nt), dim3(256), 0, st, tri, g.n, g.tiles, g.rp);
+  hipLaunchKernelGGL(k_ego_fill, dim3(item_grid(g.n, num_cu)), dim3(256), 0, st, a, g);
+  return hipGetLastError();
+}
+
+hipError_t launch_p10_rows(const EgoArgs& g, uint64_t* out, int num_cu, hipStream_t st) {
+  hipLaunchKernelGGL(k_p10_rows, dim3(item_grid(g.n, num_cu)), dim3(256), 0, st, g, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_edge_base(const int64_t* rp, const int32_t* ci, const int32_t* src, const int32_t* tri, int64_t e0,
+                            int64_t e1, int mode, uint64_t* out, int num_cu, hipStream_t st) {
+  if (e1 <= e0) return hipSuccess;
+  const int64_t blocks = (e1 - e0 + 255) / 256;
+  hipLaunchKernelGGL(k_edge_base, dim3((unsigned)(blocks < num_cu * 8 ? blocks : num_cu * 8)), dim3(256), 0, st, rp, ci,
+                     src, tri, e0, e1, mode, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_root_tri(const int64_t* rp, const int32_t* tri, int32_t nv, int64_t* sum, int num_cu, hipStream_t st) {
+  hipLaunchKernelGGL(k_root_tri, dim3(item_grid(nv, num_cu)), dim3(256), 0, st, rp, tri, nv, sum);
+  return hipGetLastError();
+}
+
 hipError_t launch_tri_sum(int p, const TriArgs& a, int num_cu, int gblocks, hipStream_t st) {
   switch (p) {
+    case 4: return launch_sum<4>(a, num_cu, gblocks, st);
+    case 10: return launch_sum<10>(a, num_cu, gblocks, st);
     case 5: return launch_sum<5>(a, num_cu, gblocks, st);
     case 7: return launch_sum<7>(a, num_cu, gblocks, st);
     case 9: return launch_sum<9>(a, num_cu, gblocks, st);

@@ -1,20 +1,33 @@
-// p1_wedge.hip — 4-cycles (P1) by wedge counting, for single queries and for
-// every 4-cycle query of a batch in the same launches.
+// wedge.hip — patterns counted by wedges: 4-cycles (P1; single queries and
+// every 4-cycle query of a batch in the same launches), P4, P6 and P8.
 //
-// The reference's per-edge value (edges (v0, v1), v1 < v0: sum over v2 in
-// N(v0), v2 < v1, of |N(v1) ∩ N(v2) ∩ [0, v0)|;
-// src/message_passing_gpu_kernels.cuh:104-186) summed over a root's edges is
-//   sum over x < v0 of C(c_x, 2),  c_x = |{v in N(v0) : v < v0, x in N(v)}|:
-// every pair v2 < v1 of the c_x such v with the common neighbour x is one
-// term.  So a root needs one pass over its wedges (v0, v, x) with v, x < v0.
-// The sum needs no second pass over the counters: an increment that finds the
-// value k closes k pairs, so adding up what the increments return gives
-// sum C(c_x, 2).
+// A root has a set of lists; c_x is the number of them that hold the id x.
+//  * P1.  The reference's per-edge value (edges (v0, v1), v1 < v0: sum over v2
+//    in N(v0), v2 < v1, of |N(v1) ∩ N(v2) ∩ [0, v0)|;
+//    src/message_passing_gpu_kernels.cuh:104-186) summed over a root's edges is
+//      sum over x < v0 of C(c_x, 2),  lists N(v) ∩ [0, v0), v in N(v0), v < v0:
+//    every pair v2 < v1 of the c_x such v with the common neighbour x is one
+//    term.
+//  * P8 (:734-818: v1, v2, v3 and x in N(v0), v2 and v3 adjacent to v1, x to v2's
+//    and v3's side, v1 the largest and x < v2) is the 4-cycle count of the
+//    graph that N(v0) induces, with v1 as its root.  The induced graphs of all
+//    roots are laid out as one graph whose vertices are the directed edges
+//    (v0, u) (launch_ego_build), so P8 is P1 on that graph.
+//  * P6 (:573-652: pairs of S = N(v0) ∩ N(v1), v1 < v0, and a common
+//    neighbour of the pair other than v0 and v1): a root is an edge, its lists
+//    are N(v), v in S, and the value is sum over x of C(c_x, 2) less C(|S|, 2)
+//    for each of x = v0 and x = v1, where c_x = |S|.
+//  * P4 (:361-447): lists N(u), u in N(v0); the edge (v0, v1) with s common
+//    neighbours adds s times sum over x in N(v1) of c_x (less terms of the
+//    triangle counts alone, added elsewhere): a second pass over the lists.
+// The sum of C(c_x, 2) needs no second pass over the counters: an increment
+// that finds the value k closes k pairs, so adding up what the increments
+// return gives it.
 //
 // Four launches:
 //   k_p1_reset     counters and per-root sums to zero (a kernel: capturable)
-//   k_p1_len       per edge (v0, v), v < v0: |{x in N(v): x < v0}|, and per
-//                  root the sum W (its wedges) and the number of such v
+//   k_p1_len       per list its length (P1, P8: of the part below the root),
+//                  and per root the sum W (its wedges) and the number of lists
 //   k_p1_classify  roots into lists by W: wave tasks, block tasks, and block
 //                  tasks cut into P1_PARTS ranges of x
 //   p1_kernel      persistent; block tasks first (the long ones), then wave
@@ -27,11 +40,13 @@
 // up to 8192 wedges, the window's width chosen from the wedges it holds.
 //
 // What bounds it: the latency of the list loads behind the LDS segment cursor
-// and the LDS atomics; every list is read once (R-MAT 18: 8.6e8 wedges, 3.5 GB
-// of list elements in 3.1 ms, 1.1 TB/s).  One wave per root with a 32 KB table
-// of its own held a CU to 4 waves, and roots above 16384 wedges counted in
-// global memory, twice: R-MAT 18 149 -> 3.1 ms, R-MAT 20 785 -> 17.5 ms,
-// 3.8M-vertex Chung-Lu 178 -> 10 ms.
+// and the LDS atomics; every list is read once (R-MAT 18 P1: 8.6e8 wedges, 3.5
+// GB of list elements in 3.1 ms, 1.1 TB/s).  One wave per root with a 32 KB
+// table of its own held a CU to 4 waves, and roots above 16384 wedges counted
+// in global memory, twice: P1 on R-MAT 18 149 -> 3.1 ms, R-MAT 20 785 -> 17.5
+// ms, 3.8M-vertex Chung-Lu 178 -> 10 ms.  With an intersection per pair of the
+// nest: P4 on R-MAT 14 152 -> 1.1 ms, P6 on R-MAT 11 282 -> 0.59, P8 on R-MAT 12
+// 384 -> 0.88, P10 on R-MAT 10 173 -> 0.46.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -60,6 +75,7 @@ constexpr int P1_PARTS = 16;           // x ranges of a split root
 constexpr uint64_t P1_SPLIT = 1ull << 19;
 constexpr uint32_t P1_EMPTY = 0xffffffffu;
 
+enum { W_P1 = WEDGE_P1, W_P4 = WEDGE_P4, W_P6 = WEDGE_P6 };  // P8 is W_P1 on another graph
 enum { C_WAVE = 0, C_BLOCK = 1, C_SPLIT = 2, C_POPB = 3, C_POPW = 4 };
 
 // A table slot is one word (key << cb | count) when the ids of the window
@@ -82,12 +98,23 @@ __device__ __forceinline__ int find_prefix(const int64_t* cs, int n, int64_t t) 
   return lo;
 }
 
+// the ids x of a root: [first, end); its lists are sorted over them
+__device__ __forceinline__ int64_t first_id(const P1Q& Q, int32_t root) {
+  return Q.csrc ? Q.crp[Q.csrc[root]] - Q.cbase : Q.xmin;
+}
+template <int M>
+__device__ __forceinline__ int64_t end_id(const P1Q& Q, int32_t root) { return M == W_P1 ? root : Q.xend; }
+
 __global__ void k_p1_reset(P1Args a) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < 8) a.ctr[i] = 0;
-  for (int64_t k = i; k < a.roots; k += (int64_t)gridDim.x * blockDim.x) a.W[k] = 0;
+  for (int64_t k = i; k < a.roots; k += (int64_t)gridDim.x * blockDim.x) {
+    a.W[k] = 0;
+    a.m0[k] = 0;
+  }
 }
 
+template <int M>
 __global__ void __launch_bounds__(256) k_p1_len(P1Args a) {
   const int64_t tile = blockIdx.x;
   const int qi = a.q ? find_prefix(a.tcs, a.nq, tile) : 0;
@@ -98,10 +125,22 @@ __global__ void __launch_bounds__(256) k_p1_len(P1Args a) {
     const int64_t e = Q.e0 + k;
     v0 = Q.src[e];
     const int32_t v = Q.ci[e];
-    if (v < v0) {
-      const int64_t b = Q.rp[v];
-      len = lb(Q.ci + b, (int)(Q.rp[v + 1] - b), v0);  // x < v0
-      if (e + 1 == Q.rp[v0 + 1] || Q.ci[e + 1] > v0) a.m0[Q.roff + v0 - Q.rb] = (int32_t)(e + 1 - Q.rp[v0]);
+    if constexpr (M == W_P1) {
+      if (v < v0) {
+        const int64_t b = Q.rp[v];
+        len = lb(Q.ci + b, (int)(Q.rp[v + 1] - b), v0);  // x < v0
+        if (e + 1 == Q.rp[v0 + 1] || Q.ci[e + 1] > v0) a.m0[Q.roff + v0 - Q.rb] = (int32_t)(e + 1 - Q.rp[v0]);
+      }
+    } else if constexpr (M == W_P4) {  // every list; only roots with a triangle on an edge to a smaller id
+      len = (int32_t)(Q.rp[v + 1] - Q.rp[v]);
+      if (v < v0 && Q.weight[e] > 0) a.m0[Q.roff + v0 - Q.rb] = (int32_t)(Q.rp[v0 + 1] - Q.rp[v0]);
+    } else {  // W_P6: v0 is an edge, v the edge to a member of S
+      const int32_t s = (int32_t)(Q.rp[v0 + 1] - Q.rp[v0]);
+      if (s >= 2 && Q.vid[v0] < Q.csrc[v0]) {
+        const int32_t y = Q.vid[v];
+        len = (int32_t)(Q.lrp[y + 1] - Q.lrp[y]);
+        if (e == Q.rp[v0]) a.m0[Q.roff + v0 - Q.rb] = s;
+      }
     }
     a.len[Q.eoff + k] = len;
   }
@@ -120,6 +159,7 @@ __global__ void __launch_bounds__(256) k_p1_len(P1Args a) {
     atomicAdd((unsigned long long*)&a.W[Q.roff + v0 - Q.rb], (unsigned long long)s);
 }
 
+template <int M>
 __global__ void __launch_bounds__(256) k_p1_classify(P1Args a) {
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int ln = lane();
@@ -128,11 +168,13 @@ __global__ void __launch_bounds__(256) k_p1_classify(P1Args a) {
   if (t < a.roots) {
     const int64_t i = a.roots - 1 - t;  // a relabelled graph ranks its widest roots last: list them first
     const uint64_t w = a.W[i];
-    if (w >= 2) {  // else no two wedges share an endpoint
+    const int m0 = a.m0[i];
+    if (w >= (M == W_P4 ? 1 : 2) && m0 > 0) {  // else no two wedges share an endpoint
       item.y = a.q ? find_prefix(a.rcs, a.nq, i) : 0;
-      const int64_t rb = a.q ? a.q[item.y].rb : a.one.rb, roff = a.q ? a.q[item.y].roff : a.one.roff;
-      item.x = (int32_t)(rb + i - roff);
-      const int cap = table_cap(P1_SLICE, packed_bits(item.x, a.m0[i]));
+      const P1Q& Q = a.q ? a.q[item.y] : a.one;
+      item.x = (int32_t)(Q.rb + i - Q.roff);
+      const int64_t span = end_id<M>(Q, item.x) - (M == W_P1 && Q.csrc ? first_id(Q, item.x) : 0);
+      const int cap = table_cap(P1_SLICE, packed_bits(span, m0));
       cls = w <= (uint64_t)cap ? C_WAVE : w <= P1_SPLIT ? C_BLOCK : C_SPLIT;
     }
   }
@@ -154,7 +196,8 @@ __global__ void __launch_bounds__(256) k_p1_classify(P1Args a) {
 }
 
 // The segments of up to 64 neighbours (lane l: len elements from ci[base]) as
-// one flattened stream, four loads in flight per lane; f(x) for every element.
+// one flattened stream, four loads in flight per lane; f(x, i) for every
+// element x of lane i's segment.
 template <class F>
 __device__ __forceinline__ void stream64(const int32_t* ci, int64_t base, int len, int32_t* off, int64_t* lbase, F f) {
   const int ln = lane();
@@ -168,17 +211,19 @@ __device__ __forceinline__ void stream64(const int32_t* ci, int64_t base, int le
   int i = 0;
   for (int f0 = ln; f0 < T; f0 += 256) {
     int32_t x[4];
+    int seg[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int fe = f0 + 64 * u;
       if (fe < T) {
         i = seg_advance(off, 64, i, fe);
+        seg[u] = i;
         x[u] = ci[lbase[i] + fe];
       }
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      if (f0 + 64 * u < T) f(x[u]);
+      if (f0 + 64 * u < T) f(x[u], seg[u]);
   }
 }
 
@@ -210,6 +255,14 @@ __device__ __forceinline__ uint32_t table_count(uint32_t* tab, int lt, int cb, u
   }
 }
 
+// the wedges to x counted in such a table (x is in it)
+__device__ __forceinline__ uint32_t table_get(const uint32_t* tab, int lt, int cb, uint32_t x) {
+  uint32_t h = (x * 2654435761u) >> (32 - lt);
+  const uint32_t mask = (1u << lt) - 1;
+  while ((cb ? tab[h] >> cb : tab[h]) != x) h = (h + 1) & mask;
+  return cb ? tab[h] & ((1u << cb) - 1) : tab[mask + 1 + h];
+}
+
 // empties such a table (t4: its words as 16-byte groups), thread t of nt
 __device__ __forceinline__ void table_clear(uint4* t4, int lt, int cb, int t, int nt) {
   const int g = (1 << lt) / 4;
@@ -232,10 +285,14 @@ __device__ __forceinline__ void lb_many(const int32_t* l, int n, const int32_t (
   }
 }
 
+template <int M>
 __global__ void __launch_bounds__(64 * P1_WAVES) p1_kernel(P1Args a) {
+  constexpr bool TWO = M == W_P4;  // a second pass over the lists reads the counters
+
   __shared__ __attribute__((aligned(16))) uint32_t s_tab[P1_TAB];
   __shared__ int32_t s_off[P1_WAVES][65];
   __shared__ int64_t s_lb[P1_WAVES][64];
+  __shared__ int32_t s_wt[TWO ? P1_WAVES : 1][64];
   __shared__ int64_t s_task;
   __shared__ unsigned long long s_tot[3];
   __shared__ int s_next;
@@ -245,11 +302,12 @@ __global__ void __launch_bounds__(64 * P1_WAVES) p1_kernel(P1Args a) {
   const int ln = lane();
   int32_t* off = s_off[wv];
   int64_t* lbs = s_lb[wv];
+  int32_t* const wts = s_wt[TWO ? wv : 0];
   uint64_t acc = 0;
   int slot = 0;  // the query that acc belongs to
   auto flush = [&](int next) {
     if (next == slot) return;
-    const uint64_t s = wave_sum_u64(acc);
+    const uint64_t s = wave_sum_u64(acc) * (uint64_t)(a.q ? 1 : a.one.scale);
     if (ln == 0 && s) atomicAdd((unsigned long long*)(a.out + slot), (unsigned long long)s);
     acc = 0;
     slot = next;
@@ -268,16 +326,19 @@ __global__ void __launch_bounds__(64 * P1_WAVES) p1_kernel(P1Args a) {
     const int2 it = part ? a.split[t / P1_PARTS] : a.list[a.roots - 1 - (t - nsplit)];
     const P1Q Q = a.q ? a.q[it.y] : a.one;
     flush(Q.slot);
-    const int32_t* ci = Q.ci;
+    const int32_t* ci = M == W_P6 ? Q.lci : Q.ci;  // the lists' elements
     const int32_t v0 = it.x;
     const int64_t b0 = Q.rp[v0];
-    const int32_t* N0 = ci + b0;
+    const int32_t* N0 = Q.ci + b0;
+    // start of the j-th list
+    auto list_at = [&](int j) -> int64_t { return M == W_P6 ? Q.lrp[Q.vid[N0[j]]] : Q.rp[N0[j]]; };
     // neighbours below the window's end, per list; a root that is one task
     // moves them down as its windows descend
     int32_t* lens = a.len + Q.eoff + (b0 - Q.e0);
     const int m0 = a.m0[Q.roff + v0 - Q.rb];
     const uint64_t W = a.W[Q.roff + v0 - Q.rb];
-    int64_t xlo = Q.xmin, xhi = v0;  // ids below xmin have one neighbour: they close no pair
+    int64_t xlo = M == W_P6 ? 0 : first_id(Q, v0), xhi = end_id<M>(Q, v0);
+    const int64_t xend = xhi;
     if (part) {
       const int64_t span = xhi - xlo;
       const int p = (int)(t % P1_PARTS);
@@ -313,7 +374,7 @@ __global__ void __launch_bounds__(64 * P1_WAVES) p1_kernel(P1Args a) {
             const int n = lens[j];
             if (!n) continue;
             int pos[3];
-            lb_many<3>(ci + Q.rp[N0[j]], n, y, pos);
+            lb_many<3>(ci + list_at(j), n, y, pos);
 #pragma unroll
             for (int k = 0; k < 3; ++k) c[k] += n - pos[k];
           }
@@ -357,38 +418,67 @@ __global__ void __launch_bounds__(64 * P1_WAVES) p1_kernel(P1Args a) {
       }
       __syncthreads();
       const int32_t lo32 = (int32_t)lo;
-      for (;;) {
-        const int jb = wave_take(&s_next, cs);
-        if (jb >= m0) break;
-        const int j = jb + ln;
-        int len = 0;
-        int64_t base = 0;
-        if (ln < cs && j < m0) {
-          int n = lens[j];
-          if (n) {
-            base = Q.rp[N0[j]];
-            if (part && hi < v0) n = lb(ci + base, n, (int32_t)hi);
-            const int s = lo32 > 0 ? lb(ci + base, n, lo32) : 0;
-            if (!part) lens[j] = s;
-            len = n - s;
-            base += s;
+      for (int pass = 0; pass < (TWO ? 2 : 1); ++pass) {
+        if (pass) {
+          __syncthreads();
+          if (tid == 0) s_next = 0;
+          __syncthreads();
+        }
+        const bool last = !TWO || pass == 1;
+        for (;;) {
+          const int jb = wave_take(&s_next, cs);
+          if (jb >= m0) break;
+          const int j = jb + ln;
+          int len = 0;
+          int64_t base = 0;
+          if (ln < cs && j < m0) {
+            int n = lens[j];
+            if (n) {
+              base = list_at(j);
+              if (part && hi < xend) n = lb(ci + base, n, (int32_t)hi);
+              const int s = lo32 > 0 ? lb(ci + base, n, lo32) : 0;
+              if (!part && last) lens[j] = s;
+              len = n - s;
+              base += s;
+            }
           }
-        }
-        if (!part) {
-          const int w = (int)wave_sum_u64((uint64_t)len);
-          if (ln == 0 && w) atomicAdd(&s_tot[0], (unsigned long long)w);
-        }
-        if (dense) {
-          if (wide) {
-            stream64(ci, base, len, off, lbs, [&](int32_t x) { acc += atomicAdd(&s_tab[x - lo32], 1u); });
+          if (!part && last) {
+            const int w = (int)wave_sum_u64((uint64_t)len);
+            if (ln == 0 && w) atomicAdd(&s_tot[0], (unsigned long long)w);
+          }
+          if (TWO && pass) {
+            // the edge to a smaller id with s common neighbours: s times the
+            // counts of its list's elements
+            int32_t wt = 0;
+            if (len && N0[j] < v0) wt = Q.weight[b0 + j];
+            if (wt == 0) len = 0;
+            wts[ln] = wt;
+            stream64(ci, base, len, off, lbs, [&](int32_t x, int i) {
+              const uint32_t k = (uint32_t)(x - lo32);
+              const uint32_t c = !dense ? table_get(s_tab, lt, cb, k)
+                                 : wide ? s_tab[k]
+                                        : (s_tab[k >> 1] >> ((k & 1u) * 16u)) & 0xffffu;
+              acc += (uint64_t)wts[i] * c;
+            });
+          } else if (dense) {
+            if (wide) {
+              stream64(ci, base, len, off, lbs, [&](int32_t x, int) {
+                const uint32_t c = atomicAdd(&s_tab[x - lo32], 1u);
+                if (!TWO) acc += c;
+              });
+            } else {
+              stream64(ci, base, len, off, lbs, [&](int32_t x, int) {
+                const uint32_t i = (uint32_t)(x - lo32), sh = (i & 1u) * 16u;
+                const uint32_t c = (atomicAdd(&s_tab[i >> 1], 1u << sh) >> sh) & 0xffffu;
+                if (!TWO) acc += c;
+              });
+            }
           } else {
-            stream64(ci, base, len, off, lbs, [&](int32_t x) {
-              const uint32_t i = (uint32_t)(x - lo32), sh = (i & 1u) * 16u;
-              acc += (atomicAdd(&s_tab[i >> 1], 1u << sh) >> sh) & 0xffffu;
+            stream64(ci, base, len, off, lbs, [&](int32_t x, int) {
+              const uint32_t c = table_count(s_tab, lt, cb, (uint32_t)(x - lo32));
+              if (!TWO) acc += c;
             });
           }
-        } else {
-          stream64(ci, base, len, off, lbs, [&](int32_t x) { acc += table_count(s_tab, lt, cb, (uint32_t)(x - lo32)); });
         }
       }
       if (!part) {
@@ -419,16 +509,33 @@ __global__ void __launch_bounds__(64 * P1_WAVES) p1_kernel(P1Args a) {
       const int32_t* lens = a.len + Q.eoff + (b0 - Q.e0);
       const int m0 = a.m0[Q.roff + v0 - Q.rb];
       const int W = (int)a.W[Q.roff + v0 - Q.rb];
-      const int cb = packed_bits(v0, m0);
+      const int32_t xlo = M == W_P1 && Q.csrc ? (int32_t)first_id(Q, v0) : 0;
+      const int cb = packed_bits(end_id<M>(Q, v0) - xlo, m0);
       int lt = 6;
       while ((1 << lt) < 2 * W) ++lt;
       __syncwarp();
       table_clear(reinterpret_cast<uint4*>(tab), lt, cb, ln, 64);
-      for (int jb = 0; jb < m0; jb += 64) {
-        const int j = jb + ln;
-        const int len = j < m0 ? lens[j] : 0;
-        const int64_t base = len ? Q.rp[Q.ci[b0 + j]] : 0;
-        stream64(Q.ci, base, len, off, lbs, [&](int32_t x) { acc += table_count(tab, lt, cb, (uint32_t)x); });
+      for (int pass = 0; pass < (TWO ? 2 : 1); ++pass) {
+        for (int jb = 0; jb < m0; jb += 64) {
+          const int j = jb + ln;
+          int len = j < m0 ? lens[j] : 0;
+          const int32_t v = len ? Q.ci[b0 + j] : 0;
+          const int64_t base = len ? (M == W_P6 ? Q.lrp[Q.vid[v]] : Q.rp[v]) : 0;
+          const int32_t* ci = M == W_P6 ? Q.lci : Q.ci;
+          if (TWO && pass) {
+            const int32_t wt = len && v < v0 ? Q.weight[b0 + j] : 0;
+            if (wt == 0) len = 0;
+            wts[ln] = wt;
+            stream64(ci, base, len, off, lbs, [&](int32_t x, int i) {
+              acc += (uint64_t)wts[i] * table_get(tab, lt, cb, (uint32_t)x);
+            });
+          } else {
+            stream64(ci, base, len, off, lbs, [&](int32_t x, int) {
+              const uint32_t c = table_count(tab, lt, cb, (uint32_t)(x - xlo));
+              if (!TWO) acc += c;
+            });
+          }
+        }
       }
     }
   }
@@ -456,15 +563,27 @@ void p1_bind_scratch(P1Args& a, void* p) {
   a.len = reinterpret_cast<int32_t*>(b);
 }
 
-hipError_t launch_p1(const P1Args& a, int num_cu, hipStream_t st) {
+template <int M>
+static hipError_t launch_wedge_m(const P1Args& a, int num_cu, hipStream_t st) {
   if (a.tiles <= 0 || a.roots <= 0) return hipSuccess;
   const unsigned rblocks = (unsigned)((a.roots + 255) / 256);
   hipLaunchKernelGGL(k_p1_reset, dim3(rblocks < 1024u ? rblocks : 1024u), dim3(256), 0, st, a);
-  hipLaunchKernelGGL(k_p1_len, dim3((unsigned)a.tiles), dim3(256), 0, st, a);
-  hipLaunchKernelGGL(k_p1_classify, dim3(rblocks), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(k_p1_len<M>, dim3((unsigned)a.tiles), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(k_p1_classify<M>, dim3(rblocks), dim3(256), 0, st, a);
   const int64_t want = (a.roots + P1_WAVES - 1) / P1_WAVES, most = (int64_t)num_cu * (16 / P1_WAVES);
-  hipLaunchKernelGGL(p1_kernel, dim3((unsigned)(want < most ? want : most)), dim3(64 * P1_WAVES), 0, st, a);
+  hipLaunchKernelGGL(p1_kernel<M>, dim3((unsigned)(want < most ? want : most)), dim3(64 * P1_WAVES), 0, st, a);
   return hipGetLastError();
+}
+
+hipError_t launch_p1(const P1Args& a, int num_cu, hipStream_t st) { return launch_wedge_m<W_P1>(a, num_cu, st); }
+
+hipError_t launch_wedge(int mode, const P1Args& a, int num_cu, hipStream_t st) {
+  switch (mode) {
+    case WEDGE_P1: return launch_wedge_m<W_P1>(a, num_cu, st);
+    case WEDGE_P4: return launch_wedge_m<W_P4>(a, num_cu, st);
+    case WEDGE_P6: return launch_wedge_m<W_P6>(a, num_cu, st);
+  }
+  return hipErrorInvalidValue;
 }
 
 }  // namespace jk
