@@ -66,23 +66,27 @@ clique_kernel(CliqueArgs a) {
   __shared__ int32_t s_wtot[G + 1];
   __shared__ int64_t s_task;
   const int slot = (G == 1) ? (int)(threadIdx.x >> 6) : 0;
-  const int ln = lane_id();
   unsigned char* ar = s_arena[slot];
   uint64_t* rowp = LROWS ? reinterpret_cast<uint64_t*>(ar + LY::R_OFF)
                          : (a.gscr + (int64_t)blockIdx.x * DM * WMAX);
   const int64_t* __restrict__ rp = a.rp;
   uint64_t acc = 0;
-  for (;;) {
+  // a group's first tasks are its own index, the queue deals the others: the
+  // small launches end without a counter round trip
+  for (bool first = true;; first = false) {
     int64_t base;
     if constexpr (G == 1) {
-      int64_t t = 0;
-      if (ln == 0) t = (int64_t)atomicAdd(a.qctr, (unsigned)a.chunk);
-      base = __shfl(t, 0);
+      base = first ? ((int64_t)blockIdx.x * WPB + slot) * a.chunk
+                   : (int64_t)gridDim.x * WPB * a.chunk + (int64_t)wave_take(a.qctr, (uint32_t)a.chunk);
     } else {
-      if (threadIdx.x == 0) s_task = (int64_t)atomicAdd(a.qctr, 1u);
-      __syncthreads();
-      base = s_task;
-      __syncthreads();
+      if (first) {
+        base = blockIdx.x;
+      } else {
+        if (threadIdx.x == 0) s_task = (int64_t)gridDim.x + (int64_t)atomicAdd(a.qctr, 1u);
+        __syncthreads();
+        base = s_task;
+        __syncthreads();
+      }
     }
     if (base >= a.ntasks) break;
     const int64_t tend = min(a.ntasks, base + (G == 1 ? (int64_t)a.chunk : 1));
