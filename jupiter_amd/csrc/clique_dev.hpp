@@ -257,6 +257,13 @@ struct RowsGlobal {
   }
 };
 
+// Rows in global memory that many waves read again (cached loads).
+struct RowsCached {
+  const uint64_t* p;
+  RowLayout lay;
+  __device__ uint64_t operator()(int i, int w) const { return p[lay(i, w)]; }
+};
+
 // Block reduction of a per-thread uint64 and one atomicAdd per block.
 template <int NT>
 __device__ void block_add(uint64_t v, uint64_t* out) {
@@ -355,6 +362,256 @@ __device__ uint64_t recR(const uint64_t (&c)[WM], int wlo, int nw, const RowT& R
       }
     }
     return s;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Cliques of a DAG on up to 64 CW members, rows of CW words: lane l holds the
+// rows of members l, l + 64, ...  Counting them lane by member leaves most
+// lanes idle behind the first members' subtrees.  Up to 4-cliques the wave
+// walks the first members together instead, their rows and sets in scalar
+// registers, and the last set is the lane mask of a population count (about
+// 35 issue cycles per edge, no memory access).  Deeper, the unit is an edge
+// j -> x (its common successors C[j] & C[x] start the search), the edges lie
+// in an LDS list, and a lane that runs out takes the next one.
+
+__device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int l) {
+  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)v, l);
+  const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(v >> 32), l);
+  return ((uint64_t)hi << 32) | lo;
+}
+__device__ __forceinline__ int below(uint64_t m) {  // set bits below this lane
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+constexpr int FLAT_LIST = 512;  // entries of a wave's edge list
+
+// Sum over the m edges of the list of the (LV + 1)-cliques among their common
+// successors (LV >= 2); the rows are in LDS (C[CW t + w]).  RANKED: rows only
+// have bits above their own position, so what is left of a set serves as the
+// set.  Each step reads one row per lane: of the next member of the lane's
+// deepest set.  Idle lanes take new edges together, once half have run out.
+template <int LV, int CW, bool RANKED>
+__device__ uint64_t flat_cliques(const uint64_t* C, const uint16_t* list, int m) {
+  uint64_t acc = 0;
+  uint64_t it[LV][CW], full[RANKED ? 1 : LV][CW];  // per level: members left, and the set
+#pragma unroll
+  for (int l = 0; l < LV; ++l)
+#pragma unroll
+    for (int w = 0; w < CW; ++w) {
+      it[l][w] = 0;
+      if (!RANKED) full[l][w] = 0;
+    }
+  auto empty = [&](int l) {
+    uint64_t x = it[l][0];
+#pragma unroll
+    for (int w = 1; w < CW; ++w) x |= it[l][w];
+    return x == 0;
+  };
+  auto idle = [&]() {
+    bool e = true;
+#pragma unroll
+    for (int l = 0; l < LV; ++l) e = e && empty(l);
+    return e;
+  };
+  int next = 0;  // next edge of the list (wave-uniform)
+  for (;;) {
+    const bool want = idle();
+    const uint64_t need = __ballot(want);
+    if (next >= m && need == ~0ull) break;
+    const int u = next + below(need);
+    next += __popcll(need);
+    if (want && u < m) {
+      const int e = list[u], j = e >> 8, x = e & 255;
+      int pc = 0;
+      uint64_t c[CW];
+#pragma unroll
+      for (int w = 0; w < CW; ++w) {
+        c[w] = C[CW * j + w] & C[CW * x + w];
+        pc += __popcll(c[w]);
+      }
+#pragma unroll
+      for (int w = 0; w < CW; ++w) {
+        it[0][w] = pc > LV ? c[w] : 0;
+        if (!RANKED) full[0][w] = it[0][w];
+      }
+    }
+    int live = __popcll(__ballot(!idle()));
+    const int stop = next < m ? live / 2 : 0;
+    while (live > stop) {
+      // the deepest set with members left, its next member z
+      int lv = -1, z = 0;
+      uint64_t base[CW] = {};
+#pragma unroll
+      for (int l = LV - 1; l >= 0; --l) {
+        if (lv < 0 && !empty(l)) {
+          lv = l;
+          bool got = false;
+#pragma unroll
+          for (int w = 0; w < CW; ++w) {
+            if (!got && it[l][w]) {
+              z = 64 * w + __builtin_ctzll(it[l][w]);
+              it[l][w] &= it[l][w] - 1;
+              got = true;
+            }
+          }
+#pragma unroll
+          for (int w = 0; w < CW; ++w) base[w] = RANKED ? it[l][w] : full[l][w];
+        }
+      }
+      if (lv >= 0) {
+        int pc = 0;
+        uint64_t v[CW];
+#pragma unroll
+        for (int w = 0; w < CW; ++w) {
+          v[w] = base[w] & C[CW * z + w];
+          pc += __popcll(v[w]);
+        }
+        if (lv == LV - 1) {
+          acc += (uint64_t)pc;
+        } else {
+#pragma unroll
+          for (int l = 1; l < LV; ++l) {
+            if (lv == l - 1) {
+#pragma unroll
+              for (int w = 0; w < CW; ++w) {
+                it[l][w] = pc > LV - l ? v[w] : 0;
+                if (!RANKED) full[l][w] = it[l][w];
+              }
+            }
+          }
+        }
+      }
+      live = __popcll(__ballot(!idle()));
+    }
+  }
+  return acc;
+}
+
+// sum over the members x of c (wave-uniform, no member below word q) of
+// |c & C[x]|, this lane's share: c is the lane mask of the count.  RANKED rows
+// have no bits in words below their own.
+template <int CW, bool RANKED>
+__device__ __forceinline__ uint32_t edges_within(const uint64_t (&c)[CW], const uint64_t (&row)[CW][CW], int q) {
+  uint32_t s = 0;
+#pragma unroll
+  for (int k = 0; k < CW; ++k) {
+    if (k < q) continue;
+    if (__builtin_amdgcn_inverse_ballot_w64(c[k])) {
+#pragma unroll
+      for (int w = 0; w < CW; ++w)
+        if (w >= (RANKED ? k : q)) s += (uint32_t)__popcll(c[w] & row[k][w]);
+    }
+  }
+  return s;
+}
+
+// M-cliques (M >= 3) whose first member is t0, t0 + ts, ... of the DAG on n <=
+// 64 CW members.  row[k] is this lane's row of member lane + 64 k; for M > 4
+// the rows are in LDS at C too, and list holds FLAT_LIST entries.  Every lane
+// of the wave calls this with uniform arguments.
+template <int M, int CW, bool RANKED>
+__device__ uint64_t count_cliques(const uint64_t (&row)[CW][CW], const uint64_t* C, uint16_t* list, int n, int t0 = 0,
+                                  int ts = 1) {
+  const int ln = lane_id();
+  uint64_t acc = 0;
+  uint32_t part = 0;  // at most 128^2 / 2 edges of at most 128 each
+  int m = 0;
+#pragma unroll
+  for (int k = 0; k < CW; ++k) {
+    const int ne = min(64, n - 64 * k);
+    for (int t = t0; t < ne; t += ts) {
+      // (RANKED: a row of word k has no bits in the words below)
+      uint64_t ct[CW];
+      int pc = 0;
+#pragma unroll
+      for (int w = 0; w < CW; ++w) {
+        ct[w] = RANKED && w < k ? 0 : readlane_u64(row[k][w], t);
+        pc += __popcll(ct[w]);
+      }
+      if (pc < M - 1) continue;
+      if constexpr (M == 3) {
+        part += edges_within<CW, RANKED>(ct, row, RANKED ? k : 0);
+      } else if constexpr (M == 4) {
+#pragma unroll
+        for (int q = 0; q < CW; ++q) {
+          if (RANKED && q < k) continue;
+          for (uint64_t b = ct[q]; b;) {
+            const int x = __builtin_ctzll(b);
+            b &= ~(1ull << x);
+            uint64_t c[CW];
+#pragma unroll
+            for (int w = 0; w < CW; ++w) c[w] = RANKED && w < q ? 0 : ct[w] & readlane_u64(row[q][w], x);
+            part += edges_within<CW, RANKED>(c, row, RANKED ? q : 0);
+          }
+        }
+      } else {
+        if (m + pc > FLAT_LIST) {
+          __syncwarp();
+          acc += flat_cliques<M - 3, CW, RANKED>(C, list, m);
+          __syncwarp();
+          m = 0;
+        }
+#pragma unroll
+        for (int q = 0; q < CW; ++q) {
+          if ((ct[q] >> ln) & 1ull) list[m + below(ct[q])] = (uint16_t)(((64 * k + t) << 8) | (64 * q + ln));
+          m += __popcll(ct[q]);
+        }
+      }
+    }
+  }
+  if constexpr (M > 4) {
+    __syncwarp();
+    if (m) acc += flat_cliques<M - 3, CW, RANKED>(C, list, m);
+    __syncwarp();
+  }
+  return acc + part;
+}
+
+// Rows of the DAG induced on the n <= 64 CW members J (ascending positions) of
+// R's DAG, as bitmaps over J: one ballot per member and word.  row[k] is the
+// row of member lane + 64 k; with out, all rows are written there.
+template <int CW, class RowT>
+__device__ void compress_rows(const RowT& R, const int16_t* J, int n, uint64_t (&row)[CW][CW], uint64_t* out) {
+  const int ln = lane_id();
+  int j[CW];
+#pragma unroll
+  for (int k = 0; k < CW; ++k) {
+    j[k] = 64 * k + ln < n ? (int)J[64 * k + ln] : -1;
+#pragma unroll
+    for (int w = 0; w < CW; ++w) row[k][w] = 0;
+  }
+  // U members at a time, so that their row loads overlap
+  constexpr int U = CW == 1 ? 8 : 4;
+#pragma unroll
+  for (int k = 0; k < CW; ++k) {
+    const int ne = min(64, n - 64 * k);
+    for (int tb = 0; tb < ne; tb += U) {
+      uint64_t v[U][CW];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int x = __builtin_amdgcn_readlane(j[k], min(tb + u, ne - 1));
+#pragma unroll
+        for (int w = 0; w < CW; ++w) v[u][w] = R(x, max(j[w], 0) >> 6);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int w = 0; w < CW; ++w) {
+          const uint64_t b = __ballot(j[w] >= 0 && ((v[u][w] >> (j[w] & 63)) & 1ull));
+          if (ln == tb + u) row[k][w] = b;
+        }
+      }
+    }
+  }
+  if (out) {
+#pragma unroll
+    for (int k = 0; k < CW; ++k)
+      if (64 * k + ln < n) {
+#pragma unroll
+        for (int w = 0; w < CW; ++w) out[CW * (64 * k + ln) + w] = row[k][w];
+      }
+    __syncwarp();
   }
 }
 
@@ -756,9 +1013,13 @@ struct Lay {
   static constexpr size_t B_RNK = al(B_KEY + (HBYTES > KBYTES ? HBYTES : KBYTES));  // int16 [DM] rank in DAG order
   static constexpr size_t B_END = al(B_RNK + (MULTI ? 2 * DM : 0));
   // count view, one slot of C_PW bytes per wave: the positions J of S
-  // (int16 [DM]) and the successor bitmap Rc (u64 [64])
-  static constexpr size_t C_RC = al(2 * (size_t)DM);
-  static constexpr size_t C_PW = MULTI ? C_RC + 8 * 64 : 0;
+  // (int16 [DM]), the successor bitmap Rc (u64 [64], or [128][2] where rows of
+  // up to 128 members are compressed) and an edge list
+  static constexpr bool FLAT = !BYTES && K >= 5 && WMAX <= 8;  // count_cliques on compressed rows
+  static constexpr bool FLAT_LISTED = FLAT && K - (MULTI ? 2 : 1) > 4;
+  static constexpr size_t C_RC = al(MULTI ? 2 * (size_t)DM : 0);
+  static constexpr size_t C_LIST = C_RC + (MULTI ? (FLAT_LISTED ? 8 * 256 : 8 * 64) : 0);
+  static constexpr size_t C_PW = MULTI || FLAT_LISTED ? C_LIST + (FLAT_LISTED ? 2 * FLAT_LIST : 0) : 0;
   static constexpr size_t C_END = al((size_t)G * C_PW);
   static constexpr size_t U_SIZE = (!CNT || B_END > C_END) ? B_END : C_END;  // CNT: the count view is used
   static constexpr size_t SLOT = al(U_OFF + U_SIZE);
@@ -968,10 +1229,12 @@ __device__ void process_root(const int64_t* __restrict__ rp, const int32_t* __re
   // ---- count (the build-phase region U is now free)
   if constexpr (!LY::MULTI) {
     // one word per row, lane i owns row i
-    if (r < d) {
-      const uint64_t Ri = rowp[r];
-      if constexpr (BYTES) acc += rec1<K - 3, true>(Ri, rowp, wL);
-      else acc += rec1<K - 2, false>(Ri, rowp, wL);
+    if constexpr (BYTES) {
+      if (r < d) acc += rec1<K - 3, true>(rowp[r], rowp, wL);
+    } else if constexpr (K >= 4) {
+      const uint64_t row[1][1] = {{ln < d ? rowp[ln] : 0ull}};
+      uint16_t* const list = reinterpret_cast<uint16_t*>(U + (size_t)wv * LY::C_PW + LY::C_LIST);
+      acc += count_cliques<K - 1, 1, false>(row, rowp, list, d, wv, G);
     }
   } else {
     using RowT = typename std::conditional<LROWS, RowsLds, RowsGlobal>::type;
@@ -1058,6 +1321,29 @@ __device__ void process_root(const int64_t* __restrict__ rp, const int32_t* __re
             uint64_t c = 0;
             for (int w = max(wlo, (j + 1) >> 6); w <= whi; ++w) c += __popcll(R(i, w) & R(j, w));
             acc += c;
+          }
+        }
+      } else if constexpr (LY::FLAT && !MMA5) {
+        // 5-cliques of the 128-wide roots, 6- and 7-cliques up to 512 wide:
+        // (K - 2)-cliques of the DAG on S, its rows compressed to S
+        if (n < K - 2) {
+        } else if (n <= 64) {
+          uint64_t row[1][1];
+          compress_rows<1>(R, J, n, row, LY::FLAT_LISTED ? Rc : nullptr);
+          acc += count_cliques<K - 2, 1, true>(row, Rc, reinterpret_cast<uint16_t*>(slot + LY::C_LIST), n);
+        } else if (n <= 128) {
+          uint64_t row[2][2];
+          compress_rows<2>(R, J, n, row, LY::FLAT_LISTED ? Rc : nullptr);
+          acc += count_cliques<K - 2, 2, true>(row, Rc, reinterpret_cast<uint16_t*>(slot + LY::C_LIST), n);
+        } else if constexpr (WMAX > 2) {
+          for (int t = ln; t < n; t += 64) {
+            const int j = J[t];
+            const int nw = whi - wlo + 1;
+            const int ws = ((j + 1) >> 6) - wlo;  // row j has no bits before its own position
+            uint64_t c[WMAX];
+#pragma unroll
+            for (int w = 0; w < WMAX; ++w) c[w] = (w >= ws && w < nw) ? (R(i, wlo + w) & R(j, wlo + w)) : 0ull;
+            acc += recR<K - 3, WMAX, false>(c, wlo, nw, R, wL);
           }
         }
       } else if (!MMA5 && n <= 64) {

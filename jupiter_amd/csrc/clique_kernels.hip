@@ -23,9 +23,9 @@
 //     step 1).  With d <= 64 every row is one 64-bit word and lane i counts
 //     the cliques starting at i with AND + popcount.  With d > 64, the rows
 //     are multi-word; for each i the wave compacts S = row i, and counts with
-//     word-wise AND/popcount (k = 4), the compressed |S| x |S| successor
-//     bitmap (k >= 5, |S| <= 64), fp4 matrix-core products (k = 5, wider S)
-//     or register word windows (k >= 6).
+//     word-wise AND/popcount (k = 4), fp4 matrix-core products (k = 5), or the
+//     rows compressed to S in registers (k = 5 on the 128-wide tier, k >= 6),
+//     the last set of a search being a lane mask (count_cliques).
 // Counts are exact uint64 (the matrix-core products are exact integers
 // below 2^24 in f32).
 #include <hip/hip_runtime.h>
@@ -191,6 +191,135 @@ hipError_t launch_clique_split(int k, bool build, const CliqueArgs& a, int grid,
 size_t split_slot_words() { return ROWW; }
 
 // ---------------------------------------------------------------------------
+// Split form of the 128- to 512-wide tiers for 6- and 7-cliques.  A root's
+// rows differ by orders of magnitude in the cliques below them, so a block per
+// root ended with a few blocks at work (R-MAT 16 P15: 1,834 128-wide roots, the
+// heaviest holding 0.3 % of the work, took 12.6 of 17 ms after the others).
+// Here the build leaves each root's rows in a global slot and the count takes
+// one (root, row) per wave, row by row over all roots: the heavy early rows
+// first.  A row's set is compressed to registers straight from the slot (L2).
+// P15 on R-MAT 16: 76 -> 12.9 ms, R-MAT 18: 528 -> 101 ms; an edge of a set costs
+// about 90 cycles of a SIMD (8 VALU and 6 SALU instructions, their latency and
+// the loop's branches), which bounds it.
+constexpr size_t rows_slot(int wmax) { return (size_t)64 * wmax * wmax; }
+
+template <int G, int WMAX>
+__global__ void __launch_bounds__(64 * G) clique_rows_build_kernel(CliqueArgs a) {
+  using LY = Lay<G, WMAX, 4, false, true, false>;
+  __shared__ __attribute__((aligned(16))) unsigned char s_arena[LY::SLOT];
+  __shared__ int32_t s_wtot[G + 1];
+  uint64_t* rowp = reinterpret_cast<uint64_t*>(s_arena + LY::R_OFF);
+  uint64_t acc = 0;
+  for (int64_t task = blockIdx.x; task < a.ntasks; task += gridDim.x) {
+    const int32_t v0 = a.ids[task];
+    const int64_t b0 = a.rp[v0];
+    const int d = (int)(a.rp[v0 + 1] - b0);
+    if (d < a.dmin || d > a.dmax || d > LY::DM) continue;
+    process_root<G, WMAX, 4, false, true, 1>(a.rp, a.ci, a.ord, b0, d, a.ratio, s_arena, rowp, s_wtot, acc);
+    const int n = d * RowLayout((d + 63) >> 6).S;
+    uint64_t* dst = a.gscr + (size_t)task * rows_slot(WMAX);
+    for (int t = threadIdx.x; t < n; t += 64 * G) dst[t] = rowp[t];
+    __syncthreads();
+  }
+}
+
+template <int K, int WMAX>
+__global__ void __launch_bounds__(256) clique_rows_count_kernel(CliqueArgs a) {
+  constexpr int DM = 64 * WMAX;
+  constexpr bool LIST = K - 2 > 4;
+  __shared__ int16_t s_J[4][DM];
+  __shared__ uint64_t s_rc[LIST ? 4 : 1][LIST ? 256 : 1];
+  __shared__ uint16_t s_list[LIST ? 4 : 1][LIST ? FLAT_LIST : 1];
+  const int wv = threadIdx.x >> 6;
+  const int ln = lane_id();
+  int16_t* const J = s_J[wv];
+  uint64_t* const rc = s_rc[LIST ? wv : 0];
+  uint16_t* const list = s_list[LIST ? wv : 0];
+  uint64_t acc = 0;
+  // the first quarter of the rows, which hold the wide sets, by PARTS waves
+  // each (a set of more than 64 members; else the first does it alone)
+  constexpr int PARTS = 4;
+  const int64_t nw = (int64_t)gridDim.x * 4, early = a.ntasks * (DM / 4) * PARTS;
+  for (int64_t t = (int64_t)blockIdx.x * 4 + wv; t < early + a.ntasks * (DM - DM / 4); t += nw) {
+    const int64_t u = t < early ? t / PARTS : t - early;
+    const int part = t < early ? (int)(t % PARTS) : 0;
+    const int i0 = (int)(u / a.ntasks);
+    const int64_t task = u - (int64_t)i0 * a.ntasks;
+    const int i = uni(t < early ? i0 : i0 + DM / 4);
+    const int32_t v0 = a.ids[task];
+    const int64_t b0 = a.rp[v0];
+    const int d = uni((int)(a.rp[v0 + 1] - b0));
+    if (i >= d || d < a.dmin || d > a.dmax || d > DM) continue;
+    const int W = (d + 63) >> 6;
+    const RowsCached R{a.gscr + (size_t)task * rows_slot(WMAX), RowLayout(W)};
+    // S = row i: its members' positions
+    const uint64_t myword = ln < W ? R(i, ln) : 0ull;
+    __syncwarp();
+    int n = 0;
+    for (int w = 0; w < W; ++w) {
+      const uint64_t word = readlane_u64(myword, w);
+      if ((word >> ln) & 1ull) J[n + below(word)] = (int16_t)((w << 6) | ln);
+      n += __popcll(word);
+    }
+    __syncwarp();
+    if (n < K - 2 || (n <= 64 && part > 0)) continue;
+    const int ps = t < early ? PARTS : 1;
+    if (n <= 64) {
+      uint64_t row[1][1];
+      compress_rows<1>(R, J, n, row, LIST ? rc : nullptr);
+      acc += count_cliques<K - 2, 1, true>(row, rc, list, n);
+    } else if (n <= 128) {
+      uint64_t row[2][2];
+      compress_rows<2>(R, J, n, row, LIST ? rc : nullptr);
+      acc += count_cliques<K - 2, 2, true>(row, rc, list, n, part, ps);
+    } else if (K == 6 && n <= 256) {
+      if constexpr (K == 6 && WMAX > 2) {
+        uint64_t row[4][4];
+        compress_rows<4>(R, J, n, row, nullptr);
+        acc += count_cliques<4, 4, true>(row, nullptr, nullptr, n, part, ps);
+      }
+    } else if constexpr (WMAX > 2) {
+      // lanes over the members: candidate sets in registers, rows from L2
+      for (int q = 64 * part + ln; q < n; q += 64 * ps) {
+        const int j = J[q];
+        const int ws = (j + 1) >> 6;  // row j has no bits before its own position
+        uint64_t c[WMAX];
+#pragma unroll
+        for (int w = 0; w < WMAX; ++w) c[w] = (w >= ws && w < W) ? (R(i, w) & R(j, w)) : 0ull;
+        acc += recR<K - 3, WMAX, false>(c, 0, W, R, nullptr);
+      }
+    }
+  }
+  block_add<256>(acc, a.out);
+}
+
+template <int K, int WMAX>
+static hipError_t launch_rows_w(bool build, const CliqueArgs& a, int num_cu, int maxgrid, hipStream_t st) {
+  constexpr int G = WMAX == 8 ? 8 : 4;
+  if (build)
+    hipLaunchKernelGGL((clique_rows_build_kernel<G, WMAX>), dim3((unsigned)(a.ntasks < maxgrid ? a.ntasks : maxgrid)),
+                       dim3(64 * G), 0, st, a);
+  else
+    hipLaunchKernelGGL((clique_rows_count_kernel<K, WMAX>), dim3(8 * num_cu), dim3(256), 0, st, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_clique_rows(int k, int tier, bool build, const CliqueArgs& a, int num_cu, int maxgrid,
+                              hipStream_t st) {
+  switch (k * 8 + tier) {
+    case 6 * 8 + TIER_LDS2: return launch_rows_w<6, 2>(build, a, num_cu, maxgrid, st);
+    case 6 * 8 + TIER_LDS4: return launch_rows_w<6, 4>(build, a, num_cu, maxgrid, st);
+    case 6 * 8 + TIER_LDS8: return launch_rows_w<6, 8>(build, a, num_cu, maxgrid, st);
+    case 7 * 8 + TIER_LDS2: return launch_rows_w<7, 2>(build, a, num_cu, maxgrid, st);
+    case 7 * 8 + TIER_LDS4: return launch_rows_w<7, 4>(build, a, num_cu, maxgrid, st);
+    case 7 * 8 + TIER_LDS8: return launch_rows_w<7, 8>(build, a, num_cu, maxgrid, st);
+  }
+  return hipErrorInvalidValue;
+}
+
+size_t rows_slot_words(int tier) { return rows_slot(tier == TIER_LDS2 ? 2 : tier == TIER_LDS4 ? 4 : 8); }
+
+// ---------------------------------------------------------------------------
 // Split form of the 2048-wide tier for 5- to 7-cliques.  The fused kernel
 // counts a root with one block of 8 waves (two per SIMD, the registers of
 // the 2x2 matrix-core tiles), so the roots of a query run about one per CU
@@ -281,6 +410,9 @@ size_t glb_slot_words() { return GSLOT; }
 
 // ---------------------------------------------------------------------------
 // Host-side launch table.
+// 6- and 7-clique roots up to this out-degree run one wave each.
+constexpr int SMALL_ROOT = 24;
+
 template <int G, int WPB, int WMAX, int K, bool BYTES, bool LROWS>
 static hipError_t launch_one(const CliqueArgs& a, int grid, hipStream_t st) {
   hipLaunchKernelGGL((clique_kernel<G, WPB, WMAX, K, BYTES, LROWS>), dim3(grid), dim3(64 * G * WPB), 0, st, a);
@@ -290,7 +422,12 @@ static hipError_t launch_one(const CliqueArgs& a, int grid, hipStream_t st) {
 template <int K, bool BYTES>
 static hipError_t launch_k(int tier, const CliqueArgs& a, int grid, hipStream_t st) {
   switch (tier) {
-    case TIER_WAVE:   return launch_one<1, 4, 1, K, BYTES, true>(a, grid, st);
+    case TIER_WAVE:
+      // 6- and 7-cliques of the wider one-word roots: four waves share a root
+      // (their subtrees would leave one wave running alone at the end)
+      if constexpr (!BYTES && K >= 6)
+        if (a.dmin > SMALL_ROOT) return launch_one<4, 1, 1, K, BYTES, true>(a, grid, st);
+      return launch_one<1, 4, 1, K, BYTES, true>(a, grid, st);
     case TIER_LDS2:   return launch_one<4, 1, 2, K, BYTES, true>(a, grid, st);
     case TIER_LDS4:   return launch_one<4, 1, 4, K, BYTES, true>(a, grid, st);
     case TIER_LDS8:   return launch_one<8, 1, 8, K, BYTES, true>(a, grid, st);
@@ -310,6 +447,8 @@ hipError_t launch_clique(int k, bool bytes, int tier, const CliqueArgs& a, int g
   }
   return hipErrorInvalidValue;
 }
+
+int clique_small_root() { return SMALL_ROOT; }
 
 int tier_max_deg(int tier) {
   switch (tier) {

@@ -548,6 +548,26 @@ int enqueue_clique(jgpm_graph_s* g, int k, bool bytes, int64_t rb, int64_t re, i
       a.ntasks = n;
       a.chunk = 1;
       grid = (int)std::min<int64_t>(maxgrid, n);
+      if (tier <= jk::TIER_LDS8 && !bytes && k >= 6 && !gscr && !c->capturing) {
+        // split form: rows into global slots, then a wave per (root, row);
+        // chunks of roots bound the slots to 1 GiB
+        const size_t slot = jk::rows_slot_words(tier);
+        const int64_t cap = std::min<int64_t>(n, std::max<int64_t>(1, ((int64_t)1 << 27) / (int64_t)slot));
+        int s2 = ensure_scratch(c, slot * (size_t)cap);
+        if (s2) return s2;
+        for (int64_t b = 0; b < n; b += cap) {
+          jk::CliqueArgs s = a;
+          s.ids = a.ids + b;
+          s.ntasks = std::min<int64_t>(cap, n - b);
+          s.gscr = c->d_scr;
+          prof_begin(c, st, kTierName[tier]);
+          hipError_t e = jk::launch_clique_rows(k, tier, true, s, c->num_cu, maxgrid, st);
+          if (e == hipSuccess) e = jk::launch_clique_rows(k, tier, false, s, c->num_cu, maxgrid, st);
+          prof_end(c, st);
+          if (e != hipSuccess) return JGPM_E_HIP;
+        }
+        continue;
+      }
       if (tier == jk::TIER_LDS16 && !bytes && k >= 4 && !gscr && !c->capturing) {
         // split form: build with 16 waves per root into global row slots,
         // then count; chunks of roots bound the slots to 1 GiB
@@ -625,7 +645,16 @@ int enqueue_clique(jgpm_graph_s* g, int k, bool bytes, int64_t rb, int64_t re, i
       }
     }
     prof_begin(c, st, kTierName[tier]);
-    hipError_t e = jk::launch_clique(k, bytes, tier, a, grid, st);
+    hipError_t e = hipSuccess;
+    if (tier == jk::TIER_WAVE && k >= 6 && !bytes) {
+      jk::CliqueArgs w = a;
+      w.dmin = std::max(a.dmin, jk::clique_small_root() + 1);
+      e = jk::launch_clique(k, bytes, tier, w, (int)std::min<int64_t>(maxgrid, a.ntasks), st);
+      a.dmax = jk::clique_small_root();
+      // the second launch's queue starts at zero again
+      hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, a.qctr, 1, 0u);
+    }
+    if (e == hipSuccess) e = jk::launch_clique(k, bytes, tier, a, grid, st);
     prof_end(c, st);
     if (e != hipSuccess) return JGPM_E_HIP;
   }

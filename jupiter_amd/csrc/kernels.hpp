@@ -54,6 +54,12 @@ hipError_t launch_clique(int k, bool bytes, int tier, const CliqueArgs& a, int g
 // a.gscr slots of split_slot_words() words per task), then count kernel.
 hipError_t launch_clique_split(int k, bool build, const CliqueArgs& a, int grid, hipStream_t st);
 size_t split_slot_words();
+// Split form of TIER_LDS2 .. TIER_LDS8 for k >= 6: build kernel (rows to a.gscr
+// slots of rows_slot_words(tier) words per task), then a count kernel with a
+// wave per (task, row).
+hipError_t launch_clique_rows(int k, int tier, bool build, const CliqueArgs& a, int num_cu, int maxgrid,
+                              hipStream_t st);
+size_t rows_slot_words(int tier);
 // Split form of TIER_GLB32 for k >= 5: build kernel (16 waves per root, rows
 // to a.gscr slots of glb_slot_words() words per task), then count kernel
 // (a.rep blocks per task share the root's rows through a.rowctr[task]).
@@ -226,6 +232,9 @@ hipError_t launch_vertex_sums(const int64_t* rp, const int32_t* tri, int64_t rb,
 hipError_t launch_p2_edges(const int32_t* src, const int32_t* ci, const int32_t* tri, int64_t e0, int64_t e1,
                            unsigned long long* out, int grid, hipStream_t st);
 int tier_max_deg(int tier);
+// TIER_WAVE of 6- and 7-cliques runs as two launches: roots up to this
+// out-degree with a wave each, wider ones (a.dmin above it) with a block each
+int clique_small_root();
 size_t tier_scratch_words(int tier);
 
 // Roots wider than the widest row tier (DAG out-degree > 2048): the level
