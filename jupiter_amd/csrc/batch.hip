@@ -447,7 +447,7 @@ extern "C" int jgpm_count_batch(jgpm_ctx_t ctx, const jgpm_query* q, int n, uint
     std::lock_guard<std::mutex> lk(ctx->mu);
     if (hipSetDevice(ctx->dev) != hipSuccess) return JGPM_E_HIP;
     if (hipEventRecord(ctx->e0, ctx->st) != hipSuccess) return JGPM_E_HIP;
-    ctx->nprof = 0;
+    prof_reset(ctx, nullptr);
     std::vector<jk::BQ> hq;
     std::vector<int64_t> cs;
     if (!qs.empty()) {
@@ -588,7 +588,7 @@ extern "C" int jgpm_batch_run(jgpm_batch_t B, uint64_t* counts, double* kernel_m
   const int n = (int)B->q.size();
   std::lock_guard<std::mutex> lk(ctx->mu);
   if (hipSetDevice(ctx->dev) != hipSuccess) return JGPM_E_HIP;
-  ctx->nprof = 0;
+  jgpm::prof_reset(ctx, nullptr);
   if (hipEventRecord(ctx->e0, ctx->st) != hipSuccess || hipGraphLaunch(B->exec, ctx->st) != hipSuccess ||
       hipEventRecord(ctx->e1, ctx->st) != hipSuccess ||
       hipMemcpyAsync(B->h.data(), B->b.bcnt, sizeof(uint64_t) * n, hipMemcpyDeviceToHost, ctx->st) != hipSuccess ||

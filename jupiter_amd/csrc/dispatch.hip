@@ -24,6 +24,7 @@ ExecScope::~ExecScope() { t_exec = prev; }
 // while capturing); its contents are lost.
 static int grow(jgpm_ctx_s* c, void*& p, size_t& have, size_t need, hipStream_t st) {
   if (have >= need) return JGPM_OK;
+  prof_stale(c);
   if (c->capturing) return JGPM_E_STATE;
   if (p) {
     if (hipStreamSynchronize(st) != hipSuccess) return JGPM_E_HIP;
@@ -80,6 +81,7 @@ static int tri_args(jgpm_graph_s* g, hipStream_t st, jk::TriArgs& a) {
 int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t st) {
   jgpm_ctx_s* c = exec_ctx(g);
   const int64_t ne = g->sym.nnz;
+  if (!g->d_src || (need_tri && !g->d_tri) || (need_nsum && !g->d_nsum)) prof_stale(c);
   if (!g->d_src) {
     if (hipMalloc(&g->d_src, sizeof(int32_t) * std::max<int64_t>(ne, 1)) != hipSuccess) return JGPM_E_NOMEM;
     g->bytes += 4 * ne;
@@ -500,6 +502,7 @@ int enqueue_vertex_sum(jgpm_graph_s* g, int mode, int64_t rb, int64_t re, int sl
   if (rc) return rc;
   if (re <= rb) return JGPM_OK;
   jgpm_ctx_s* c = exec_ctx(g);
+  prof_stale(c);
   return jk::launch_vertex_sums(g->sym.rp, g->d_tri, rb, re, mode, (unsigned long long*)(c->d_out + slot),
                                 grid_for(c, 4), st) == hipSuccess
              ? JGPM_OK
@@ -557,7 +560,7 @@ int prepare_pattern(jgpm_graph_s* g, int pattern, int64_t rb, int64_t re) {
   std::lock_guard<std::mutex> lk(c->mu);
   if (hipSetDevice(c->dev) != hipSuccess) return JGPM_E_HIP;
   ExecScope own(c);
-  c->nprof = 0;
+  prof_reset(c, nullptr);
   int rc = JGPM_OK;
   if (clique_k(pattern)) {
     if (g->has_dag) rc = ensure_huge_ids(g);

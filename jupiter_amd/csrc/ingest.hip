@@ -423,6 +423,7 @@ int ensure_rank_csr(jgpm_graph_s* g, hipStream_t st) {
   if (g->rsym.ci || !g->has_sym) return JGPM_OK;
   jgpm_ctx_s* c = exec_ctx(g);
   if (c->capturing) return JGPM_E_STATE;
+  prof_stale(c);
   int rc = ensure_sym_aux(g, false, false, st);  // COO sources
   if (rc) return rc;
   const int32_t nv = (int32_t)g->sym.nv;

@@ -53,6 +53,11 @@ __global__ void k_fill_u64(uint64_t* p, int n, uint64_t v) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
+__global__ void k_reset_counters(uint64_t* out, uint32_t* q, unsigned long long* q64) {
+  out[threadIdx.x] = 0;
+  q[threadIdx.x] = 0;
+  q64[threadIdx.x] = 0;
+}
 __global__ void k_fill_u32(uint32_t* p, int n, uint32_t v) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -66,25 +71,37 @@ int zero_u64(uint64_t* p, int n, hipStream_t st) {
 }
 
 int ctx_reset_counters(jgpm_ctx_s* c, hipStream_t st) {
-  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(CTX_SLOTS), 0, st, c->d_out, CTX_SLOTS, 0ull);
-  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(CTX_SLOTS), 0, st, c->d_q, CTX_SLOTS, 0u);
-  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(CTX_SLOTS), 0, st, (uint64_t*)c->d_q64, CTX_SLOTS, 0ull);
+  hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(CTX_SLOTS), 0, st, c->d_out, c->d_q, c->d_q64);
   return hipGetLastError() == hipSuccess ? JGPM_OK : JGPM_E_HIP;
 }
 
+// An event costs a call and a gap on the stream, so a span that starts where
+// the one before it (or the query) was marked takes that mark as its begin.
+void prof_reset(jgpm_ctx_s* c, hipEvent_t open) {
+  c->nprof = 0;
+  c->popen = open;
+}
+void prof_stale(jgpm_ctx_s* c) { c->popen = nullptr; }
 void prof_begin(jgpm_ctx_s* c, hipStream_t st, const char* name) {
   if (!c->prof_on || st != c->st || c->nprof >= jgpm_ctx_s::MAX_PROF) return;
-  c->pname[c->nprof] = name;
-  (void)hipEventRecord(c->pev[2 * c->nprof], st);
+  const int n = c->nprof;
+  c->pname[n] = name;
+  c->pbeg[n] = c->popen ? c->popen : c->pev[2 * n];
+  if (!c->popen) (void)hipEventRecord(c->pev[2 * n], st);
 }
 void prof_end(jgpm_ctx_s* c, hipStream_t st) {
-  if (!c->prof_on || st != c->st || c->nprof >= jgpm_ctx_s::MAX_PROF) return;
-  (void)hipEventRecord(c->pev[2 * c->nprof + 1], st);
+  if (!c->prof_on || st != c->st || c->nprof >= jgpm_ctx_s::MAX_PROF) {
+    prof_stale(c);
+    return;
+  }
+  c->popen = c->pev[2 * c->nprof + 1];
+  (void)hipEventRecord(c->popen, st);
   c->nprof++;
 }
 
 int ensure_scratch(jgpm_ctx_s* c, size_t words) {
   if (c->scr_words >= words) return JGPM_OK;
+  prof_stale(c);
   if (c->d_scr) {
     HIP_TRY(hipStreamSynchronize(c->st));
     HIP_TRY(hipFree(c->d_scr));
@@ -276,7 +293,8 @@ extern "C" int jgpm_init(int dev, jgpm_ctx_t* out) {
     }
   if (hipMalloc(&c->d_out, CTX_SLOTS * sizeof(uint64_t)) != hipSuccess ||
       hipMalloc(&c->d_q, CTX_SLOTS * sizeof(uint32_t)) != hipSuccess ||
-      hipMalloc(&c->d_q64, CTX_SLOTS * sizeof(unsigned long long)) != hipSuccess) {
+      hipMalloc(&c->d_q64, CTX_SLOTS * sizeof(unsigned long long)) != hipSuccess ||
+      hipHostMalloc(&c->h_out, CTX_SLOTS * sizeof(uint64_t), hipHostMallocDefault) != hipSuccess) {
     delete c;
     return JGPM_E_NOMEM;
   }
@@ -299,6 +317,7 @@ extern "C" int jgpm_shutdown(jgpm_ctx_t c) {
   if (c->d_out) (void)hipFree(c->d_out);
   if (c->d_q) (void)hipFree(c->d_q);
   if (c->d_q64) (void)hipFree(c->d_q64);
+  if (c->h_out) (void)hipHostFree(c->h_out);
   if (c->d_sscr) (void)hipFree(c->d_sscr);
   if (c->d_hlist) (void)hipFree(c->d_hlist);
   if (c->d_hctr) (void)hipFree(c->d_hctr);
@@ -683,23 +702,29 @@ extern "C" int jgpm_count(jgpm_graph_t g, int pattern, int64_t root_begin, int64
   jgpm_ctx_s* c = g->ctx;
   std::lock_guard<std::mutex> lk(c->mu);
   HIP_TRY(hipSetDevice(c->dev));
-  HIP_TRY(hipEventRecord(c->e0, c->st));
   st = ctx_reset_counters(c, c->st);
   if (st) return st;
-  c->nprof = 0;
+  HIP_TRY(hipEventRecord(c->e0, c->st));
+  prof_reset(c, c->e0);
   st = enqueue_pattern(g, pattern, root_begin, root_end, 0, c->st);
   if (st) {
     (void)hipStreamSynchronize(c->st);
     return st;
   }
-  HIP_TRY(hipEventRecord(c->e1, c->st));
-  uint64_t h[CTX_SLOTS];
-  HIP_TRY(hipMemcpyAsync(h, c->d_out, sizeof(h), hipMemcpyDeviceToHost, c->st));
+  // the last span's end is the query's, unless something ran after it
+  hipEvent_t end = c->popen;
+  if (!end) {
+    end = c->e1;
+    HIP_TRY(hipEventRecord(end, c->st));
+  }
+  // the accumulators the pattern uses, to pinned memory
+  HIP_TRY(hipMemcpyAsync(c->h_out, c->d_out, sizeof(uint64_t) * (size_t)pattern_slots(pattern), hipMemcpyDeviceToHost,
+                         c->st));
   HIP_TRY(hipStreamSynchronize(c->st));
-  *count = finish_pattern(pattern, h);
+  *count = finish_pattern(pattern, c->h_out);
   if (kernel_ms) {
     float ms = 0;
-    HIP_TRY(hipEventElapsedTime(&ms, c->e0, c->e1));
+    if (end != c->e0) HIP_TRY(hipEventElapsedTime(&ms, c->e0, end));
     *kernel_ms = ms;
   }
   return JGPM_OK;
@@ -733,7 +758,7 @@ extern "C" int jgpm_last_profile(jgpm_ctx_t c, int n, const char** names, double
   std::lock_guard<std::mutex> lk(c->mu);
   for (int i = 0; i < c->nprof && i < n; ++i) {
     float t = 0;
-    if (hipEventElapsedTime(&t, c->pev[2 * i], c->pev[2 * i + 1]) != hipSuccess) return JGPM_E_HIP;
+    if (hipEventElapsedTime(&t, c->pbeg[i], c->pev[2 * i + 1]) != hipSuccess) return JGPM_E_HIP;
     if (names) names[i] = c->pname[i];
     if (ms) ms[i] = t;
   }
@@ -752,7 +777,7 @@ extern "C" int jgpm_work_bytes_split(jgpm_graph_t g, int pattern, int64_t root_b
   HIP_TRY(hipSetDevice(c->dev));
   st = ctx_reset_counters(c, c->st);
   if (st) return st;
-  c->nprof = 0;
+  prof_reset(c, nullptr);
   st = enqueue_clique(g, k, true, root_begin, root_end, 0, c->st, true);
   if (st) {
     (void)hipStreamSynchronize(c->st);

@@ -33,6 +33,7 @@ struct jgpm_ctx_s {
   char name[128] = {0};
   jgpm_tuning tune{};
   uint64_t* d_out = nullptr;  // CTX_SLOTS accumulators
+  uint64_t* h_out = nullptr;  // pinned: where a query's accumulators are read back
   uint32_t* d_q = nullptr;    // CTX_SLOTS work-queue counters
   unsigned long long* d_q64 = nullptr;  // CTX_SLOTS 64-bit work-queue counters
   int32_t* d_sscr = nullptr;  // list scratch of the symmetric-pattern kernels
@@ -61,6 +62,8 @@ struct jgpm_ctx_s {
   // per-launch profile of the current query (events around every kernel)
   static constexpr int MAX_PROF = 16;
   hipEvent_t pev[2 * MAX_PROF] = {nullptr};
+  hipEvent_t pbeg[MAX_PROF] = {nullptr};  // begin of each span: pev, or an event already there
+  hipEvent_t popen = nullptr;  // marks the stream's end as of now (null: something was enqueued since)
   const char* pname[MAX_PROF] = {nullptr};
   int nprof = 0;
   bool prof_on = true;
@@ -160,6 +163,10 @@ bool pattern_uses_tri(int p);
 // whether a single-query launch of pattern p on context c reads the triangle array
 bool query_needs_tri(const jgpm_ctx_s* c, int p);
 // profile hooks around one kernel launch on the context stream
+// prof_reset: a new query, whose begin is marked by `open` (may be null);
+// prof_stale: work outside the spans was enqueued, or the host waited.
+void prof_reset(jgpm_ctx_s* c, hipEvent_t open);
+void prof_stale(jgpm_ctx_s* c);
 void prof_begin(jgpm_ctx_s* c, hipStream_t st, const char* name);
 void prof_end(jgpm_ctx_s* c, hipStream_t st);
 int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int out_slot, hipStream_t st);

@@ -228,7 +228,7 @@ extern "C" int jgpm_count_plan(jgpm_graph_t g, jgpm_plan_t p, int64_t rb, int64_
   a.stride = stride;
   a.out = c->d_out;
   a.plan = *P;
-  c->nprof = 0;
+  jgpm::prof_reset(c, nullptr);
   uint64_t h = 0;
   if (hipEventRecord(c->e0, c->st) != hipSuccess) return JGPM_E_HIP;
   if (re > rb && jk::launch_plan(a, grid, c->st) != hipSuccess) return JGPM_E_HIP;

@@ -150,14 +150,15 @@ static int run_heavy(jgpm_ctx_s* main, jgpm_ctx_s* lc, const Req& r, uint64_t* c
     std::lock_guard<std::mutex> gl(main->mu);
     if (!st) st = jgpm::ctx_reset_counters(lc, lc->st);
     if (!st) {
-      lc->nprof = 0;
+      jgpm::prof_reset(lc, nullptr);
       st = jgpm::enqueue_pattern(r.g, r.pattern, r.rb, r.re, 0, lc->st);
     }
   }
-  uint64_t hc[CTX_SLOTS];
-  if (!st && hipMemcpyAsync(hc, lc->d_out, sizeof(hc), hipMemcpyDeviceToHost, lc->st) != hipSuccess) st = JGPM_E_HIP;
+  if (!st && hipMemcpyAsync(lc->h_out, lc->d_out, sizeof(uint64_t) * (size_t)jgpm::pattern_slots(r.pattern),
+                            hipMemcpyDeviceToHost, lc->st) != hipSuccess)
+    st = JGPM_E_HIP;
   if (hipStreamSynchronize(lc->st) != hipSuccess && !st) st = JGPM_E_HIP;
-  if (!st) *count = jgpm::finish_pattern(r.pattern, hc);
+  if (!st) *count = jgpm::finish_pattern(r.pattern, lc->h_out);
   return st;
 }
 
@@ -276,7 +277,7 @@ static void serve_loop(jgpm_serve_s* s) {
         st = (hipSetDevice(c->dev) == hipSuccess) ? JGPM_OK : JGPM_E_HIP;
         if (!st) st = jgpm::ctx_reset_counters(c, c->st);
         if (!st) {
-          c->nprof = 0;
+          jgpm::prof_reset(c, nullptr);
           st = jgpm::enqueue_batch_q(c, qs.data(), (int)qs.size(), c->st);
         }
         h.assign(qs.size(), 0);
@@ -344,6 +345,7 @@ extern "C" int jgpm_serve_start(jgpm_ctx_t ctx, const jgpm_serve_config* cfg, jg
       return st;
     }
     L->ctx->tune = ctx->tune;
+    L->ctx->prof_on = false;  // nobody can ask a lane's context for its profile
     s->lanes.push_back(L);
     L->th = std::thread(lane_loop, s, L);
   }
