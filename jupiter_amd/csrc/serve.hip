@@ -15,8 +15,9 @@
 //    meanwhile are admitted before the next launch, so their work overlaps
 //    with the tails of earlier ones on the device;
 //  * heavy requests: a request whose work (edges of its range times the
-//    pattern weight) exceeds one slice would fill the device by itself, so
-//    it is not sliced: it runs whole with the single-query kernels (its count
+//    pattern weight) exceeds one slice would fill the device by itself (and
+//    P3 .. P12 are counted faster by their single-query kernels), so it is not
+//    sliced: it runs whole with the single-query kernels (its count
 //    is then exactly jgpm_count's, from the same kernels, including the
 //    degree-order relabelling a whole-graph 4-cycle count uses).  Heavy
 //    requests run on lanes: each lane is a thread with a context of its own
@@ -94,6 +95,19 @@ double pattern_weight(int p) {
   return 8;
 }
 
+bool is_dag_pattern(int p) { return jgpm::clique_k(p) != 0 && p != JGPM_I_K4; }
+
+// Edges of the range above which a request runs whole on a lane.  P3 .. P12:
+// their single-query kernels count over triangles and wedges, where the
+// batched launch takes an edge at a time (8 R-MAT graphs of scales 12 to 16,
+// all served: P5 114 ms in batches and 2.4 on lanes).  Cliques: the batched launch
+// keeps a root in one wave up to the hub degree, so a mid-sized graph ends
+// with few waves at work (the same graphs: P14 8.8 ms in batches and 2.5 on lanes, P13 3.5 and 1.5).
+int64_t single_edges(int p) {
+  if (p >= JGPM_P3 && p <= JGPM_P12) return 4096;
+  return is_dag_pattern(p) ? 32768 : INT64_MAX;
+}
+
 }  // namespace
 
 struct jgpm_serve_s {
@@ -116,8 +130,6 @@ struct jgpm_serve_s {
   std::vector<HeavyDone> heavy_done;  // finished on a lane, not yet merged by the scheduler
   bool lanes_stop = false;
 };
-
-static bool is_dag_pattern(int p) { return jgpm::clique_k(p) != 0 && p != JGPM_I_K4; }
 
 // HBM the request's intermediates need beyond the resident graph.
 static int64_t footprint(jgpm_graph_s* g, int p, const jgpm_ctx_s* c, int grid) {
@@ -382,7 +394,8 @@ extern "C" int jgpm_serve_submit(jgpm_serve_t s, jgpm_graph_t g, int pattern, in
   r.footprint = footprint(g, pattern, s->ctx, grid);
   {
     const std::vector<int64_t>& rp = is_dag_pattern(pattern) ? g->dag_rp_h : g->sym_rp_h;
-    r.heavy = wide || (double)(rp[re] - rp[rb]) * pattern_weight(pattern) > (double)s->slice_edges;
+    r.heavy = wide || (double)(rp[re] - rp[rb]) * pattern_weight(pattern) > (double)s->slice_edges ||
+              rp[re] - rp[rb] > single_edges(pattern);
   }
   r.t_submit = clk::now();
   std::lock_guard<std::mutex> lk(s->mu);
