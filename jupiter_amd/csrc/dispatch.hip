@@ -21,9 +21,11 @@ ExecScope::ExecScope(jgpm_ctx_s* c) : prev(t_exec) { t_exec = c; }
 ExecScope::~ExecScope() { t_exec = prev; }
 
 // Grows one of the context's scratch buffers to `need` bytes (allocates, never
-// while capturing); its contents are lost.
-static int grow(jgpm_ctx_s* c, void*& p, size_t& have, size_t need, hipStream_t st) {
+// while capturing); its contents are lost.  More than `cap` bytes are
+// JGPM_E_NOMEM, as where the device has no room.
+static int grow(jgpm_ctx_s* c, void*& p, size_t& have, size_t need, size_t cap, hipStream_t st) {
   if (have >= need) return JGPM_OK;
+  if (need > cap) return JGPM_E_NOMEM;
   prof_stale(c);
   if (c->capturing) return JGPM_E_STATE;
   if (p) {
@@ -64,11 +66,16 @@ static int tri_args(jgpm_graph_s* g, hipStream_t st, jk::TriArgs& a) {
   a.hwords = (((int64_t)nv + 31) / 32 + 3) & ~(int64_t)3;
   a.nhub = (int32_t)std::min<int64_t>(g->hubs, TRI_HUB_BYTES / (4 * a.hwords));
   a.lstride = std::max(1, g->dag.max_deg);
-  const size_t hub_b = 4 * (size_t)a.hwords * (size_t)a.nhub;
+  size_t hub_b = 4 * (size_t)a.hwords * (size_t)a.nhub;
   const size_t list_b = (sizeof(int32_t) * 3 * (size_t)nv + 15) & ~(size_t)15;
   const size_t lscr_b = a.wide ? sizeof(int32_t) * 3 * (size_t)a.lstride * (size_t)(jk::TRI_SMALL_PER_CU * c->num_cu) : 0;
-  const size_t need = 64 + hub_b + list_b + lscr_b;
-  if (int rc = grow(c, c->d_te, c->te_bytes, need, st)) return rc;
+  int rc = grow(c, c->d_te, c->te_bytes, 64 + hub_b + list_b + lscr_b, c->ws_cap, st);
+  if (rc == JGPM_E_NOMEM) {  // without bitmaps: every row searched for
+    a.nhub = 0;
+    hub_b = 0;
+    rc = grow(c, c->d_te, c->te_bytes, 64 + list_b + lscr_b, SIZE_MAX, st);
+  }
+  if (rc) return rc;
   unsigned char* b = static_cast<unsigned char*>(c->d_te);
   a.ctr = reinterpret_cast<unsigned long long*>(b);
   a.hub = reinterpret_cast<const uint32_t*>(b + 64);
@@ -213,11 +220,12 @@ static int enqueue_ego(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot,
   uint64_t* const out = c->d_out + slot;
   const int64_t *rp = g->sym_rp_h.data(), *pre = g->tri_pre_h.data();
   // chunks of whole roots, and the scratch of the largest
+  const int64_t cap = std::min<int64_t>(EGO_CAP, (int64_t)(c->ws_cap / 32));
   std::vector<int64_t> cut{rb};
   int64_t most_e = 0, most_n = 0;
   for (int64_t r = rb; r < re;) {
-    int64_t r2 = std::upper_bound(pre + r + 1, pre + re + 1, pre[r] + EGO_CAP) - pre - 1;
-    r2 = std::min(r2, (int64_t)(std::upper_bound(rp + r + 1, rp + re + 1, rp[r] + EGO_CAP) - rp - 1));
+    int64_t r2 = std::upper_bound(pre + r + 1, pre + re + 1, pre[r] + cap) - pre - 1;
+    r2 = std::min(r2, (int64_t)(std::upper_bound(rp + r + 1, rp + re + 1, rp[r] + cap) - rp - 1));
     r2 = std::max(r2, r + 1);
     most_e = std::max(most_e, pre[r2] - pre[r]);
     most_n = std::max(most_n, rp[r2] - rp[r]);
@@ -225,7 +233,7 @@ static int enqueue_ego(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot,
   }
   const size_t rp_b = sizeof(int64_t) * (size_t)(most_n + 1), tiles_b = sizeof(int64_t) * (size_t)jk::ego_tiles(most_n);
   const size_t ent_b = sizeof(int32_t) * (size_t)most_e;
-  int rc = grow(c, c->d_ego, c->ego_bytes, rp_b + tiles_b + 2 * ent_b + 64, st);
+  int rc = grow(c, c->d_ego, c->ego_bytes, rp_b + tiles_b + 2 * ent_b + 64, c->ws_cap, st);
   if (!rc) rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(most_n, most_e), st);
   jk::TriArgs ta;
   if (!rc) rc = tri_args(g, st, ta);
@@ -331,7 +339,9 @@ static bool heavy_split_on(const jgpm_ctx_s* c, int p) {
 
 bool query_needs_tri(const jgpm_ctx_s* c, int p) { return p == 2 || pattern_uses_tri(p) || heavy_split_on(c, p); }
 
-int ensure_p1_scratch(jgpm_ctx_s* c, size_t bytes, hipStream_t st) { return grow(c, c->d_p1, c->p1_bytes, bytes, st); }
+int ensure_p1_scratch(jgpm_ctx_s* c, size_t bytes, hipStream_t st) {
+  return grow(c, c->d_p1, c->p1_bytes, bytes, SIZE_MAX, st);
+}
 
 int p1_query(jgpm_graph_s* g, int64_t rb, int64_t re, hipStream_t st, jk::P1Q& q) {
   q = jk::P1Q{};
@@ -394,6 +404,15 @@ int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStr
     prof_end(c, st);
     return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
   }
+  if (p == 3) {
+    int rc = ensure_sym_aux(g, true, true, st);
+    if (rc) return rc;
+    prof_begin(c, st, "sym_p3");
+    hipError_t e = jk::launch_edge_sum(true, g->sym.rp, g->sym.ci, g->d_src, g->d_tri, g->d_nsum, g->sym_rp_h[rb],
+                                       g->sym_rp_h[re], c->d_q64 + slot, c->d_out + slot, c->num_cu, st);
+    prof_end(c, st);
+    return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
+  }
   // patterns that run over triangles or wedges of the whole range; where
   // there is no room for their scratch (nothing launched), per edge
   const int64_t ne_q = g->sym_rp_h[re] - g->sym_rp_h[rb];
@@ -410,7 +429,7 @@ int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStr
     if (rr != JGPM_E_NOMEM) return rr;
     (void)hipGetLastError();
   }
-  int rc = ensure_sym_aux(g, query_needs_tri(c, p), p == 3, st);
+  int rc = ensure_sym_aux(g, query_needs_tri(c, p), false, st);
   if (rc) return rc;
   // the heavy-edge split needs its three edge lists, each as long as the
   // range's edge count up to 2^26 (grown per context, so not while a launch
@@ -458,7 +477,7 @@ int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStr
   a.ne = g->sym_rp_h[re] - a.e0;
   if (a.ne <= 0) return JGPM_OK;
   a.qctr = c->d_q64 + (slot % (CTX_SLOTS - 1));
-  a.chunk = (p == 2 || p == 3) ? 64 : 8;
+  a.chunk = 8;
   a.scr = c->d_sscr;
   a.scr_stride = (int64_t)stride;
   a.out = c->d_out + slot;
@@ -471,12 +490,10 @@ int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStr
   a.heavy_mid = heavy ? jk::sym_heavy_mid(p) : 0;
   // list counters to zero (a kernel, so the sequence can be captured)
   if (heavy && zero_u64(reinterpret_cast<uint64_t*>(c->d_hctr), 6, st)) return JGPM_E_HIP;
-  static const char* const kSymName[13] = {"", "sym_p1", "sym_p2", "sym_p3", "sym_p4", "sym_p5", "sym_p6",
+  static const char* const kSymName[13] = {"", "", "", "", "sym_p4", "sym_p5", "sym_p6",
                                            "sym_p7", "sym_p8", "sym_p9", "sym_p10", "sym_p11", "sym_p12"};
   prof_begin(c, st, kSymName[p]);
-  // a whole-graph P3 counts each triangle once instead of per directed edge
-  hipError_t e = (p == 3 && rb == 0 && re == g->sym.nv) ? jk::launch_p3_triangles(a, grid, st)
-                                                        : jk::launch_sym(p, a, grid, st);
+  hipError_t e = jk::launch_sym(p, a, grid, st);
   prof_end(c, st);
   if (e != hipSuccess) return JGPM_E_HIP;
   if (heavy) {
@@ -503,10 +520,11 @@ int enqueue_vertex_sum(jgpm_graph_s* g, int mode, int64_t rb, int64_t re, int sl
   if (re <= rb) return JGPM_OK;
   jgpm_ctx_s* c = exec_ctx(g);
   prof_stale(c);
-  return jk::launch_vertex_sums(g->sym.rp, g->d_tri, rb, re, mode, (unsigned long long*)(c->d_out + slot),
-                                grid_for(c, 4), st) == hipSuccess
-             ? JGPM_OK
-             : JGPM_E_HIP;
+  const hipError_t e =
+      mode == 0 ? jk::launch_star3(g->sym.rp, rb, re, (unsigned long long*)(c->d_out + slot), grid_for(c, 4), st)
+                : jk::launch_edge_sum(false, g->sym.rp, g->sym.ci, g->d_src, g->d_tri, nullptr, g->sym_rp_h[rb],
+                                      g->sym_rp_h[re], c->d_q64 + slot, c->d_out + slot, c->num_cu, st);
+  return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
 }
 
 // Induced 4-vertex motifs from non-induced counts (exact inverse of the

@@ -569,12 +569,14 @@ int enqueue_clique(jgpm_graph_s* g, int k, bool bytes, int64_t rb, int64_t re, i
       grid = (int)std::min<int64_t>(maxgrid, n);
       if (tier <= jk::TIER_LDS8 && !bytes && k >= 6 && !gscr && !c->capturing) {
         // split form: rows into global slots, then a wave per (root, row);
-        // chunks of roots bound the slots to 1 GiB
+        // chunks of roots bound the slots to 1 GiB.  Without room for them
+        // the roots run fused, like 4- and 5-cliques.
         const size_t slot = jk::rows_slot_words(tier);
-        const int64_t cap = std::min<int64_t>(n, std::max<int64_t>(1, ((int64_t)1 << 27) / (int64_t)slot));
+        const size_t words = std::min<size_t>((size_t)1 << 27, c->ws_cap / sizeof(uint64_t));
+        const int64_t cap = std::min<int64_t>(n, std::max<int64_t>(1, (int64_t)(words / slot)));
         int s2 = ensure_scratch(c, slot * (size_t)cap);
-        if (s2) return s2;
-        for (int64_t b = 0; b < n; b += cap) {
+        if (s2 && s2 != JGPM_E_NOMEM) return s2;
+        for (int64_t b = 0; !s2 && b < n; b += cap) {
           jk::CliqueArgs s = a;
           s.ids = a.ids + b;
           s.ntasks = std::min<int64_t>(cap, n - b);
@@ -585,7 +587,8 @@ int enqueue_clique(jgpm_graph_s* g, int k, bool bytes, int64_t rb, int64_t re, i
           prof_end(c, st);
           if (e != hipSuccess) return JGPM_E_HIP;
         }
-        continue;
+        if (!s2) continue;
+        (void)hipGetLastError();
       }
       if (tier == jk::TIER_LDS16 && !bytes && k >= 4 && !gscr && !c->capturing) {
         // split form: build with 16 waves per root into global row slots,

@@ -41,6 +41,7 @@ struct jgpm_ctx_s {
   int32_t* d_hlist = nullptr;  // heavy-edge lists of P5/P7/P9/P11/P12 (3 x hcap ints)
   int64_t hcap = 0;
   unsigned long long* d_hctr = nullptr;  // their append and pop counters (6)
+  size_t ws_cap = SIZE_MAX;    // bytes any one of the workspaces may take that a query can also do without
   void* d_ego = nullptr;       // the graph of induced neighbourhoods of P6, P8, P10
   size_t ego_bytes = 0;
   void* d_te = nullptr;        // scratch of the triangle launches (lists, hub bitmaps)

@@ -95,9 +95,6 @@ struct SymArgs {
   int32_t heavy_mid;
 };
 hipError_t launch_sym(int p, const SymArgs& a, int grid, hipStream_t st);
-// Whole-graph P3 from one intersection per undirected edge (each triangle
-// once, its three oriented terms); needs tri and nsum, e0 = 0, ne = all edges.
-hipError_t launch_p3_triangles(const SymArgs& a, int grid, hipStream_t st);
 // The heavy edges of P5, P7, P9, P11 and P12, one block per edge, popped
 // from list `shape` (0, 1, 2 as above) that launch_sym filled; shape 2 keeps
 // S in the block's slice of a.scr (a.scr_stride ints, grid slices).
@@ -219,15 +216,19 @@ hipError_t launch_p10_rows(const EgoArgs& g, uint64_t* out, int num_cu, hipStrea
 // closed per-edge parts: P4 (mode 0: root range, 1: whole graph), P6 (mode 2)
 hipError_t launch_edge_base(const int64_t* rp, const int32_t* ci, const int32_t* src, const int32_t* tri, int64_t e0,
                             int64_t e1, int mode, uint64_t* out, int num_cu, hipStream_t st);
+// P3 (p3; needs nsum) or tailed triangles over the edges [e0, e1) of a root
+// range; *flag zero before
+hipError_t launch_edge_sum(bool p3, const int64_t* rp, const int32_t* ci, const int32_t* src, const int32_t* tri,
+                           const int64_t* nsum, int64_t e0, int64_t e1, unsigned long long* flag, uint64_t* out,
+                           int num_cu, hipStream_t st);
 hipError_t launch_root_tri(const int64_t* rp, const int32_t* tri, int32_t nv, int64_t* sum, int num_cu, hipStream_t st);
 
 int sym_waves_per_block();
 int sym_lists_per_wave();
 hipError_t launch_aux_src(const int64_t* rp, int32_t nv, int32_t* src, int grid, hipStream_t st);
 hipError_t launch_aux_nsum(const int64_t* rp, const int32_t* ci, int32_t nv, int64_t* nsum, int grid, hipStream_t st);
-// mode 0: sum C(d,3) (3-stars); mode 1: sum t_v (d_v - 2) (tailed triangles)
-hipError_t launch_vertex_sums(const int64_t* rp, const int32_t* tri, int64_t rb, int64_t re, int mode,
-                              unsigned long long* out, int grid, hipStream_t st);
+// 3-stars: sum of C(d, 3) over the vertices [rb, re)
+hipError_t launch_star3(const int64_t* rp, int64_t rb, int64_t re, unsigned long long* out, int grid, hipStream_t st);
 // Diamonds over the directed edges [e0, e1) from the per-edge triangle array.
 hipError_t launch_p2_edges(const int32_t* src, const int32_t* ci, const int32_t* tri, int64_t e0, int64_t e1,
                            unsigned long long* out, int grid, hipStream_t st);

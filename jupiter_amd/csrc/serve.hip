@@ -358,6 +358,8 @@ extern "C" int jgpm_serve_start(jgpm_ctx_t ctx, const jgpm_serve_config* cfg, jg
     }
     L->ctx->tune = ctx->tune;
     L->ctx->prof_on = false;  // nobody can ask a lane's context for its profile
+    // workspaces beyond the footprints that admission counts share the budget
+    L->ctx->ws_cap = (size_t)(s->cfg.hbm_budget_bytes / s->cfg.heavy_lanes);
     s->lanes.push_back(L);
     L->th = std::thread(lane_loop, s, L);
   }

@@ -293,16 +293,20 @@ __device__ __forceinline__ int32_t dag_t(const TriArgs& a, int32_t x, int32_t y,
 // Adds a wave's sum to the result.  P5's and P10's sums count every value
 // twice: the half is added, and an odd sum pairs up with another through a
 // flag (the total is even).
-template <int P>
-__device__ __forceinline__ void tri_add(const TriArgs& a, uint64_t acc) {
+__device__ __forceinline__ void add_half(uint64_t acc, unsigned long long* flag, uint64_t* out) {
   acc = wave_sum_u64(acc);
   if (lane() != 0 || !acc) return;
+  const uint64_t half = (uint64_t)((int64_t)acc >> 1);
+  const uint64_t odd = (acc & 1) ? atomicXor(flag, 1ull) : 0;
+  atomicAdd((unsigned long long*)out, (unsigned long long)(half + odd));
+}
+template <int P>
+__device__ __forceinline__ void tri_add(const TriArgs& a, uint64_t acc) {
   if constexpr (is_twice<P>()) {
-    const uint64_t half = (uint64_t)((int64_t)acc >> 1);
-    const uint64_t odd = (acc & 1) ? atomicXor(a.ctr + 6, 1ull) : 0;
-    atomicAdd((unsigned long long*)a.out, (unsigned long long)(half + odd));
+    add_half(acc, a.ctr + 6, a.out);
   } else {
-    atomicAdd((unsigned long long*)a.out, (unsigned long long)acc);
+    acc = wave_sum_u64(acc);
+    if (lane() == 0 && acc) atomicAdd((unsigned long long*)a.out, (unsigned long long)acc);
   }
 }
 
@@ -713,6 +717,36 @@ __global__ void __launch_bounds__(256) k_edge_base(const int64_t* rp, const int3
   if (lane() == 0 && acc) atomicAdd((unsigned long long*)out, (unsigned long long)acc);
 }
 
+// P3 and tailed triangles over the edges [e0, e1) of a root range, from the
+// triangle counts alone.  P3's value of (v0, v1) sums, over the triangles v0
+// v1 v2 with v2 > v1, D0 - d0 + 4 - (d1 + d2) - (t01 + t02), which is symmetric in
+// v1 and v2: per vertex o with T = half the sum of t over its edges, it is
+//   T (D - d + 4) - sum over its edges (o, p) of t (t + d(p)),
+// D the sum of its neighbours' degrees.  Tailed triangles: T (d - 2).  Edge by
+// edge, twice the value: three coalesced streams and, where t > 0, the degree
+// of p (R-MAT 18 P3: 14.7 ms over triangles, an intersection per edge of the
+// range below that, 0.1 ms so).
+template <bool P3>
+__global__ void __launch_bounds__(256) k_edge_sum(const int64_t* rp, const int32_t* ci, const int32_t* src,
+                                                  const int32_t* tri, const int64_t* nsum, int64_t e0, int64_t e1,
+                                                  unsigned long long* flag, uint64_t* out) {
+  uint64_t acc = 0;
+  for (int64_t e = e0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < e1; e += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t t = tri[e];
+    if (t == 0) continue;
+    const int32_t o = src[e];
+    const int64_t d = rp[o + 1] - rp[o];
+    if constexpr (P3) {
+      const int32_t p = ci[e];
+      const int64_t dp = rp[p + 1] - rp[p];
+      acc += (uint64_t)(t * (nsum[o] - d + 4) - 2 * t * (t + dp));
+    } else {
+      acc += (uint64_t)(t * (d - 2));
+    }
+  }
+  add_half(acc, flag, out);
+}
+
 // sum of tri over each vertex's edges
 __global__ void __launch_bounds__(256) k_root_tri(const int64_t* rp, const int32_t* tri, int32_t nv, int64_t* sum) {
   const int64_t nw = (int64_t)gridDim.x * 4;
@@ -793,6 +827,19 @@ hipError_t launch_edge_base(const int64_t* rp, const int32_t* ci, const int32_t*
   const int64_t blocks = (e1 - e0 + 255) / 256;
   hipLaunchKernelGGL(k_edge_base, dim3((unsigned)(blocks < num_cu * 8 ? blocks : num_cu * 8)), dim3(256), 0, st, rp, ci,
                      src, tri, e0, e1, mode, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_edge_sum(bool p3, const int64_t* rp, const int32_t* ci, const int32_t* src, const int32_t* tri,
+                           const int64_t* nsum, int64_t e0, int64_t e1, unsigned long long* flag, uint64_t* out,
+                           int num_cu, hipStream_t st) {
+  if (e1 <= e0) return hipSuccess;
+  const int64_t blocks = (e1 - e0 + 255) / 256;
+  const dim3 grid((unsigned)(blocks < num_cu * 8 ? blocks : num_cu * 8));
+  if (p3)
+    hipLaunchKernelGGL(k_edge_sum<true>, grid, dim3(256), 0, st, rp, ci, src, tri, nsum, e0, e1, flag, out);
+  else
+    hipLaunchKernelGGL(k_edge_sum<false>, grid, dim3(256), 0, st, rp, ci, src, tri, nsum, e0, e1, flag, out);
   return hipGetLastError();
 }
 
