@@ -1025,6 +1025,47 @@ struct Lay {
   static constexpr size_t SLOT = al(U_OFF + U_SIZE);
 };
 
+// v with lane l's value replaced by the wave-uniform x (v_writelane; there is no
+// builtin for the intrinsic)
+extern "C" __device__ int lane_set(int x, int l, int v) __asm("llvm.amdgcn.writelane.i32");
+
+// ---------------------------------------------------------------------------
+// Hub rows: out-neighbourhoods as bitmaps, of the vertices at the `top` last
+// positions of the DAG's order.  Counted from the end (p = nv - 1 - ord[v]) all
+// out-neighbours of p are below p, so row p holds p + 1 bits, in lines of 128
+// bytes (1,024 bits), the rows one after another.
+struct HubRows {
+  const uint32_t* bits = nullptr;
+  int32_t top = 0;  // 0: none
+  int32_t nv = 0;
+};
+__host__ __device__ __forceinline__ uint32_t hub_row_word(uint32_t p) {  // first word of row p; p <= 65,536
+  const uint32_t b = p >> 10;
+  return 32u * (1024u * (b * (b + 1) / 2) + (p & 1023u) * (b + 1));
+}
+
+// Tests this lane's column (word cw, bit mask cm of a hub row) in RB rows
+// whose first words lanes 0 .. RB - 1 hold in rw; f(k, word) gets row k's 64
+// answers.  Every row is one gather of 4 bytes a lane and a ballot, 16 rows in
+// flight.
+template <int RB, class F>
+__device__ __forceinline__ void hub_test(const uint32_t* bits, uint32_t rw, uint32_t cw, uint32_t cm, int n, F f) {
+  constexpr int U = RB < 16 ? RB : 16;
+  const uint32_t cb = cw * 4u;
+#pragma unroll
+  for (int k0 = 0; k0 < RB; k0 += U) {
+    if (k0 >= n) break;
+    uint32_t w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t so = (uint32_t)__builtin_amdgcn_readlane((int)rw, k0 + u);
+      w[u] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(bits + so) + cb);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) f(k0 + u, __ballot((w[u] & cm) != 0u));
+  }
+}
+
 // Process one root v0 (list N+(v0) = ci[b0 .. b0 + d)) with a group of G
 // waves: build the bitmap rows in `rowp` and add the root's k-cliques (or,
 // with BYTES, its work-model bytes) to `acc`.  `ar` is the group's LDS
@@ -1032,7 +1073,8 @@ struct Lay {
 template <int G, int WMAX, int K, bool BYTES, bool LROWS, int PHASE = 0>
 __device__ void process_root(const int64_t* __restrict__ rp, const int32_t* __restrict__ ci,
                              const int32_t* __restrict__ ord, int64_t b0, int d, int ratio, unsigned char* ar,
-                             uint64_t* rowp, int32_t* s_wtot, uint64_t& acc, uint32_t* grow = nullptr) {
+                             uint64_t* rowp, int32_t* s_wtot, uint64_t& acc, uint32_t* grow = nullptr,
+                             const HubRows hub = HubRows()) {
   // PHASE 0: build and count; 1: build only (rows left in rowp); 2: count
   // only (rowp already holds the rows of this root).  grow: a global row
   // counter (zero before) that several groups counting the same root share;
@@ -1064,6 +1106,7 @@ __device__ void process_root(const int64_t* __restrict__ rp, const int32_t* __re
   // Multi-word roots number their members in DAG order (rank of ord[]), so
   // every row only has bits above its own position.
   constexpr bool RANK = LY::MULTI;
+  constexpr bool SORT = WMAX > 1 && !BYTES;  // members in that order for their hub rows
   const int W = (d + 63) >> 6;
   const RowLayout lay(W);
   if constexpr (PHASE != 2) {
@@ -1073,34 +1116,121 @@ __device__ void process_root(const int64_t* __restrict__ rp, const int32_t* __re
   // ---- stage root list and segment descriptors
   for (int t = r; t < d; t += Grp<G>::size) L[t] = ci[b0 + t];
   for (int t = r; t < (d + 31) / 32; t += Grp<G>::size) hfl[t] = 0u;
+  if constexpr (NEED_ROWS) {
+    for (int t = r; t < d * lay.S; t += Grp<G>::size) rowp[t] = 0;
+  }
   Grp<G>::sync();
+  // places from the end of the DAG's order, of the members as they are
+  // ranked (the second half of the key region, before the hash table)
+  int32_t* const sp = key + DM;
   for (int t = r; t < d; t += Grp<G>::size) {
     int32_t u = L[t];
+    int32_t o = 0;
+    if (RANK || hub.top) o = ord[u];
+    if (RANK || SORT) key[t] = o;
+    if (hub.top && hub.nv - 1 - o < hub.top) {  // its row is read from its bitmap
+      off[t] = 0;
+      continue;
+    }
     int64_t s = rp[u];
     int du = (int)(rp[u + 1] - s);
     bool heavy = du > 64 && du > ratio * d;
     ub[t] = s;
     off[t] = heavy ? 0 : du;
     if (heavy) atomicOr(&hfl[t >> 5], 1u << (t & 31));
-    if constexpr (RANK) key[t] = ord[u];
     if constexpr (BYTES) acc += 16 + 4 * (uint64_t)du;  // f(v1) of the edge (v0, L[t])
   }
-  if constexpr (RANK) {
+  if (RANK || (SORT && hub.top)) {
     Grp<G>::sync();
     for (int t = r; t < d; t += Grp<G>::size) {
       const int32_t kt = key[t];
       int c = 0;
       for (int s2 = 0; s2 < d; ++s2) c += key[s2] < kt;
-      rnk[t] = (int16_t)c;
+      if constexpr (RANK) rnk[t] = (int16_t)c;
+      if (SORT && hub.top) sp[c] = hub.nv - 1 - kt;
     }
   }
+  if constexpr (!LROWS && NEED_ROWS) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
   Grp<G>::sync();
+  // ---- rows of the members with a bitmap: 64 members are tested in a row by
+  // one gather.  A member after another in the order is its neighbour or
+  // not, so ranked members only need the pairs above the diagonal.
+  int nout = d;  // members without one
+  if (!BYTES && hub.top) {
+    const int hd = uni(d), hwv = uni(wv);
+    if constexpr (WMAX == 1) {
+      constexpr int RB = 64 / G;
+      const int r0 = hwv * RB;
+      const uint32_t p = ln < d ? (uint32_t)(hub.nv - 1 - ord[L[ln]]) : 0xffffffffu;
+      const bool mine = p < (uint32_t)hub.top;
+      const uint64_t hm = __ballot(mine);
+      nout = d - __popcll(hm);
+      const uint32_t rw = (uint32_t)__shfl((int)(mine ? hub_row_word(p) : 0u), (r0 + ln) & 63);
+      uint32_t lo = 0, hi = 0;
+      uint32_t hits = 0;
+      hub_test<RB>(hub.bits, rw, mine ? p >> 5 : 0u, mine ? 1u << (p & 31) : 0u, hd - r0, [&](int k, uint64_t m) {
+        const uint32_t pk = (uint32_t)__builtin_amdgcn_readlane((int)p, r0 + k);
+        m &= __ballot(p < pk);
+        if (!((hm >> (r0 + k)) & 1)) m = 0;
+        if constexpr (NEED_ROWS) {
+          lo = (uint32_t)lane_set((int)(uint32_t)m, k, (int)lo);
+          hi = (uint32_t)lane_set((int)(uint32_t)(m >> 32), k, (int)hi);
+        } else {
+          hits += (uint32_t)__popcll(m);
+        }
+      });
+      if constexpr (NEED_ROWS) {
+        if (ln < RB && r0 + ln < d) rowp[r0 + ln] = ((uint64_t)hi << 32) | lo;
+      } else if (ln == 0) {
+        acc += hits;
+      }
+    } else {
+      nout = 0;
+      for (int t0 = 0; t0 < hd; t0 += 64) nout += __popcll(__ballot(t0 + ln < hd && sp[min(t0 + ln, hd - 1)] >= hub.top));
+      // units of 32 rows by 64 columns, column by column, round robin
+      const int nb = (hd + 31) >> 5, hW = (hd + 63) >> 6;
+      uint32_t hits = 0;
+      for (int u = hwv, c = 0, first = 0; nout < hd;) {
+        const int rows = min(nb, 2 * c + 2);  // row blocks of column c
+        if (u - first >= rows) {
+          first += rows;
+          if (++c >= hW) break;
+          continue;
+        }
+        const int r0 = (u - first) * 32;
+        u += G;
+        if (r0 + 32 <= nout) continue;
+        const int col = c * 64 + ln;
+        const uint32_t q = col < d ? (uint32_t)sp[col] : 0xffffffffu;
+        const bool mine = q < (uint32_t)hub.top;
+        const int ri = r0 + (ln & 31);
+        const uint32_t p = ri < d ? (uint32_t)sp[ri] : 0xffffffffu;
+        const uint32_t rw = p < (uint32_t)hub.top ? hub_row_word(p) : 0u;
+        uint32_t lo = 0, hi = 0;
+        hub_test<32>(hub.bits, rw, mine ? q >> 5 : 0u, mine ? 1u << (q & 31) : 0u, hd - r0, [&](int k, uint64_t m) {
+          if (c == (r0 >> 6)) m &= ~1ull << ((r0 + k) & 63);
+          if constexpr (RANK) {
+            lo = (uint32_t)lane_set((int)(uint32_t)m, k, (int)lo);
+            hi = (uint32_t)lane_set((int)(uint32_t)(m >> 32), k, (int)hi);
+          } else {
+            if (r0 + k >= nout) hits += (uint32_t)__popcll(m);
+          }
+        });
+        if constexpr (RANK)
+          if (ln < 32 && ri >= nout && ri < d) rowp[lay(ri, c)] = ((uint64_t)hi << 32) | lo;
+      }
+      if (!RANK && ln == 0) acc += hits;
+    }
+    Grp<G>::sync();
+  }
   if constexpr (BYTES) {
     for (int t = r; t < d; t += Grp<G>::size) {
       const int pos = RANK ? (int)rnk[t] : t;
       wL[pos] = 16u + 4u * (uint32_t)(rp[L[t] + 1] - ub[t]);
     }
   }
+  if constexpr (K == 3 && BYTES) return;  // TC work model needs no build
+  if (nout > 0) {
   // hash table of the members: slot -> position in L (power of two >= 4d
   // slots, so probes stay short and an empty slot always exists)
   int hs = 0, hshift = 0;
@@ -1131,12 +1261,7 @@ __device__ void process_root(const int64_t* __restrict__ rp, const int32_t* __re
       }
     }
   }
-  if constexpr (NEED_ROWS) {
-    for (int t = r; t < d * lay.S; t += Grp<G>::size) rowp[t] = 0;
-  }
-  if constexpr (!LROWS && NEED_ROWS) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
   Grp<G>::sync();
-  if constexpr (K == 3 && BYTES) return;  // TC work model needs no build
   group_excl_scan<G>(off, d, s_wtot);
   const int T = off[d];
   // light lists: element f of the stream sits at ci[ub[i] + f] (one LDS read
@@ -1220,6 +1345,7 @@ __device__ void process_root(const int64_t* __restrict__ rp, const int32_t* __re
       }
     }
   }
+  }  // members without a bitmap
   if constexpr (!LROWS && NEED_ROWS) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
   if (G > 1 && r == 0) s_wtot[G] = 0;  // row counter of the count phase (multi-word rows)
   Grp<G>::sync();

@@ -9,8 +9,14 @@
 // whose DAG source is v0.
 //
 // Design (one root vertex v0 per task, L = N+(v0) sorted, d = |L|):
-//  1. Build.  L is staged in LDS.  The out-lists N+(L[i]) of all i are
-//     streamed as one flattened, coalesced sequence (a thread's element knows
+//  1. Build.  L is staged in LDS.  The members among the last places of the
+//     DAG's order have their out-neighbourhoods as bitmaps (hub rows), so 64
+//     pairs of members are one gather and a ballot, and ranked members need
+//     the pairs above the diagonal only: on R-MAT 22, 1.1e8 gathers in place of
+//     nine tenths of 2.9e10 streamed elements, each with its hash probes in LDS
+//     (one quarter of the roots, P13: all builds 33 -> 7.5 ms, the query 36.0 ->
+//     9.8; what is left waits on the gathers' cache lines).  The out-lists
+//     N+(L[i]) of the other members i are streamed as one flattened, coalesced sequence (a thread's element knows
 //     its list by a forward cursor over the LDS segment offsets); each element
 //     is looked up in L (binary search for one-word roots, a 16-bit position
 //     hash otherwise) and, if present at position p, bit p of row i is set
@@ -36,6 +42,54 @@
 namespace jk {
 
 // ----------------------------------------------------------------------------
+// Hub rows.  First the vertices of the places (inv), then a wave per row: set
+// in LDS, written once (65,536 rows of R-MAT 22: 272 MB).
+__global__ void __launch_bounds__(256) k_hub_places(const int32_t* ord, int32_t nv, int32_t top, int32_t* inv) {
+  for (int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x; v < nv; v += (int64_t)gridDim.x * 256) {
+    const int32_t p = nv - 1 - ord[v];
+    if (p < top) inv[p] = (int32_t)v;
+  }
+}
+__global__ void __launch_bounds__(256) k_hub_rows(const int64_t* rp, const int32_t* ci, const int32_t* ord, int32_t nv,
+                                                  int32_t top, const int32_t* inv, uint32_t* bits) {
+  __shared__ __attribute__((aligned(16))) uint32_t s_row[4][HUB_TOP_MAX / 32];
+  uint32_t* const row = s_row[threadIdx.x >> 6];
+  uint4* const row4 = reinterpret_cast<uint4*>(row);
+  const int ln = lane_id();
+  for (int p = uni((int)(blockIdx.x * 4 + (threadIdx.x >> 6))); p < top; p += (int)gridDim.x * 4) {
+    const int32_t v = inv[p];
+    const int64_t b = rp[v], e = rp[v + 1];
+    const int n4 = 8 * ((p >> 10) + 1);
+    for (int t = ln; t < n4; t += 64) row4[t] = make_uint4(0u, 0u, 0u, 0u);
+    __syncwarp();
+    for (int64_t k = b + ln; k < e; k += 64) {
+      const int32_t q = nv - 1 - ord[ci[k]];
+      if (q < p) atomicOr(&row[q >> 5], 1u << (q & 31));
+    }
+    __syncwarp();
+    uint4* const dst = reinterpret_cast<uint4*>(bits + hub_row_word((uint32_t)p));
+    for (int t = ln; t < n4; t += 64) dst[t] = row4[t];
+    __syncwarp();
+  }
+}
+
+// a test of place q in row p reads word q / 32 also where q > p: past the last
+// row at most top / 32 words
+size_t hub_rows_words(int top) { return (size_t)hub_row_word((uint32_t)top) + (size_t)top / 32 + 32; }
+
+hipError_t launch_hub_rows(const int64_t* rp, const int32_t* ci, const int32_t* ord, int32_t nv, int32_t top,
+                           int32_t* inv, uint32_t* bits, int num_cu, hipStream_t st) {
+  if (top < 1 || top > nv || top > HUB_TOP_MAX) return hipErrorInvalidValue;
+  const int64_t vb = ((int64_t)nv + 255) / 256;
+  hipLaunchKernelGGL(k_hub_places, dim3((unsigned)(vb < num_cu * 8 ? vb : num_cu * 8)), dim3(256), 0, st, ord, nv, top,
+                     inv);
+  const int rb = (top + 3) / 4;
+  hipLaunchKernelGGL(k_hub_rows, dim3((unsigned)(rb < num_cu * 5 ? rb : num_cu * 5)), dim3(256), 0, st, rp, ci, ord, nv,
+                     top, inv, bits);
+  return hipGetLastError();
+}
+
+// ----------------------------------------------------------------------------
 // Kernel.  G waves per root; WPB roots (groups) per block when G == 1.
 // WMAX words per row => roots with d <= 64 * WMAX.  LROWS: rows in LDS,
 // otherwise in a per-block slice of global scratch.
@@ -49,6 +103,7 @@ namespace jk {
 template <int WMAX, int K, bool BYTES>
 constexpr int min_waves() {
   if (BYTES) return 1;
+  if (WMAX == 1 && K < 6) return 8;  // all blocks of the grid resident: roots are dealt by index
   if (K == 4 && WMAX == 8) return 6;
   if (K == 5 && WMAX == 4) return 8;
   if (K == 5 && WMAX == 8) return 6;
@@ -64,38 +119,88 @@ clique_kernel(CliqueArgs a) {
   constexpr int NT = 64 * G * WPB;
   __shared__ __attribute__((aligned(16))) unsigned char s_arena[WPB][LY::SLOT];
   __shared__ int32_t s_wtot[G + 1];
-  __shared__ int64_t s_task;
+  __shared__ int32_t s_task;
   const int slot = (G == 1) ? (int)(threadIdx.x >> 6) : 0;
   unsigned char* ar = s_arena[slot];
   uint64_t* rowp = LROWS ? reinterpret_cast<uint64_t*>(ar + LY::R_OFF)
                          : (a.gscr + (int64_t)blockIdx.x * DM * WMAX);
   const int64_t* __restrict__ rp = a.rp;
   uint64_t acc = 0;
-  // a group's first tasks are its own index, the queue deals the others: the
-  // small launches end without a counter round trip
-  for (bool first = true;; first = false) {
-    int64_t base;
-    if constexpr (G == 1) {
-      base = first ? ((int64_t)blockIdx.x * WPB + slot) * a.chunk
-                   : (int64_t)gridDim.x * WPB * a.chunk + (int64_t)wave_take(a.qctr, (uint32_t)a.chunk);
-    } else {
-      if (first) {
-        base = blockIdx.x;
-      } else {
-        if (threadIdx.x == 0) s_task = (int64_t)gridDim.x + (int64_t)atomicAdd(a.qctr, 1u);
-        __syncthreads();
-        base = s_task;
-        __syncthreads();
+  const HubRows hub{a.hub, a.hub_top, a.nv};
+  if constexpr (G == 1) {
+    // Roots are dealt by index, without a counter (one address takes an atomic
+    // every 12 ns or so: 8,192 waves that only learn that the queue is empty
+    // would wait 100 us).  A wave looks at 64 roots at a time, a lane each, so
+    // roots outside [dmin, dmax] cost nothing: a.chunk neighbours from each of
+    // 64 / a.chunk places all over the range, turned by an odd number from place
+    // to place, since R-MAT degrees follow the bits of the id.
+    const int ln = lane_id();
+    const uint32_t nw = gridDim.x * WPB, w = blockIdx.x * WPB + slot;  // waves, this one
+    const int lg = __builtin_ctz(a.chunk);
+    const int64_t nplace = (a.ntasks + a.chunk - 1) >> lg;
+    const int per = 64 >> lg;  // places per look
+    for (int64_t s0 = 0; s0 * nw < nplace; s0 += per) {
+      const int64_t row = s0 + (ln >> lg);
+      const int64_t place = row * nw + (uint32_t)(w + (uint32_t)row * 0x9e3779b1u) % nw;
+      const int64_t task = (place << lg) + (ln & (a.chunk - 1));
+      int64_t lb = 0;
+      int ld = -1;
+      if (task < a.ntasks) {
+        const int32_t v0 = a.ids ? a.ids[task] : (int32_t)(a.rb + task);
+        lb = rp[v0];
+        ld = (int)(rp[v0 + 1] - lb);
+      }
+      uint64_t m = __ballot(ld >= a.dmin && ld <= a.dmax && ld <= DM && ld >= 0);
+      while (m) {
+        const int l = __builtin_ctzll(m);
+        m &= m - 1;
+        process_root<G, WMAX, K, BYTES, LROWS>(rp, a.ci, a.ord, (int64_t)readlane_u64((uint64_t)lb, l),
+                                               __builtin_amdgcn_readlane(ld, l), a.ratio, ar, rowp, s_wtot, acc,
+                                               nullptr, hub);
       }
     }
-    if (base >= a.ntasks) break;
-    const int64_t tend = min(a.ntasks, base + (G == 1 ? (int64_t)a.chunk : 1));
-    for (int64_t task = base; task < tend; ++task) {
+  } else if constexpr (WMAX == 1) {
+    // 6- and 7-cliques of one-word roots differ too much to be dealt by index:
+    // a.chunk neighbours at a time from the queue
+    const int ln = lane_id();
+    for (int64_t base = (int64_t)blockIdx.x * a.chunk; base < a.ntasks;) {
+      int64_t lb = 0;
+      int ld = -1;
+      if (ln < a.chunk && base + ln < a.ntasks) {
+        const int32_t v0 = (int32_t)(a.rb + base + ln);
+        lb = rp[v0];
+        ld = (int)(rp[v0 + 1] - lb);
+      }
+      uint64_t m = __ballot(ld >= a.dmin && ld <= a.dmax && ld <= DM);
+      while (m) {
+        const int l = __builtin_ctzll(m);
+        m &= m - 1;
+        process_root<G, WMAX, K, BYTES, LROWS>(rp, a.ci, a.ord, (int64_t)readlane_u64((uint64_t)lb, l),
+                                               __builtin_amdgcn_readlane(ld, l), a.ratio, ar, rowp, s_wtot, acc,
+                                               nullptr, hub);
+      }
+      if (threadIdx.x == 0) s_task = (int32_t)(gridDim.x * (uint32_t)a.chunk + atomicAdd(a.qctr, (uint32_t)a.chunk));
+      __syncthreads();
+      base = s_task;
+      __syncthreads();
+    }
+  } else {
+    // a group's first root is its own index, the queue deals the others: the
+    // small launches end without a counter round trip
+    for (bool first = true;; first = false) {
+      int32_t task = (int32_t)blockIdx.x;
+      if (!first) {
+        if (threadIdx.x == 0) s_task = (int32_t)(gridDim.x + atomicAdd(a.qctr, 1u));
+        __syncthreads();
+        task = s_task;
+        __syncthreads();
+      }
+      if (task >= a.ntasks) break;
       const int32_t v0 = a.ids ? a.ids[task] : (int32_t)(a.rb + task);
       const int64_t b0 = rp[v0];
       const int d = (int)(rp[v0 + 1] - b0);
       if (d < a.dmin || d > a.dmax || d > DM) continue;
-      process_root<G, WMAX, K, BYTES, LROWS>(rp, a.ci, a.ord, b0, d, a.ratio, ar, rowp, s_wtot, acc);
+      process_root<G, WMAX, K, BYTES, LROWS>(rp, a.ci, a.ord, b0, d, a.ratio, ar, rowp, s_wtot, acc, nullptr, hub);
     }
   }
   block_add<NT>(acc, a.out);
@@ -121,14 +226,15 @@ __global__ void __launch_bounds__(64 * 16) clique_build_kernel(CliqueArgs a) {
   for (;;) {
     if (threadIdx.x == 0) s_task = (int64_t)atomicAdd(a.qctr, 1u);
     __syncthreads();
-    const int64_t task = s_task;
+    const int64_t task = uni((int)s_task);
     __syncthreads();
     if (task >= a.ntasks) break;
-    const int32_t v0 = a.ids[task];
+    const int32_t v0 = uni(a.ids[task]);
     const int64_t b0 = a.rp[v0];
-    const int d = (int)(a.rp[v0 + 1] - b0);
+    const int d = uni((int)(a.rp[v0 + 1] - b0));
     if (d < a.dmin || d > a.dmax || d > LY::DM) continue;
-    process_root<G, SPLIT_WMAX, K, false, true, 1>(a.rp, a.ci, a.ord, b0, d, a.ratio, s_arena, rowp, s_wtot, acc);
+    process_root<G, SPLIT_WMAX, K, false, true, 1>(a.rp, a.ci, a.ord, b0, d, a.ratio, s_arena, rowp, s_wtot, acc,
+                                                   nullptr, HubRows{a.hub, a.hub_top, a.nv});
     const int n = d * RowLayout((d + 63) >> 6).S;
     uint64_t* dst = a.gscr + (size_t)task * ROWW;
     for (int t = threadIdx.x; t < n; t += 64 * G) dst[t] = rowp[t];
@@ -154,12 +260,12 @@ __global__ void __launch_bounds__(64 * split_count_waves<K>()) clique_count_kern
   for (;;) {
     if (threadIdx.x == 0) s_task = (int64_t)atomicAdd(a.qctr, 1u);
     __syncthreads();
-    const int64_t task = s_task;
+    const int64_t task = uni((int)s_task);
     __syncthreads();
     if (task >= a.ntasks) break;
-    const int32_t v0 = a.ids[task];
+    const int32_t v0 = uni(a.ids[task]);
     const int64_t b0 = a.rp[v0];
-    const int d = (int)(a.rp[v0 + 1] - b0);
+    const int d = uni((int)(a.rp[v0 + 1] - b0));
     if (d < a.dmin || d > a.dmax || d > LY::DM) continue;
     const int n = d * RowLayout((d + 63) >> 6).S;
     const uint64_t* src = a.gscr + (size_t)task * ROWW;
@@ -211,11 +317,12 @@ __global__ void __launch_bounds__(64 * G) clique_rows_build_kernel(CliqueArgs a)
   uint64_t* rowp = reinterpret_cast<uint64_t*>(s_arena + LY::R_OFF);
   uint64_t acc = 0;
   for (int64_t task = blockIdx.x; task < a.ntasks; task += gridDim.x) {
-    const int32_t v0 = a.ids[task];
+    const int32_t v0 = uni(a.ids[task]);
     const int64_t b0 = a.rp[v0];
-    const int d = (int)(a.rp[v0 + 1] - b0);
+    const int d = uni((int)(a.rp[v0 + 1] - b0));
     if (d < a.dmin || d > a.dmax || d > LY::DM) continue;
-    process_root<G, WMAX, 4, false, true, 1>(a.rp, a.ci, a.ord, b0, d, a.ratio, s_arena, rowp, s_wtot, acc);
+    process_root<G, WMAX, 4, false, true, 1>(a.rp, a.ci, a.ord, b0, d, a.ratio, s_arena, rowp, s_wtot, acc, nullptr,
+                                             HubRows{a.hub, a.hub_top, a.nv});
     const int n = d * RowLayout((d + 63) >> 6).S;
     uint64_t* dst = a.gscr + (size_t)task * rows_slot(WMAX);
     for (int t = threadIdx.x; t < n; t += 64 * G) dst[t] = rowp[t];
@@ -246,7 +353,7 @@ __global__ void __launch_bounds__(256) clique_rows_count_kernel(CliqueArgs a) {
     const int i0 = (int)(u / a.ntasks);
     const int64_t task = u - (int64_t)i0 * a.ntasks;
     const int i = uni(t < early ? i0 : i0 + DM / 4);
-    const int32_t v0 = a.ids[task];
+    const int32_t v0 = uni(a.ids[task]);
     const int64_t b0 = a.rp[v0];
     const int d = uni((int)(a.rp[v0 + 1] - b0));
     if (i >= d || d < a.dmin || d > a.dmax || d > DM) continue;
@@ -342,15 +449,16 @@ __global__ void __launch_bounds__(64 * 16) clique_glb_build_kernel(CliqueArgs a)
   for (;;) {
     if (threadIdx.x == 0) s_task = (int64_t)atomicAdd(a.qctr, 1u);
     __syncthreads();
-    const int64_t task = s_task;
+    const int64_t task = uni((int)s_task);
     __syncthreads();
     if (task >= a.ntasks) break;
-    const int32_t v0 = a.ids[task];
+    const int32_t v0 = uni(a.ids[task]);
     const int64_t b0 = a.rp[v0];
-    const int d = (int)(a.rp[v0 + 1] - b0);
+    const int d = uni((int)(a.rp[v0 + 1] - b0));
     if (d < a.dmin || d > a.dmax || d > LY::DM) continue;
     process_root<G, GLB_WMAX, K, false, false, 1>(a.rp, a.ci, a.ord, b0, d, a.ratio, s_arena,
-                                                  a.gscr + (size_t)task * GSLOT, s_wtot, acc);
+                                                  a.gscr + (size_t)task * GSLOT, s_wtot, acc, nullptr,
+                                                  HubRows{a.hub, a.hub_top, a.nv});
   }
 }
 
@@ -375,13 +483,13 @@ __global__ void __launch_bounds__(64 * 8) clique_glb_count_kernel(CliqueArgs a) 
     for (;;) {
       if (threadIdx.x == 0) s_item = (int64_t)atomicAdd(qx + q, 1u);
       __syncthreads();
-      const int64_t item = s_item;
+      const int64_t item = uni((int)s_item);
       __syncthreads();
       if (item >= nq) break;
       const int64_t task = (item / a.rep) * 8 + q;
-      const int32_t v0 = a.ids[task];
+      const int32_t v0 = uni(a.ids[task]);
       const int64_t b0 = a.rp[v0];
-      const int d = (int)(a.rp[v0 + 1] - b0);
+      const int d = uni((int)(a.rp[v0 + 1] - b0));
       if (d < a.dmin || d > a.dmax || d > LY::DM) continue;
       process_root<G, GLB_WMAX, K, false, false, 2>(a.rp, a.ci, a.ord, b0, d, a.ratio, s_arena,
                                                     a.gscr + (size_t)task * GSLOT, s_wtot, acc, a.rowctr + task);

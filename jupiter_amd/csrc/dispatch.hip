@@ -84,6 +84,37 @@ static int tri_args(jgpm_graph_s* g, hipStream_t st, jk::TriArgs& a) {
   return JGPM_OK;
 }
 
+// Hub rows for a clique launch over the roots [rb, re), made on the stream.
+// None where the range holds too few edges to pay for two small launches
+// (R-MAT 10, 10,000 edges: TC 23 us without and 26 with; R-MAT 12, 52,000: 66 and
+// 38), where there is no room, or while capturing.  As many rows as take no more
+// than four words an edge of the range, at least 16,384 (8 MiB at half the
+// square), at most 65,536 (R-MAT 22, a quarter of the roots: 0.21 ms for 272
+// MB; P13 9.75 ms, with 32,768 rows 10.2); triangle counts, whose streams are
+// cheaper, at most 32,768 (TC 7.9 ms, with 65,536 rows 8.7).
+int clique_hub_rows(jgpm_graph_s* g, int k, int64_t rb, int64_t re, hipStream_t st, jk::CliqueArgs& a) {
+  jgpm_ctx_s* c = exec_ctx(g);
+  const int32_t nv = g->dag.nv;
+  const int64_t ne = g->dag_rp_h[re] - g->dag_rp_h[rb];
+  if (c->capturing || ne < 16384) return JGPM_OK;
+  const int32_t cap = std::min(nv, k == 3 ? jk::HUB_TOP_MAX / 2 : jk::HUB_TOP_MAX);
+  int32_t top = std::min(cap, 16384);
+  while (top < cap && (int64_t)jk::hub_rows_words(std::min(cap, 2 * top)) <= 4 * ne) top = std::min(cap, 2 * top);
+  const size_t bits_b = sizeof(uint32_t) * jk::hub_rows_words(top);
+  const int rc = grow(c, c->d_hub, c->hub_bytes, bits_b + sizeof(int32_t) * (size_t)top, c->ws_cap, st);
+  if (rc == JGPM_E_NOMEM) return JGPM_OK;
+  if (rc) return rc;
+  uint32_t* bits = static_cast<uint32_t*>(c->d_hub);
+  int32_t* inv = reinterpret_cast<int32_t*>(static_cast<unsigned char*>(c->d_hub) + bits_b);
+  prof_begin(c, st, "hub_rows");
+  const hipError_t e = jk::launch_hub_rows(g->dag.rp, g->dag.ci, g->d_ord, nv, top, inv, bits, c->num_cu, st);
+  prof_end(c, st);
+  a.hub = bits;
+  a.hub_top = top;
+  a.nv = nv;
+  return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
+}
+
 // Lazily built per-graph arrays of the symmetric kernels.
 int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t st) {
   jgpm_ctx_s* c = exec_ctx(g);

@@ -324,6 +324,7 @@ extern "C" int jgpm_shutdown(jgpm_ctx_t c) {
   if (c->d_p1) (void)hipFree(c->d_p1);
   if (c->d_te) (void)hipFree(c->d_te);
   if (c->d_ego) (void)hipFree(c->d_ego);
+  if (c->d_hub) (void)hipFree(c->d_hub);
   if (c->d_bq) (void)hipFree(c->d_bq);
   if (c->d_bcs) (void)hipFree(c->d_bcs);
   if (c->d_bcnt) (void)hipFree(c->d_bcnt);
@@ -528,8 +529,13 @@ int enqueue_clique(jgpm_graph_s* g, int k, bool bytes, int64_t rb, int64_t re, i
     }
   }
   const int maxgrid = std::max(1, c->tune.blocks_per_cu) * c->num_cu;
+  jk::CliqueArgs hub{};
+  if (!bytes && !gscr && !qctr_base && re > rb) {
+    int s4 = clique_hub_rows(g, k, rb, re, st, hub);
+    if (s4) return s4;
+  }
   for (int tier = jk::NUM_TIERS - 1; tier >= first_tier; --tier) {
-    jk::CliqueArgs a{};
+    jk::CliqueArgs a = hub;
     a.rp = g->dag.rp;
     a.ci = g->dag.ci;
     a.ord = g->d_ord;
@@ -551,9 +557,9 @@ int enqueue_clique(jgpm_graph_s* g, int k, bool bytes, int64_t rb, int64_t re, i
       a.rb = rb;
       a.ntasks = re - rb;
       if (a.ntasks <= 0) continue;
-      // roots per grab: 16 on large ranges, fewer where 16 would leave waves
-      // without work (R-MAT 14, 16,384 roots: 1024 waves of 16 roots took 362 us)
-      a.chunk = (int32_t)std::max<int64_t>(1, std::min<int64_t>(16, a.ntasks / ((int64_t)maxgrid * 8)));
+      // neighbouring roots a wave takes together (their lists lie together), as
+      // many as leave each wave some of every part of the range
+      a.chunk = a.ntasks >= (int64_t)maxgrid * 256 ? 16 : a.ntasks >= (int64_t)maxgrid * 64 ? 4 : 1;
       int64_t waves = (a.ntasks + a.chunk - 1) / a.chunk;
       grid = (int)std::min<int64_t>(maxgrid, (waves + 3) / 4);
     } else {
@@ -565,7 +571,6 @@ int enqueue_clique(jgpm_graph_s* g, int k, bool bytes, int64_t rb, int64_t re, i
       a.ids = g->tier_d[tier] + (lo - v.begin());
       a.rb = 0;
       a.ntasks = n;
-      a.chunk = 1;
       grid = (int)std::min<int64_t>(maxgrid, n);
       if (tier <= jk::TIER_LDS8 && !bytes && k >= 6 && !gscr && !c->capturing) {
         // split form: rows into global slots, then a wave per (root, row);
@@ -671,10 +676,9 @@ int enqueue_clique(jgpm_graph_s* g, int k, bool bytes, int64_t rb, int64_t re, i
     if (tier == jk::TIER_WAVE && k >= 6 && !bytes) {
       jk::CliqueArgs w = a;
       w.dmin = std::max(a.dmin, jk::clique_small_root() + 1);
-      e = jk::launch_clique(k, bytes, tier, w, (int)std::min<int64_t>(maxgrid, a.ntasks), st);
+      w.chunk = (int32_t)std::max<int64_t>(1, std::min<int64_t>(8, a.ntasks / ((int64_t)maxgrid * 8)));
+      e = jk::launch_clique(k, bytes, tier, w, (int)std::min<int64_t>(maxgrid, (a.ntasks + w.chunk - 1) / w.chunk), st);
       a.dmax = jk::clique_small_root();
-      // the second launch's queue starts at zero again
-      hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, a.qctr, 1, 0u);
     }
     if (e == hipSuccess) e = jk::launch_clique(k, bytes, tier, a, grid, st);
     prof_end(c, st);

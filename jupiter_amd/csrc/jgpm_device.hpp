@@ -42,6 +42,8 @@ struct jgpm_ctx_s {
   int64_t hcap = 0;
   unsigned long long* d_hctr = nullptr;  // their append and pop counters (6)
   size_t ws_cap = SIZE_MAX;    // bytes any one of the workspaces may take that a query can also do without
+  void* d_hub = nullptr;       // hub rows of the clique engine
+  size_t hub_bytes = 0;
   void* d_ego = nullptr;       // the graph of induced neighbourhoods of P6, P8, P10
   size_t ego_bytes = 0;
   void* d_te = nullptr;        // scratch of the triangle launches (lists, hub bitmaps)
@@ -144,6 +146,7 @@ int graph_from_host_sym(jgpm_ctx_s* c, const int64_t* rowptr, const int32_t* col
                         bool dag_only, jgpm_graph_t* out);
 int ensure_scratch(jgpm_ctx_s* c, size_t words);
 int clique_k(int pattern);
+int clique_hub_rows(jgpm_graph_s* g, int k, int64_t rb, int64_t re, hipStream_t st, jk::CliqueArgs& a);
 int enqueue_clique(jgpm_graph_s* g, int k, bool bytes, int64_t rb, int64_t re, int out_slot, hipStream_t st,
                    bool split_slots = false, int first_tier = 0, uint64_t* out_ptr = nullptr,
                    unsigned* qctr_base = nullptr, uint64_t* gscr = nullptr, size_t gscr_words = 0);

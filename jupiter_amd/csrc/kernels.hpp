@@ -33,7 +33,17 @@ struct CliqueArgs {
   uint32_t* rowctr;      // split 2048-wide count: one row counter per task, 8 queue
                          // counters before them (all zero before)
   int32_t rep;           // split 2048-wide count: blocks per task
+  const uint32_t* hub;   // hub rows (launch_hub_rows), of the hub_top last places of ord
+  int32_t hub_top;       // 0: none
+  int32_t nv;
 };
+
+// Out-neighbourhoods of the `top` last vertices of ord as bitmaps
+// (hub_rows_words(top) 32-bit words at bits; inv: top entries of scratch).
+constexpr int HUB_TOP_MAX = 65536;
+size_t hub_rows_words(int top);
+hipError_t launch_hub_rows(const int64_t* rp, const int32_t* ci, const int32_t* ord, int32_t nv, int32_t top,
+                           int32_t* inv, uint32_t* bits, int num_cu, hipStream_t st);
 
 // Query descriptor as the persistent kernel sees it.
 struct BQ {
