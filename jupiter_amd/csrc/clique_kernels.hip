@@ -77,12 +77,18 @@ __global__ void __launch_bounds__(256) k_hub_rows(const int64_t* rp, const int32
 // row at most top / 32 words
 size_t hub_rows_words(int top) { return (size_t)hub_row_word((uint32_t)top) + (size_t)top / 32 + 32; }
 
-hipError_t launch_hub_rows(const int64_t* rp, const int32_t* ci, const int32_t* ord, int32_t nv, int32_t top,
-                           int32_t* inv, uint32_t* bits, int num_cu, hipStream_t st) {
-  if (top < 1 || top > nv || top > HUB_TOP_MAX) return hipErrorInvalidValue;
+hipError_t launch_hub_places(const int32_t* ord, int32_t nv, int32_t top, int32_t* inv, int num_cu, hipStream_t st) {
   const int64_t vb = ((int64_t)nv + 255) / 256;
   hipLaunchKernelGGL(k_hub_places, dim3((unsigned)(vb < num_cu * 8 ? vb : num_cu * 8)), dim3(256), 0, st, ord, nv, top,
                      inv);
+  return hipGetLastError();
+}
+
+hipError_t launch_hub_rows(const int64_t* rp, const int32_t* ci, const int32_t* ord, int32_t nv, int32_t top,
+                           int32_t* inv, uint32_t* bits, int num_cu, hipStream_t st) {
+  if (top < 1 || top > nv || top > HUB_TOP_MAX) return hipErrorInvalidValue;
+  const hipError_t e = launch_hub_places(ord, nv, top, inv, num_cu, st);
+  if (e != hipSuccess) return e;
   const int rb = (top + 3) / 4;
   hipLaunchKernelGGL(k_hub_rows, dim3((unsigned)(rb < num_cu * 5 ? rb : num_cu * 5)), dim3(256), 0, st, rp, ci, ord, nv,
                      top, inv, bits);

@@ -43,8 +43,12 @@ static int grow(jgpm_ctx_s* c, void*& p, size_t& have, size_t need, size_t cap, 
 }
 
 // Hub bitmaps of the triangle launches: the highest-degree vertices whose
-// bitmaps fit this (R-MAT 18: its 4,096 widest vertices).
-constexpr int64_t TRI_HUB_BYTES = (int64_t)128 << 20;
+// bitmaps fit 16 bytes a directed edge, at least 128 and at most 512 MiB
+// (R-MAT 18: its 4,096 widest vertices; twice the bytes cost 0.3 of 7.8 ms for
+// P5.  R-MAT 20, 128 / 256 / 512 MiB: 92.5 / 81.4 / 75.4 ms).
+static int64_t tri_hub_bytes(int64_t nnz) {
+  return std::max<int64_t>((int64_t)128 << 20, std::min<int64_t>((int64_t)512 << 20, 16 * nnz));
+}
 
 // Arguments of the triangle launches on g, their scratch on the executing
 // context (the hub bitmaps still to be made by launch_hub_bitmaps).
@@ -64,7 +68,7 @@ static int tri_args(jgpm_graph_s* g, hipStream_t st, jk::TriArgs& a) {
   // it takes to fill the device (32 waves per CU)
   a.vchunk = std::max(1, std::min(64, nv / (64 * c->num_cu)));
   a.hwords = (((int64_t)nv + 31) / 32 + 3) & ~(int64_t)3;
-  a.nhub = (int32_t)std::min<int64_t>(g->hubs, TRI_HUB_BYTES / (4 * a.hwords));
+  a.nhub = (int32_t)std::min<int64_t>(g->hubs, tri_hub_bytes(g->sym.nnz) / (4 * a.hwords));
   a.lstride = std::max(1, g->dag.max_deg);
   size_t hub_b = 4 * (size_t)a.hwords * (size_t)a.nhub;
   const size_t list_b = (sizeof(int32_t) * 3 * (size_t)nv + 15) & ~(size_t)15;

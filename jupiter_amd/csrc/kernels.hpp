@@ -42,6 +42,8 @@ struct CliqueArgs {
 // (hub_rows_words(top) 32-bit words at bits; inv: top entries of scratch).
 constexpr int HUB_TOP_MAX = 65536;
 size_t hub_rows_words(int top);
+// inv[p] = the vertex p places from the end of ord, p < top
+hipError_t launch_hub_places(const int32_t* ord, int32_t nv, int32_t top, int32_t* inv, int num_cu, hipStream_t st);
 hipError_t launch_hub_rows(const int64_t* rp, const int32_t* ci, const int32_t* ord, int32_t nv, int32_t top,
                            int32_t* inv, uint32_t* bits, int num_cu, hipStream_t st);
 
