@@ -123,7 +123,9 @@ clique_kernel(CliqueArgs a) {
   using LY = Lay<G, WMAX, K, BYTES, LROWS>;
   constexpr int DM = LY::DM;
   constexpr int NT = 64 * G * WPB;
-  __shared__ __attribute__((aligned(16))) unsigned char s_arena[WPB][LY::SLOT];
+  constexpr bool SMALL = WMAX == 1 && K <= 5 && !BYTES;  // roots of few members many at a time
+  constexpr size_t ARENA = SMALL && sizeof(SmallRoots) > LY::SLOT ? sizeof(SmallRoots) : LY::SLOT;
+  __shared__ __attribute__((aligned(16))) unsigned char s_arena[WPB][ARENA];
   __shared__ int32_t s_wtot[G + 1];
   __shared__ int32_t s_task;
   const int slot = (G == 1) ? (int)(threadIdx.x >> 6) : 0;
@@ -157,6 +159,12 @@ clique_kernel(CliqueArgs a) {
         ld = (int)(rp[v0 + 1] - lb);
       }
       uint64_t m = __ballot(ld >= a.dmin && ld <= a.dmax && ld <= DM && ld >= 0);
+      if constexpr (SMALL) {
+        const bool small = ((m >> ln) & 1) && ld <= SMALL_D;
+        small_roots<K>(rp, a.ci, a.ord, hub, lb, small ? ld : 0, *reinterpret_cast<SmallRoots*>(ar), acc);
+        m &= ~__ballot(small);
+        __syncwarp();
+      }
       while (m) {
         const int l = __builtin_ctzll(m);
         m &= m - 1;

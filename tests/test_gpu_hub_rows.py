@@ -54,3 +54,25 @@ def test_against_general_path(ctx, name):
             print(f"[case] {name} {p} {r}", flush=True)
             assert G.count(p, r)[0] == noalloc(G, p, r), (name, p, r)
     G.free()
+
+
+@pytest.mark.parametrize("copies", [1, 300])
+def test_small_roots(ctx, copies):
+    """Disjoint cliques of 2 to 36 vertices, without bitmaps and with some of
+    the members outside them: roots of 1 to 35 members, batched and not."""
+    u, v, n = [], [], 0
+    sizes = list(range(2, 37))
+    for s in sizes:
+        a, b = np.triu_indices(s, 1)
+        u.append(n + a)
+        v.append(n + b)
+        n += s
+    u, v = np.concatenate(u), np.concatenate(v)
+    shift = np.repeat(np.arange(copies) * n, len(u))
+    perm = np.random.default_rng(1).permutation(n * copies) if copies > 1 else np.arange(n)
+    g = J.CSR.from_edges(n * copies, perm[np.tile(u, copies) + shift], perm[np.tile(v, copies) + shift])
+    G = ctx.upload(g)
+    for p, k in (("TC", 3), ("P13", 4), ("P14", 5)):
+        print(f"[case] cliques x {copies} {p}", flush=True)
+        assert G.count(p)[0] == copies * sum(comb(s, k) for s in sizes), p
+    G.free()
