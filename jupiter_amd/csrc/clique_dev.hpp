@@ -801,13 +801,13 @@ __device__ uint64_t tri_mfma1_bits(const RowT& R, const int16_t* J, int n_, int 
 // count its registers allow 12 waves per root where the 2x2 tiles of
 // tri_mfma held 8 (23.0 -> 20.7 ms).
 template <class RowT>
-__device__ uint64_t tri_mfma1(const RowT& R, const int16_t* J, int n_, int i_, int whi_, int zr_) {
+__device__ uint64_t tri_mfma1(const RowT& R, const int16_t* J, int n_, int i_, int whi_, int zr_, int Y_ = 0) {
   const int n = uni(n_), i = uni(i_), whi = uni(whi_), zr = uni(zr_);
   const int ln = lane_id();
   const int col = ln & 31, half = ln >> 5;
   const int T = (n + 31) >> 5;
   uint64_t s = 0;
-  for (int Y = 0; Y < T; ++Y) {
+  for (int Y = uni(Y_); Y < T; ++Y) {
     const int ay = 32 * Y + col;
     const int y = ay < n ? (int)J[ay] : -1;
     // words qa .. qb hold the block's members (qb <= whi: S lies in row i)
@@ -845,6 +845,91 @@ __device__ uint64_t tri_mfma1(const RowT& R, const int16_t* J, int n_, int i_, i
       s += dot16(acc, msk);
     }
   }
+  return s;
+}
+
+// The same count with 2 x 2 tiles of block pairs: a word's five loads and four
+// encodings feed four products, where one pair takes three and two for one.  The
+// 1024-wide count is bound by VALU issue (a product kept 36 % of the matrix
+// cores' cycles busy), its 12 waves per root leave 168 registers each: four
+// count accumulators, and the edge mask of one pair at a time from the words that
+// hold the Y members, after them.  (P14 on R-MAT 22, roots [0, 2^20): 20.0 -> 18.4
+// ms; 1 x 2 tiles with their masks beside them 18.3; on the 512-wide tier at four
+// waves per SIMD 8.9, one pair at six 6.1.)
+template <class RowT>
+__device__ uint64_t tri_mfma2(const RowT& R, const int16_t* J, int n_, int i_, int whi_, int zr_) {
+  const int n = uni(n_), i = uni(i_), whi = uni(whi_), zr = uni(zr_);
+  const int ln = lane_id();
+  const int col = ln & 31, half = ln >> 5;
+  const int T = (n + 31) >> 5;
+  auto member = [&](int B) -> int {
+    const int a = 32 * B + col;
+    return a < n ? (int)J[a] : -1;
+  };
+  uint64_t s = 0;
+  int Y0 = 0;
+  for (; Y0 + 1 < T; Y0 += 2) {
+    int y[2];
+    RowCur ky[2];
+    int qa[2], qb[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      y[k] = member(Y0 + k);
+      ky[k] = R.cur(y[k] >= 0 ? y[k] : zr, half);
+      qa[k] = uni(J[32 * (Y0 + k)]) >> 6;
+      qb[k] = uni(J[min(n - 1, 32 * (Y0 + k) + 31)]) >> 6;
+    }
+    const RowCur ki = R.cur(i, half);
+    for (int X0 = 0; X0 <= Y0; X0 += 2) {
+      RowCur kx[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int x = member(X0 + k);
+        kx[k] = R.cur(x >= 0 ? x : zr, half);
+      }
+      v16f32 c[2][2];
+      uint32_t va[5], vb[5];
+      auto load = [&](int q, uint32_t(&v)[5]) {
+        v[0] = R.at(ki, q);
+        v[1] = R.at(ky[0], q);
+        v[2] = R.at(ky[1], q);
+        v[3] = R.at(kx[0], q);
+        v[4] = R.at(kx[1], q);
+      };
+      auto step = [&](int q, bool first, const uint32_t(&v)[5], uint32_t(&nx)[5]) {
+        load(min(q + 1, whi), nx);
+        const v8i32 a0 = enc_a(v[1] & v[0]), a1 = enc_a(v[2] & v[0]);
+        const v8i32 b0 = enc_b(v[3]), b1 = enc_b(v[4]);
+        const v16f32 z = zero16();
+        c[0][0] = mma_fp4(a0, b0, first ? z : c[0][0]);
+        c[0][1] = mma_fp4(a0, b1, first ? z : c[0][1]);
+        c[1][0] = mma_fp4(a1, b0, first ? z : c[1][0]);
+        c[1][1] = mma_fp4(a1, b1, first ? z : c[1][1]);
+      };
+      load(qa[0], va);
+      step(qa[0], true, va, vb);
+      int q = qa[0] + 1;
+      for (; q + 1 <= whi; q += 2) {
+        step(q, false, vb, va);
+        step(q + 1, false, va, vb);
+      }
+      if (q <= whi) step(q, false, vb, va);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const uint32_t hbit = (y[k] >= 0 && ((y[k] >> 5) & 1) == half) ? 1u << (y[k] & 31) : 0u;
+        const int hq = y[k] >= 0 ? y[k] >> 6 : -1;
+#pragma unroll
+        for (int l = 0; l < 2; ++l) {
+          if (X0 + l > Y0 + k) continue;  // no edge into an earlier block
+          v16f32 m = mma_fp4(enc_a(hq == qa[k] ? hbit : 0u), enc_b(R.at(kx[l], qa[k])), zero16());
+          for (int w = qa[k] + 1; w <= qb[k]; ++w)
+            m = mma_fp4(enc_a(hq == w ? hbit : 0u), enc_b(R.at(kx[l], w)), m);
+          s += dot16(c[k][l], m);
+        }
+      }
+    }
+  }
+  if (Y0 < T) s += tri_mfma1(R, J, n, i, whi, zr, Y0);
   return s;
 }
 
@@ -1647,7 +1732,7 @@ __device__ void process_root(const int64_t* __restrict__ rp, const int32_t* __re
           // roots (rows in global memory); the edge mask is a product from
           // 512 wide up
           if constexpr (WMAX >= 32) acc += tri_mfma(R, J, n, i, whi, d - 1);
-          else if constexpr (WMAX >= 16) acc += tri_mfma1(R, J, n, i, whi, d - 1);
+          else if constexpr (WMAX >= 16) acc += tri_mfma2(R, J, n, i, whi, d - 1);
           else if constexpr (WMAX >= 8)
             __hip_atomic_fetch_add(racc, (uint32_t)tri_mfma1(R, J, n, i, whi, d - 1), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WAVEFRONT);
