@@ -72,11 +72,12 @@ struct MaxI {
   static constexpr int v = A > B ? A : B;
 };
 
-__global__ void __launch_bounds__(64 * BWPB) batch_kernel(BatchArgs a) {
+__global__ void __launch_bounds__(64 * BWPB) __attribute__((amdgpu_waves_per_eu(3))) batch_kernel(BatchArgs a) {
   constexpr int CL = MaxI<MaxI<Lay<1, 2, 7, false, true>::SLOT, Lay<1, 2, 5, false, true>::SLOT>::v,
                           MaxI<Lay<1, 2, 4, false, true>::SLOT, Lay<1, 1, 7, false, true>::SLOT>::v>::v;
   constexpr int SY = (symd::NLIST * symd::CAP + symd::STAGE) * 4;
   constexpr int ARENA = ((CL > SY ? CL : SY) + 15) & ~15;
+  static_assert(sizeof(SmallRoots) <= ARENA, "the small roots' arrays share the arena");
   __shared__ __attribute__((aligned(16))) unsigned char s_arena[BWPB][ARENA];
   __shared__ int32_t s_wtot[BWPB][2];
   const int wv = threadIdx.x >> 6;
@@ -86,20 +87,28 @@ __global__ void __launch_bounds__(64 * BWPB) batch_kernel(BatchArgs a) {
   symd::Wave w{lds_lists + symd::NLIST * symd::CAP};
   int32_t* glist = a.scr + ((int64_t)blockIdx.x * BWPB + wv) * symd::NLIST * a.scr_stride;
   const int64_t nchunks = a.cstart[a.nq];
+  // chunks per grab, as an atomic on one address takes about 12 ns: two where
+  // there are many (TC on 96 graphs of 1,000 to 131,072 vertices, 1 / 2 / 4 / 8
+  // chunks of 16 roots: 3.54 / 3.35 / 3.56 / 4.10 ms; more end in a longer tail of
+  // roots up to the hub degree)
+  const int64_t take = max((int64_t)1, min((int64_t)2, nchunks / ((int64_t)gridDim.x * BWPB * 6)));
   for (;;) {
-    int64_t t = 0;
-    if (ln == 0) t = (int64_t)atomicAdd(a.qctr, 1ull);
-    const int64_t k = __shfl(t, 0);
-    if (k >= nchunks) break;
-    // query of chunk k: last q with cstart[q] <= k
+    const int64_t k0 = (int64_t)wave_take(a.qctr, (unsigned long long)take);
+    if (k0 >= nchunks) break;
+    const int64_t k1 = min(nchunks, k0 + take);
+    // query of chunk k0: last q with cstart[q] <= k0
     int lo = 0, hi = a.nq;
     while (hi - lo > 1) {
       int mid = (lo + hi) >> 1;
-      if (a.cstart[mid] <= k) lo = mid; else hi = mid;
+      if (a.cstart[mid] <= k0) lo = mid; else hi = mid;
     }
+    for (int64_t k = k0; k < k1;) {
+    while (a.cstart[lo + 1] <= k) ++lo;
+    const int64_t kq = min(k1, a.cstart[lo + 1]);  // the grab's chunks of this query
     const BQ Q = a.q[lo];
     const int64_t u0 = (k - a.cstart[lo]) * Q.chunk;
-    int64_t u1 = min(Q.ntasks, u0 + Q.chunk);
+    int64_t u1 = min(Q.ntasks, (kq - a.cstart[lo]) * Q.chunk);
+    k = kq;
     uint64_t acc = 0;
     if (Q.kind == 102 && Q.tri) {
       // diamonds from the per-edge triangle array: lanes over the edges
@@ -109,20 +118,44 @@ __global__ void __launch_bounds__(64 * BWPB) batch_kernel(BatchArgs a) {
       }
       u1 = u0;  // no per-edge pass
     }
-    for (int64_t u = u0; u < u1; ++u) {
-      if (Q.kind < 100) {
-        const int64_t v0 = Q.base + u;
-        const int64_t b0 = Q.rp[v0];
-        const int d = (int)(Q.rp[v0 + 1] - b0);
-        if (d < Q.kind - 1 || d > a.hub) continue;
-        switch (Q.kind) {
-          case 3: batch_root<3>(Q.rp, Q.ci, Q.ord, b0, d, a.ratio, ar, s_wtot[wv], acc); break;
-          case 4: batch_root<4>(Q.rp, Q.ci, Q.ord, b0, d, a.ratio, ar, s_wtot[wv], acc); break;
-          case 5: batch_root<5>(Q.rp, Q.ci, Q.ord, b0, d, a.ratio, ar, s_wtot[wv], acc); break;
-          case 6: batch_root<6>(Q.rp, Q.ci, Q.ord, b0, d, a.ratio, ar, s_wtot[wv], acc); break;
-          case 7: batch_root<7>(Q.rp, Q.ci, Q.ord, b0, d, a.ratio, ar, s_wtot[wv], acc); break;
+    if (Q.kind < 100) {
+      // roots: a lane looks at the degree of one of 64, the small roots of 3-
+      // to 5-cliques are counted together
+      for (int64_t u = u0; u < u1; u += 64) {
+        int64_t lb = 0;
+        int ld = -1;
+        if (u + ln < u1) {
+          const int64_t v0 = Q.base + u + ln;
+          lb = Q.rp[v0];
+          ld = (int)(Q.rp[v0 + 1] - lb);
         }
-      } else {
+        uint64_t m = __ballot(ld >= Q.kind - 1 && ld <= a.hub);
+        const bool small = Q.kind <= 5 && ((m >> ln) & 1) && ld <= SMALL_D;
+        const int sd = small ? ld : 0;
+        SmallRoots& S = *reinterpret_cast<SmallRoots*>(ar);
+        switch (Q.kind) {
+          case 3: small_roots<3>(Q.rp, Q.ci, Q.ord, HubRows(), lb, sd, S, acc); break;
+          case 4: small_roots<4>(Q.rp, Q.ci, Q.ord, HubRows(), lb, sd, S, acc); break;
+          case 5: small_roots<5>(Q.rp, Q.ci, Q.ord, HubRows(), lb, sd, S, acc); break;
+        }
+        m &= ~__ballot(small);
+        __syncwarp();
+        while (m) {
+          const int l = __builtin_ctzll(m);
+          m &= m - 1;
+          const int64_t b0 = (int64_t)readlane_u64((uint64_t)lb, l);
+          const int d = __builtin_amdgcn_readlane(ld, l);
+          switch (Q.kind) {
+            case 3: batch_root<3>(Q.rp, Q.ci, Q.ord, b0, d, a.ratio, ar, s_wtot[wv], acc); break;
+            case 4: batch_root<4>(Q.rp, Q.ci, Q.ord, b0, d, a.ratio, ar, s_wtot[wv], acc); break;
+            case 5: batch_root<5>(Q.rp, Q.ci, Q.ord, b0, d, a.ratio, ar, s_wtot[wv], acc); break;
+            case 6: batch_root<6>(Q.rp, Q.ci, Q.ord, b0, d, a.ratio, ar, s_wtot[wv], acc); break;
+            case 7: batch_root<7>(Q.rp, Q.ci, Q.ord, b0, d, a.ratio, ar, s_wtot[wv], acc); break;
+          }
+        }
+      }
+    } else {
+      for (int64_t u = u0; u < u1; ++u) {
         const int64_t e = Q.base + u;
         const int32_t v0 = Q.src[e], v1 = Q.ci[e];
         int64_t v = 0;
@@ -144,6 +177,7 @@ __global__ void __launch_bounds__(64 * BWPB) batch_kernel(BatchArgs a) {
     }
     acc = wave_sum_u64(acc);
     if (ln == 0 && acc) atomicAdd((unsigned long long*)&a.counts[lo], (unsigned long long)acc);
+    }
   }
 }
 
@@ -256,7 +290,9 @@ static int plan_batch(jgpm_ctx_s* c, const jgpm_query* q, int n, std::vector<jk:
       b.nsum = g->d_nsum;
       b.base = g->sym_rp_h[rb];
       b.ntasks = g->sym_rp_h[re] - b.base;
-      b.chunk = p == 2 ? 64 * echunk : p == 3 ? 8 * echunk : echunk;
+      // (diamonds only read the triangle array: 2,048 edges a chunk at the
+      // default, all 96 graphs above 1.7 ms with 512 of them)
+      b.chunk = p == 2 ? 256 * echunk : p == 3 ? 8 * echunk : echunk;
       max_sym = std::max(max_sym, g->sym_mmin);
     }
   }
