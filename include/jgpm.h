@@ -170,14 +170,15 @@ typedef struct {
                                persistent kernel for block-per-hub launches: 64 (one-word
                                LDS rows) or 128 (two-word rows)                             */
   int32_t batch_root_chunk; /* roots per work item of a clique query                      */
-  int32_t batch_edge_chunk; /* directed edges per work item of a P1..P12 query (P2 and P3,
-                               whose per-edge work is O(1) after the intersection, use 8x) */
+  int32_t batch_edge_chunk; /* directed edges per work item of a P2..P12 query (P3, whose
+                               per-edge work is O(1) after the intersection, uses 8x, P2,
+                               which only reads the triangle array, 256x)                  */
   int32_t batch_blocks_per_cu; /* persistent batched grid = this * num_cu, capped by the
                                   kernel's occupancy                                       */
-  int32_t sym_heavy_min;    /* P5, P7, P9, P11, P12 (single-query launches): directed edges
-                               with more than this many common neighbours (up to 8192) run
-                               one block per edge, S in an LDS hash (default 32; 8192
-                               turns it off)                                               */
+  int32_t sym_heavy_min;    /* P5, P7, P9, P11, P12 (single queries over small root ranges;
+                               larger ones run over triangles): directed edges with more
+                               than this many common neighbours (up to 8192) run one block
+                               per edge, S in an LDS hash (default 32; 8192 turns it off)  */
 } jgpm_tuning;
 int  jgpm_get_tuning(jgpm_ctx_t ctx, jgpm_tuning* t);
 int  jgpm_set_tuning(jgpm_ctx_t ctx, const jgpm_tuning* t);

@@ -423,10 +423,8 @@ int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStr
   jgpm_ctx_s* c = exec_ctx(g);
   if (p == 1) return enqueue_p1(g, rb, re, slot, st);
   if (p == 2) {
-    // diamonds from the per-edge triangle array: the array's one pass of
-    // intersections (k_edge_tri) costs about what one P2 pass costs, and
-    // every later diamond or induced-motif query on the graph then only
-    // reads it (a few bytes per edge)
+    // diamonds from the per-edge triangle array, which every later diamond,
+    // P3 or induced-motif query on the graph then only reads
     int rc = ensure_sym_aux(g, true, false, st);
     if (rc) return rc;
     const int64_t e0 = g->sym_rp_h[rb], e1 = g->sym_rp_h[re];
