@@ -44,7 +44,7 @@
 // GB of list elements in 3.1 ms, 1.1 TB/s).  One wave per root with a 32 KB
 // table of its own held a CU to 4 waves, and roots above 16384 wedges counted
 // in global memory, twice: P1 on R-MAT 18 149 -> 3.1 ms, R-MAT 20 785 -> 17.5
-// ms, 3.8M-vertex Chung-Lu 178 -> 10 ms.  With an intersection per pair of the
+// ms, 3.8M-vertex Chung-Lu 178 -> 6.2 ms.  With an intersection per pair of the
 // nest: P4 on R-MAT 14 152 -> 1.1 ms, P6 on R-MAT 11 282 -> 0.59, P8 on R-MAT 12
 // 384 -> 0.88, P10 on R-MAT 10 173 -> 0.46.
 #include <hip/hip_runtime.h>
