@@ -120,10 +120,9 @@ int clique_hub_rows(jgpm_graph_s* g, int k, int64_t rb, int64_t re, hipStream_t 
 }
 
 // Lazily built per-graph arrays of the symmetric kernels.
-int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t st) {
+static int build_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t st) {
   jgpm_ctx_s* c = exec_ctx(g);
   const int64_t ne = g->sym.nnz;
-  if (!g->d_src || (need_tri && !g->d_tri) || (need_nsum && !g->d_nsum)) prof_stale(c);
   if (!g->d_src) {
     if (hipMalloc(&g->d_src, sizeof(int32_t) * std::max<int64_t>(ne, 1)) != hipSuccess) return JGPM_E_NOMEM;
     g->bytes += 4 * ne;
@@ -161,6 +160,23 @@ int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t s
       return JGPM_E_HIP;
   }
   return JGPM_OK;
+}
+
+// Makes sure of a graph's lazy arrays.  They are built on
+// the graph's own context: its stream orders the build before every later
+// reader there, and g->aux_built before the readers on other streams.  A
+// context that runs a query of another's graph (a serving lane) would publish
+// an array that its stream is still filling, so where one is missing it gets
+// JGPM_E_NOMEM and does without, like a query that found no room.
+int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t st) {
+  jgpm_ctx_s* c = exec_ctx(g);
+  if (g->d_src && (!need_tri || g->d_tri) && (!need_nsum || g->d_nsum)) return JGPM_OK;
+  if (c != g->ctx) return JGPM_E_NOMEM;
+  prof_stale(c);
+  if (!g->aux_built && hipEventCreateWithFlags(&g->aux_built, hipEventDisableTiming) != hipSuccess) return JGPM_E_HIP;
+  const int rc = build_sym_aux(g, need_tri, need_nsum, st);
+  const hipError_t e = hipEventRecord(g->aux_built, st);
+  return rc ? rc : e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
 }
 
 bool pattern_uses_tri(int p) { return p == 3 || p == 4 || p == 7 || p == 10 || p == 11; }
@@ -210,6 +226,7 @@ static int enqueue_tri_sum(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int s
 int ensure_tri_prefix(jgpm_graph_s* g, hipStream_t st) {
   if (!g->tri_pre_h.empty()) return JGPM_OK;
   jgpm_ctx_s* c = exec_ctx(g);
+  if (c != g->ctx) return JGPM_E_NOMEM;  // as in ensure_sym_aux
   if (c->capturing) return JGPM_E_STATE;
   int rc = ensure_sym_aux(g, true, false, st);
   if (rc) return rc;
@@ -372,7 +389,9 @@ static bool heavy_split_on(const jgpm_ctx_s* c, int p) {
   return jk::sym_heavy_pattern(p) && c->tune.sym_heavy_min < jk::sym_heavy_nmax();
 }
 
-bool query_needs_tri(const jgpm_ctx_s* c, int p) { return p == 2 || pattern_uses_tri(p) || heavy_split_on(c, p); }
+bool edge_route_needs_tri(const jgpm_ctx_s* c, int p) {
+  return p == 2 || pattern_uses_tri(p) || heavy_split_on(c, p);
+}
 
 int ensure_p1_scratch(jgpm_ctx_s* c, size_t bytes, hipStream_t st) {
   return grow(c, c->d_p1, c->p1_bytes, bytes, SIZE_MAX, st);
@@ -462,7 +481,7 @@ int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStr
     if (rr != JGPM_E_NOMEM) return rr;
     (void)hipGetLastError();
   }
-  int rc = ensure_sym_aux(g, query_needs_tri(c, p), false, st);
+  int rc = ensure_sym_aux(g, edge_route_needs_tri(c, p), false, st);
   if (rc) return rc;
   // the heavy-edge split needs its three edge lists, each as long as the
   // range's edge count up to 2^26 (grown per context, so not while a launch
@@ -619,9 +638,16 @@ int prepare_pattern(jgpm_graph_s* g, int pattern, int64_t rb, int64_t re) {
     jk::P1Q q;
     if (g->has_sym && re > rb) rc = p1_query(g, rb, re, c->st, q);
   } else if (pattern >= JGPM_P2 && pattern <= JGPM_P12) {
-    if (g->has_sym) rc = ensure_sym_aux(g, query_needs_tri(c, pattern), pattern == JGPM_P3, c->st);
-    if (g->has_sym && !rc && (pattern == JGPM_P6 || pattern == JGPM_P8 || pattern == JGPM_P10))
-      rc = ensure_tri_prefix(g, c->st);
+    // every one of them reads the triangle array on one of its routes; what
+    // there is no room for is left out where the per-edge launches do without
+    if (g->has_sym) {
+      rc = ensure_sym_aux(g, true, pattern == JGPM_P3, c->st);
+      if (!rc && (pattern == JGPM_P6 || pattern == JGPM_P8 || pattern == JGPM_P10)) rc = ensure_tri_prefix(g, c->st);
+      if (rc == JGPM_E_NOMEM && (g->d_tri || !edge_route_needs_tri(c, pattern))) {
+        (void)hipGetLastError();
+        rc = ensure_sym_aux(g, false, pattern == JGPM_P3, c->st);
+      }
+    }
   }
   if (hipStreamSynchronize(c->st) != hipSuccess && !rc) rc = JGPM_E_HIP;
   return rc;

@@ -94,6 +94,7 @@ struct jgpm_graph_s {
   int32_t hubs = 0;                            // vertices of at least HUB_MIN_DEG neighbours
   int64_t tri_rows = -1;                       // widest rows of the triangle sums beyond LDS, words (-1: not known yet)
   int64_t* d_nsum = nullptr;                   // neighbour-degree sums (lazy)
+  hipEvent_t aux_built = nullptr;              // after the last build of d_src, d_tri, d_dtri or d_nsum
   DevCSR rsym;                                 // symmetric CSR relabelled by d_ord (lazy, 4-cycle totals)
   int32_t* d_rsrc = nullptr;                   // ... and the source of each of its edges
   int32_t rank_min2 = 0;                       // vertices with at most one neighbour: the first ranks
@@ -164,8 +165,8 @@ int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t s
 int enqueue_batch_q(jgpm_ctx_s* c, const jgpm_query* q, int n, hipStream_t st);
 bool batch_supported(int pattern);
 bool pattern_uses_tri(int p);
-// whether a single-query launch of pattern p on context c reads the triangle array
-bool query_needs_tri(const jgpm_ctx_s* c, int p);
+// whether the per-edge launches of pattern p on context c read the triangle array
+bool edge_route_needs_tri(const jgpm_ctx_s* c, int p);
 // profile hooks around one kernel launch on the context stream
 // prof_reset: a new query, whose begin is marked by `open` (may be null);
 // prof_stale: work outside the spans was enqueued, or the host waited.

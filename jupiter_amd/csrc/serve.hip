@@ -136,7 +136,7 @@ static int64_t footprint(jgpm_graph_s* g, int p, const jgpm_ctx_s* c, int grid) 
   int64_t b = 64;  // count slot and queue counters
   if (!is_dag_pattern(p)) {
     if (!g->d_src) b += 4 * g->sym.nnz;
-    if (!g->d_tri && jgpm::query_needs_tri(c, p)) b += 4 * g->sym.nnz;
+    if (!g->d_tri && jgpm::edge_route_needs_tri(c, p)) b += 4 * g->sym.nnz;
     if (jk::sym_heavy_pattern(p))  // the heavy-edge lists of the context that runs it
       b += 12 * std::max<int64_t>(0, std::min<int64_t>(g->sym.nnz, (int64_t)1 << 26) - c->hcap);
     if (!g->d_nsum && p == JGPM_P3) b += 8 * (int64_t)g->sym.nv;
@@ -161,6 +161,8 @@ static int run_heavy(jgpm_ctx_s* main, jgpm_ctx_s* lc, const Req& r, uint64_t* c
     jgpm::ExecScope scope(lc);
     std::lock_guard<std::mutex> gl(main->mu);
     if (!st) st = jgpm::ctx_reset_counters(lc, lc->st);
+    // an array that a batch built since may still be under way on its stream
+    if (!st && r.g->aux_built && hipStreamWaitEvent(lc->st, r.g->aux_built, 0) != hipSuccess) st = JGPM_E_HIP;
     if (!st) {
       jgpm::prof_reset(lc, nullptr);
       st = jgpm::enqueue_pattern(r.g, r.pattern, r.rb, r.re, 0, lc->st);

@@ -119,3 +119,32 @@ def test_heavy_lanes_on_fresh_graphs(ctx):
             G.free()
     assert got[4] == alone
     assert got[1] == alone
+
+
+def test_lanes_read_finished_arrays_at_every_tuning(ctx):
+    """The triangle array that P5 to P12 read is built before a lane runs
+    them, also where sym_heavy_min turns the heavy-edge split off (the
+    per-edge launches of P5, P9 and P12 then do without it, their triangle
+    sums never do): lanes and batched diamonds on fresh graphs give their
+    counts alone."""
+    csrs = [J.rmat(14, 16, seed=s) for s in (21, 22)]
+    spec = [(i, p) for p in ("P5", "P2", "P9", "P12", "P6", "P8", "P2", "P10", "P4", "P7", "P11") for i in (0, 1)]
+    gs = [ctx.upload(c) for c in csrs]
+    alone = [gs[i].count(p)[0] for i, p in spec]
+    for G in gs:
+        G.free()
+    try:
+        ctx.set_tuning(sym_heavy_min=8192)
+        for first in range(0, 8, 2):  # the request that finds the graphs bare
+            order = spec[first:] + spec[:first]
+            want = alone[first:] + alone[:first]
+            gs = [ctx.upload(c) for c in csrs]
+            print(f"[case] sym_heavy_min 8192, {order[0][1]} first", flush=True)
+            with J.Server(ctx, heavy_lanes=4) as srv:
+                tickets = [srv.submit(gs[i], p) for i, p in order]
+                got = [srv.wait(t)[0] for t in tickets]
+            for G in gs:
+                G.free()
+            assert got == want
+    finally:
+        ctx.set_tuning(sym_heavy_min=-1)
