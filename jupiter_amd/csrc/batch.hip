@@ -134,9 +134,9 @@ __global__ void __launch_bounds__(64 * BWPB) __attribute__((amdgpu_waves_per_eu(
         const int sd = small ? ld : 0;
         SmallRoots& S = *reinterpret_cast<SmallRoots*>(ar);
         switch (Q.kind) {
-          case 3: small_roots<3>(Q.rp, Q.ci, Q.ord, HubRows(), lb, sd, S, acc); break;
-          case 4: small_roots<4>(Q.rp, Q.ci, Q.ord, HubRows(), lb, sd, S, acc); break;
-          case 5: small_roots<5>(Q.rp, Q.ci, Q.ord, HubRows(), lb, sd, S, acc); break;
+          case 3: small_roots<3, true>(Q.rp, Q.ci, Q.ord, HubRows(), a.ratio, lb, sd, S, acc); break;
+          case 4: small_roots<4, true>(Q.rp, Q.ci, Q.ord, HubRows(), a.ratio, lb, sd, S, acc); break;
+          case 5: small_roots<5, true>(Q.rp, Q.ci, Q.ord, HubRows(), a.ratio, lb, sd, S, acc); break;
         }
         m &= ~__ballot(small);
         __syncwarp();

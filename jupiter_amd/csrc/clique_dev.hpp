@@ -1159,8 +1159,15 @@ __device__ __forceinline__ void hub_test(const uint32_t* bits, uint32_t rw, uint
 // waits for a handful of dependent loads with most lanes idle (15 us a root in
 // flight); here a batch of some 30 roots does (Chung-Lu, 3M vertices: TC 2.6 ->
 // 0.8 ms, P13 2.1 -> 0.78; with roots of up to 16 members only 0.83 and 0.79).
+// FAR: a list that is long for its root is left out of the stream, and its
+// lane searches it for the root's members (a vertex early in an uploaded DAG's
+// order may point to millions and be a member of thousands of roots).  Asked
+// for where such vertices can be, as it costs registers: always, R-MAT 22 P13 +
+// P14 took 47.6 ms instead of 46.1, R-MAT 14 TC 116 us instead of 112.
 constexpr int SMALL_D = 32;
 constexpr int SMALL_E = 128;
+// longest list in the stream at any ratio: SMALL_E of them fit 31 bits
+constexpr int SMALL_STREAM = 1 << 23;
 struct SmallRoots {
   int64_t base[SMALL_E];      // of the edge's root list, then of u's own list: element f of the stream is ci[base + f]
   int32_t off[SMALL_E + 4];   // first element of u's list in the stream
@@ -1169,10 +1176,10 @@ struct SmallRoots {
   uint32_t row[SMALL_E];      // u's row over the root's members
   uint16_t at[SMALL_E];       // the root's first edge, and its members << 8
 };
-template <int K>
+template <int K, bool FAR>
 __device__ void small_roots(const int64_t* __restrict__ rp, const int32_t* __restrict__ ci,
-                            const int32_t* __restrict__ ord, const HubRows hub, int64_t b, int d, SmallRoots& S,
-                            uint64_t& acc) {
+                            const int32_t* __restrict__ ord, const HubRows hub, int ratio, int64_t b, int d,
+                            SmallRoots& S, uint64_t& acc) {
   const int ln = lane_id();
   uint64_t todo = __ballot(d > 0);
   while (todo) {
@@ -1198,7 +1205,7 @@ __device__ void small_roots(const int64_t* __restrict__ rp, const int32_t* __res
       u[i] = f < E ? ci[S.base[f] + f] : 0;
     }
     uint32_t p[2];
-    int len[2];
+    int len[2];  // below zero: of a list that is searched
     int64_t s[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -1213,14 +1220,16 @@ __device__ void small_roots(const int64_t* __restrict__ rp, const int32_t* __res
         if (p[i] == 0xffffffffu) {
           s[i] = rp[u[i]];
           len[i] = (int)(rp[u[i] + 1] - s[i]);
+          if (FAR && len[i] > 64 && len[i] > min(ratio * (S.at[64 * i + ln] >> 8), SMALL_STREAM)) len[i] = -len[i];
         }
       }
     }
-    const int in0 = wave_incl_scan(len[0]), T0 = __shfl(in0, 63);
-    const int in1 = wave_incl_scan(len[1]) + T0, T = __shfl(in1, 63);
+    auto streamed = [](int n) { return FAR ? max(n, 0) : n; };
+    const int in0 = wave_incl_scan(streamed(len[0])), T0 = __shfl(in0, 63);
+    const int in1 = wave_incl_scan(streamed(len[1])) + T0, T = __shfl(in1, 63);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const int f = 64 * i + ln, o = (i ? in1 : in0) - len[i];
+      const int f = 64 * i + ln, o = (i ? in1 : in0) - streamed(len[i]);
       S.L[f] = u[i];
       S.P[f] = p[i];
       S.row[f] = 0;
@@ -1249,6 +1258,22 @@ __device__ void small_roots(const int64_t* __restrict__ rp, const int32_t* __res
       }
       if constexpr (K == 3) acc += (uint64_t)__popc(r);
       else if (mine) S.row[f] = r;
+    }
+    // long lists
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if (!FAR || !__ballot(len[i] < 0)) continue;
+      const int f = 64 * i + ln;
+      const int st = S.at[f] & 255, dr = len[i] < 0 ? S.at[f] >> 8 : 0;
+      const int32_t* const l = ci + S.base[f] + S.off[f];
+      uint32_t r = 0;
+      for (int j = 0; j < dr; ++j) {
+        const int32_t y = S.L[st + j];
+        const int q = lower_bound_dev(l, -len[i], y);
+        if (q < -len[i] && l[q] == y) r |= 1u << j;
+      }
+      if constexpr (K == 3) acc += (uint64_t)__popc(r);
+      else if (len[i] < 0) S.row[f] = r;
     }
     if constexpr (K > 3) __syncwarp();
     // the others' lists

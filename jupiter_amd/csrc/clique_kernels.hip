@@ -117,7 +117,7 @@ constexpr int min_waves() {
   if (K == 7 && WMAX == 4) return 5;
   return 1;
 }
-template <int G, int WPB, int WMAX, int K, bool BYTES, bool LROWS>
+template <int G, int WPB, int WMAX, int K, bool BYTES, bool LROWS, bool FAR>
 __global__ void __launch_bounds__(64 * G * WPB) __attribute__((amdgpu_waves_per_eu(min_waves<WMAX, K, BYTES>())))
 clique_kernel(CliqueArgs a) {
   using LY = Lay<G, WMAX, K, BYTES, LROWS>;
@@ -161,7 +161,7 @@ clique_kernel(CliqueArgs a) {
       uint64_t m = __ballot(ld >= a.dmin && ld <= a.dmax && ld <= DM && ld >= 0);
       if constexpr (SMALL) {
         const bool small = ((m >> ln) & 1) && ld <= SMALL_D;
-        small_roots<K>(rp, a.ci, a.ord, hub, lb, small ? ld : 0, *reinterpret_cast<SmallRoots*>(ar), acc);
+        small_roots<K, FAR>(rp, a.ci, a.ord, hub, a.ratio, lb, small ? ld : 0, *reinterpret_cast<SmallRoots*>(ar), acc);
         m &= ~__ballot(small);
         __syncwarp();
       }
@@ -535,9 +535,9 @@ size_t glb_slot_words() { return GSLOT; }
 // 6- and 7-clique roots up to this out-degree run one wave each.
 constexpr int SMALL_ROOT = 24;
 
-template <int G, int WPB, int WMAX, int K, bool BYTES, bool LROWS>
+template <int G, int WPB, int WMAX, int K, bool BYTES, bool LROWS, bool FAR = false>
 static hipError_t launch_one(const CliqueArgs& a, int grid, hipStream_t st) {
-  hipLaunchKernelGGL((clique_kernel<G, WPB, WMAX, K, BYTES, LROWS>), dim3(grid), dim3(64 * G * WPB), 0, st, a);
+  hipLaunchKernelGGL((clique_kernel<G, WPB, WMAX, K, BYTES, LROWS, FAR>), dim3(grid), dim3(64 * G * WPB), 0, st, a);
   return hipGetLastError();
 }
 
@@ -549,6 +549,8 @@ static hipError_t launch_k(int tier, const CliqueArgs& a, int grid, hipStream_t 
       // (their subtrees would leave one wave running alone at the end)
       if constexpr (!BYTES && K >= 6)
         if (a.dmin > SMALL_ROOT) return launch_one<4, 1, 1, K, BYTES, true>(a, grid, st);
+      if constexpr (!BYTES && K < 6)
+        if (a.far) return launch_one<1, 4, 1, K, BYTES, true, true>(a, grid, st);
       return launch_one<1, 4, 1, K, BYTES, true>(a, grid, st);
     case TIER_LDS2:   return launch_one<4, 1, 2, K, BYTES, true>(a, grid, st);
     case TIER_LDS4:   return launch_one<4, 1, 4, K, BYTES, true>(a, grid, st);

@@ -219,6 +219,9 @@ static int graph_from_host(jgpm_ctx_s* c, const jgpm_csr_s* sym, const jgpm_csr_
       *out = g;
       return JGPM_OK;
     }
+    // (in the degree order only the last vertices, which get hub rows, have
+    // long lists; 256 is 8 times a small root's 32 members, the wave tier's ratio)
+    g->far = dag->max_deg > 256;
     std::vector<int32_t> ord((size_t)dag->nv);
     {
       std::vector<int32_t> indeg((size_t)dag->nv, 0), q;
@@ -540,6 +543,7 @@ int enqueue_clique(jgpm_graph_s* g, int k, bool bytes, int64_t rb, int64_t re, i
     a.rp = g->dag.rp;
     a.ci = g->dag.ci;
     a.ord = g->d_ord;
+    a.far = g->far;
     // roots up to 256 wide search all members of a long list in one pass of
     // their waves, so binary search pays earlier: from a quarter of the ratio
     // up to 128 wide, an eighth at 256 (R-MAT 22, one quarter of the roots:

@@ -91,6 +91,7 @@ struct jgpm_graph_s {
   int32_t* d_dtri = nullptr;                   // ... and per DAG edge (built with d_tri)
   std::vector<int64_t> tri_pre_h;              // prefix of d_tri over the vertices (P6, P8, P10; empty: not known yet)
   int64_t tri_max = 0;                         // ... and its largest vertex
+  bool far = false;                            // an uploaded DAG with long lists anywhere in its order
   int32_t hubs = 0;                            // vertices of at least HUB_MIN_DEG neighbours
   int64_t tri_rows = -1;                       // widest rows of the triangle sums beyond LDS, words (-1: not known yet)
   int64_t* d_nsum = nullptr;                   // neighbour-degree sums (lazy)

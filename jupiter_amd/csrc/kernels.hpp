@@ -36,6 +36,7 @@ struct CliqueArgs {
   const uint32_t* hub;   // hub rows (launch_hub_rows), of the hub_top last places of ord
   int32_t hub_top;       // 0: none
   int32_t nv;
+  int32_t far;           // some vertex may have a list that is long for a small root (small_roots)
 };
 
 // Out-neighbourhoods of the `top` last vertices of ord as bitmaps
