@@ -189,12 +189,16 @@ bool pattern_uses_tri(int p) { return p == 3 || p == 4 || p == 7 || p == 10 || p
 // triangles; P7 10.5 and 10.1; P9 0.85 and 8.8, P12 1.7 and 10.1).
 static int64_t tri_sum_share(int p) { return p == 5 || p == 7 ? 32 : 8; }
 
-static int enqueue_tri_sum(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStream_t st) {
+// given: arguments the caller has already (a second tri_args could move the
+// scratch that they point to).
+static int enqueue_tri_sum(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStream_t st,
+                           const jk::TriArgs* given = nullptr) {
   jgpm_ctx_s* c = exec_ctx(g);
   int rc = ensure_sym_aux(g, true, false, st);
   if (rc) return rc;
   jk::TriArgs a;
-  if ((rc = tri_args(g, st, a))) return rc;
+  if (given) a = *given;
+  else if ((rc = tri_args(g, st, a))) return rc;
   a.rb = rb;
   a.re = re;
   a.out = c->d_out + slot;
@@ -289,7 +293,7 @@ static int enqueue_ego(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot,
   if (!rc) rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(most_n, most_e), st);
   jk::TriArgs ta;
   if (!rc) rc = tri_args(g, st, ta);
-  if (!rc && p == 10) rc = enqueue_tri_sum(g, 10, rb, re, slot, st);
+  if (!rc && p == 10) rc = enqueue_tri_sum(g, 10, rb, re, slot, st, &ta);
   if (rc) return rc;  // (nothing is launched when there was no room)
   static const char* const kName[11] = {"", "", "", "", "", "", "sym_p6_wedge", "", "sym_p8_wedge", "", "sym_p10_wedge"};
   prof_begin(c, st, kName[p]);
