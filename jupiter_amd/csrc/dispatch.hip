@@ -194,6 +194,7 @@ static int64_t tri_sum_share(int p) { return p == 5 || p == 7 ? 32 : 8; }
 static int enqueue_tri_sum(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStream_t st,
                            const jk::TriArgs* given = nullptr) {
   jgpm_ctx_s* c = exec_ctx(g);
+  if (g->dag.max_deg > jk::TRI_MAX_OUT) return JGPM_E_NOMEM;  // per edge
   int rc = ensure_sym_aux(g, true, false, st);
   if (rc) return rc;
   jk::TriArgs a;

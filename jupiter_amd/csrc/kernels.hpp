@@ -199,6 +199,7 @@ struct TriArgs {
   int64_t rstride;
   uint64_t* out;
 };
+constexpr int TRI_MAX_OUT = 1 << 16;   // out-neighbours of a root: the sums' pair queues hold 16-bit positions
 constexpr int TRI_SMALL_PER_CU = 6;  // blocks per CU of the narrow block tier
 int64_t tri_row_words(int64_t d, int64_t dp);  // words of the rows of a root (degree d, out-degree dp)
 bool tri_rows_global(int64_t d, int64_t dp);   // ... which do not fit LDS
