@@ -181,13 +181,19 @@ int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t s
 
 bool pattern_uses_tri(int p) { return p == 3 || p == 4 || p == 7 || p == 10 || p == 11; }
 
-// P5, P7, P9, P11 and P12 over a root range that holds at least 1 / this of
-// the directed edges run as sums over all triangles, the terms of other roots
-// left out; smaller ranges run per edge.  P5 and P7 have work at every edge
-// of the range, the others only towards larger ids (R-MAT 18, the last
-// quarter of the ids with 1/17 of the edges: P5 16.7 ms per edge, 10.1 over
-// triangles; P7 10.5 and 10.1; P9 0.85 and 8.8, P12 1.7 and 10.1).
-static int64_t tri_sum_share(int p) { return p == 5 || p == 7 ? 32 : 8; }
+// Words of the widest root's rows among those that do not fit LDS (0: none):
+// a slice of the row scratch per block.
+static int64_t widest_rows(jgpm_graph_s* g) {
+  if (g->tri_rows < 0) {
+    g->tri_rows = 0;
+    if (jk::tri_rows_global(g->sym.max_deg, g->dag.max_deg))
+      for (int32_t v = 0; v < g->sym.nv; ++v) {
+        const int64_t d = g->sym_rp_h[v + 1] - g->sym_rp_h[v], dp = g->dag_rp_h[v + 1] - g->dag_rp_h[v];
+        if (jk::tri_rows_global(d, dp)) g->tri_rows = std::max(g->tri_rows, jk::tri_row_words(d, dp));
+      }
+  }
+  return g->tri_rows;
+}
 
 // given: arguments the caller has already (a second tri_args could move the
 // scratch that they point to).
@@ -203,17 +209,8 @@ static int enqueue_tri_sum(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int s
   a.rb = rb;
   a.re = re;
   a.out = c->d_out + slot;
-  // roots whose rows do not fit LDS: one slice of the row scratch per block
-  if (g->tri_rows < 0) {
-    g->tri_rows = 0;
-    if (jk::tri_rows_global(g->sym.max_deg, g->dag.max_deg))
-      for (int32_t v = 0; v < g->sym.nv; ++v) {
-        const int64_t d = g->sym_rp_h[v + 1] - g->sym_rp_h[v], dp = g->dag_rp_h[v + 1] - g->dag_rp_h[v];
-        if (jk::tri_rows_global(d, dp)) g->tri_rows = std::max(g->tri_rows, jk::tri_row_words(d, dp));
-      }
-  }
   int gblocks = 0;
-  if (g->tri_rows > 0) {
+  if (widest_rows(g) > 0) {
     a.rstride = g->tri_rows;
     gblocks = (int)std::max<int64_t>(1, std::min<int64_t>(c->num_cu, ((int64_t)1 << 27) / a.rstride));  // 1 GiB
     if ((rc = ensure_scratch(c, (size_t)a.rstride * (size_t)gblocks))) return rc;
@@ -228,6 +225,22 @@ static int enqueue_tri_sum(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int s
   return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
 }
 
+// An array of n entries that `launch` fills on the device, to the host (through
+// the triangle launches' scratch).
+template <class T, class F>
+static int device_array(jgpm_ctx_s* c, size_t n, hipStream_t st, std::vector<T>& h, F launch) {
+  const int rc = grow(c, c->d_te, c->te_bytes, sizeof(T) * std::max<size_t>(n, 1), SIZE_MAX, st);
+  if (rc) return rc;
+  try {
+    h.resize(n);
+  } catch (const std::bad_alloc&) {
+    return JGPM_E_NOMEM;
+  }
+  const bool ok = launch(static_cast<T*>(c->d_te)) == hipSuccess &&
+                  hipMemcpyAsync(h.data(), c->d_te, sizeof(T) * n, hipMemcpyDeviceToHost, st) == hipSuccess;
+  return hipStreamSynchronize(st) == hipSuccess && ok ? JGPM_OK : JGPM_E_HIP;
+}
+
 int ensure_tri_prefix(jgpm_graph_s* g, hipStream_t st) {
   if (!g->tri_pre_h.empty()) return JGPM_OK;
   jgpm_ctx_s* c = exec_ctx(g);
@@ -235,22 +248,115 @@ int ensure_tri_prefix(jgpm_graph_s* g, hipStream_t st) {
   if (c->capturing) return JGPM_E_STATE;
   int rc = ensure_sym_aux(g, true, false, st);
   if (rc) return rc;
+  prof_stale(c);
   const int32_t nv = g->sym.nv;
-  int64_t* d = nullptr;
-  if (hipMalloc(&d, sizeof(int64_t) * std::max(nv, 1)) != hipSuccess) return JGPM_E_NOMEM;
-  std::vector<int64_t> pre((size_t)nv + 1, 0);
-  bool ok = jk::launch_root_tri(g->sym.rp, g->d_tri, nv, d, c->num_cu, st) == hipSuccess &&
-            hipMemcpyAsync(pre.data() + 1, d, sizeof(int64_t) * (size_t)nv, hipMemcpyDeviceToHost, st) == hipSuccess;
-  ok = (hipStreamSynchronize(st) == hipSuccess) && ok;
-  (void)hipFree(d);
-  if (!ok) return JGPM_E_HIP;
-  int64_t most = 0;
-  for (int32_t v = 0; v < nv; ++v) {
-    most = std::max(most, pre[v + 1]);
-    pre[v + 1] += pre[v];
+  std::vector<int64_t> sum;
+  rc = device_array(c, (size_t)nv, st, sum,
+                    [&](int64_t* d) { return jk::launch_root_tri(g->sym.rp, g->d_tri, nv, d, c->num_cu, st); });
+  if (rc) return rc;
+  try {
+    sum.push_back(0);
+  } catch (const std::bad_alloc&) {
+    return JGPM_E_NOMEM;
+  }
+  int64_t most = 0, run = 0;
+  for (int32_t v = 0; v <= nv; ++v) {
+    const int64_t x = sum[v];
+    most = std::max(most, x);
+    sum[v] = run;
+    run += x;
   }
   g->tri_max = most;
-  g->tri_pre_h.swap(pre);
+  g->tri_pre_h.swap(sum);
+  return JGPM_OK;
+}
+
+int ensure_edge_work(jgpm_graph_s* g, hipStream_t st) {
+  if (!g->work_pre_h.empty()) return JGPM_OK;
+  jgpm_ctx_s* c = exec_ctx(g);
+  if (c != g->ctx) return JGPM_E_NOMEM;  // as in ensure_sym_aux
+  if (c->capturing) return JGPM_E_STATE;
+  int rc = ensure_sym_aux(g, true, false, st);
+  if (rc) return rc;
+  prof_stale(c);
+  const int32_t nv = g->sym.nv;
+  (void)widest_rows(g);  // while the device builds the triangle array
+  const int64_t nb = jk::edge_work_blocks(nv);
+  std::vector<float4> work;
+  jk::TriArgs a{};
+  a.rp = g->sym.rp;
+  a.ci = g->sym.ci;
+  a.drp = g->dag.rp;
+  a.nv = nv;
+  rc = device_array(c, (size_t)nb, st, work,
+                    [&](float4* d) { return jk::launch_edge_work(a, g->d_src, g->d_tri, d, st); });
+  if (rc) return rc;
+  std::vector<jgpm_graph_s::EdgeWork> pre;
+  try {
+    pre.resize((size_t)nb + 1);
+  } catch (const std::bad_alloc&) {
+    return JGPM_E_NOMEM;
+  }
+  double pass = 0;
+  pre[0] = {0, 0, 0};
+  for (int64_t k = 0; k < nb; ++k) {
+    pre[k + 1] = {pre[k].lo_a + work[k].x, pre[k].lo_b + work[k].y, pre[k].hi_b + work[k].z};
+    pass += work[k].w;
+  }
+  // measured: R-MAT 12 / 14 / 16 / 18: P9 0.13 / 0.32 / 1.27 / 6.5 ms, P5 - / 0.38 / 1.57 / 7.8; Barabasi-Albert
+  // (60,000 vertices, 12 a vertex) 0.30, 0.32; Erdos-Renyi (32,768, degree 40) 0.34, 0.34; Chung-Lu (200,000) 0.49, 0.53
+  g->tri_pass_a = 100e3 + 0.8 * nv + 0.08 * (double)g->sym.nnz + pass;
+  g->tri_pass_b = 150e3 + 1.1 * nv + 1.25 * pass;
+  g->work_pre_h.swap(pre);
+  return JGPM_OK;
+}
+
+// Whether P4, P5, P7, P9, P11 or P12 over a root range runs over all triangles
+// of the graph (the terms of other roots left out) or per edge of the range.
+// The pass takes the same time whatever the range; the per-edge launches take
+// 1.45 ns for each edge of the range and, for the edges that the pattern
+// credits to the range (P9, P11, P12 to the smaller end, P5 and P4 to the
+// larger, P7 to both) and that lie in t > 0 triangles, what k_edge_work adds
+// up: R-MAT ids fall with the degree, so the last eighth of the edges of R-MAT 18 takes P9
+// 1.6 ms per edge (6.5 over triangles), the first eighth 64.  P4 per edge waits
+// for one intersection after the other at an edge to a hub, about 3 us each.
+// Over ranges of 1/2 to 1/2048 of the edges at both ends and in the middle, on
+// those graphs, the route taken was at most 1.2 times slower than per edge,
+// and than the better one 2 times (a range of R-MAT 12's first roots 2.8: 0.35
+// and 0.13 ms).  A share of the edges as the line (1/8 for P9, P11, P12, 1/32 for P5,
+// P7, 1/1024 for P4) was up to 4.7, 3.9 and 16 times slower than per edge.
+static int over_triangles(jgpm_graph_s* g, int p, int64_t rb, int64_t re, hipStream_t st, bool& yes) {
+  const int64_t ne = g->sym_rp_h[re] - g->sym_rp_h[rb];
+  yes = ne == g->sym.nnz;
+  if (yes) return JGPM_OK;
+  // not worth the triangle array if nothing has built it yet
+  if (!g->d_tri && !edge_route_needs_tri(exec_ctx(g), p) && ne < g->sym.nnz / 64) return JGPM_OK;
+  const int rc = ensure_edge_work(g, st);
+  if (rc) return rc;
+  // the prefix at a vertex: of its block's work the share of its edges
+  const int64_t *rp = g->sym_rp_h.data(), nv = g->sym.nv, B = jk::EDGE_WORK_BLOCK;
+  auto at = [&](int64_t v) {
+    const int64_t k = std::min(v / B, (int64_t)g->work_pre_h.size() - 2);
+    const int64_t e0 = rp[k * B], e1 = rp[std::min(nv, (k + 1) * B)];
+    const double f = e1 > e0 ? (double)(rp[v] - e0) / (double)(e1 - e0) : 0.0;
+    const jgpm_graph_s::EdgeWork &x = g->work_pre_h[k], &y = g->work_pre_h[k + 1];
+    return jgpm_graph_s::EdgeWork{x.lo_a + f * (y.lo_a - x.lo_a), x.lo_b + f * (y.lo_b - x.lo_b),
+                                  x.hi_b + f * (y.hi_b - x.hi_b)};
+  };
+  const jgpm_graph_s::EdgeWork x = at(rb), y = at(re);
+  const double lo_a = y.lo_a - x.lo_a, lo_b = y.lo_b - x.lo_b;
+  const double hi_b = re > 1 ? y.hi_b - x.hi_b : 0;  // (vertex 0 has no smaller neighbour)
+  const double base = 120e3 + 1.45 * (double)ne;
+  switch (p) {
+    case 4:
+      yes = 75e3 + (hi_b > 0 ? 3e3 * g->sym.max_deg : 0.0) + 1.7 * (double)ne > g->tri_pass_b + 100e3;
+      break;
+    case 5: yes = base + hi_b > g->tri_pass_b; break;
+    case 7: yes = base + lo_b + hi_b > g->tri_pass_b; break;
+    case 9: yes = base + lo_a > g->tri_pass_a; break;
+    case 11: yes = base + lo_a > g->tri_pass_b; break;
+    case 12: yes = base + lo_b > g->tri_pass_b; break;
+  }
   return JGPM_OK;
 }
 
@@ -344,13 +450,6 @@ static int enqueue_ego(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot,
   }
   prof_end(c, st);
   return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
-}
-
-// P4 over a root range that is not a sliver of the graph (the triangle part
-// of a partial range covers all triangles): wedges from every root of the
-// range.
-static bool p4_route(const jgpm_graph_s* g, int64_t rb, int64_t re) {
-  return g->sym_rp_h[re] - g->sym_rp_h[rb] >= g->sym.nnz / 1024;
 }
 
 static int enqueue_p4(jgpm_graph_s* g, int64_t rb, int64_t re, int slot, hipStream_t st) {
@@ -472,13 +571,12 @@ int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStr
   }
   // patterns that run over triangles or wedges of the whole range; where
   // there is no room for their scratch (nothing launched), per edge
-  const int64_t ne_q = g->sym_rp_h[re] - g->sym_rp_h[rb];
-  if (ne_q > 0) {
+  if (g->sym_rp_h[re] > g->sym_rp_h[rb]) {
     int rr = JGPM_E_NOMEM;
-    if (jk::sym_heavy_pattern(p) && ne_q >= g->sym.nnz / tri_sum_share(p)) {
-      rr = enqueue_tri_sum(g, p, rb, re, slot, st);
-    } else if (p == 4 && p4_route(g, rb, re)) {
-      rr = enqueue_p4(g, rb, re, slot, st);
+    if (p == 4 || jk::sym_heavy_pattern(p)) {
+      bool yes = false;
+      rr = over_triangles(g, p, rb, re, st, yes);
+      if (!rr) rr = !yes ? JGPM_E_NOMEM : p == 4 ? enqueue_p4(g, rb, re, slot, st) : enqueue_tri_sum(g, p, rb, re, slot, st);
     } else if (p == 6 || p == 8 || p == 10) {
       rr = ensure_tri_prefix(g, st);
       if (!rr) rr = ego_route(g, p, rb, re) ? enqueue_ego(g, p, rb, re, slot, st) : JGPM_E_NOMEM;
@@ -648,6 +746,8 @@ int prepare_pattern(jgpm_graph_s* g, int pattern, int64_t rb, int64_t re) {
     if (g->has_sym) {
       rc = ensure_sym_aux(g, true, pattern == JGPM_P3, c->st);
       if (!rc && (pattern == JGPM_P6 || pattern == JGPM_P8 || pattern == JGPM_P10)) rc = ensure_tri_prefix(g, c->st);
+      if (!rc && (pattern == JGPM_P4 || jk::sym_heavy_pattern(pattern)) && (rb > 0 || re < g->sym.nv))
+        rc = ensure_edge_work(g, c->st);
       if (rc == JGPM_E_NOMEM && (g->d_tri || !edge_route_needs_tri(c, pattern))) {
         (void)hipGetLastError();
         rc = ensure_sym_aux(g, false, pattern == JGPM_P3, c->st);

@@ -92,6 +92,13 @@ struct jgpm_graph_s {
   std::vector<int64_t> tri_pre_h;              // prefix of d_tri over the vertices (P6, P8, P10; empty: not known yet)
   int64_t tri_max = 0;                         // ... and its largest vertex
   bool far = false;                            // an uploaded DAG with long lists anywhere in its order
+  // partial root ranges of P4, P5, P7, P9, P11, P12 (ensure_edge_work; empty: not known yet): prefix over
+  // blocks of vertices of what the per-edge launches spend, and what a pass over all triangles takes, in ns
+  struct EdgeWork {
+    double lo_a, lo_b, hi_b;
+  };
+  std::vector<EdgeWork> work_pre_h;
+  double tri_pass_a = 0, tri_pass_b = 0;
   int32_t hubs = 0;                            // vertices of at least HUB_MIN_DEG neighbours
   int64_t tri_rows = -1;                       // widest rows of the triangle sums beyond LDS, words (-1: not known yet)
   int64_t* d_nsum = nullptr;                   // neighbour-degree sums (lazy)
@@ -159,6 +166,8 @@ int build_tiers(jgpm_graph_s* g, const int64_t* rp, int32_t nv);
 int set_degree_order(jgpm_graph_s* g, const std::vector<int64_t>& sym_rp, int32_t max_deg);
 // g->tri_pre_h (waits for the stream once per graph).
 int ensure_tri_prefix(jgpm_graph_s* g, hipStream_t st);
+// g->work_pre_h (likewise).
+int ensure_edge_work(jgpm_graph_s* g, hipStream_t st);
 int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t st);
 // Batched persistent launch over queries the kernel supports (TC, P1..P16);
 // counts land in c->d_bcnt[0..n).  hq / cs are host staging that must stay

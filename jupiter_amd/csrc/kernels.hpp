@@ -235,6 +235,11 @@ hipError_t launch_edge_base(const int64_t* rp, const int32_t* ci, const int32_t*
 hipError_t launch_edge_sum(bool p3, const int64_t* rp, const int32_t* ci, const int32_t* src, const int32_t* tri,
                            const int64_t* nsum, int64_t e0, int64_t e1, unsigned long long* flag, uint64_t* out,
                            int num_cu, hipStream_t st);
+// what the edges of every EDGE_WORK_BLOCK vertices cost the per-edge launches of P4 to P12, and the triangle sums
+// (a.rp, ci, drp and nv)
+constexpr int EDGE_WORK_BLOCK = 16;
+__host__ __device__ inline int64_t edge_work_blocks(int64_t nv) { return (nv + EDGE_WORK_BLOCK - 1) / EDGE_WORK_BLOCK; }
+hipError_t launch_edge_work(const TriArgs& a, const int32_t* src, const int32_t* tri, float4* work, hipStream_t st);
 hipError_t launch_root_tri(const int64_t* rp, const int32_t* tri, int32_t nv, int64_t* sum, int num_cu, hipStream_t st);
 
 int sym_waves_per_block();

@@ -778,6 +778,61 @@ __global__ void __launch_bounds__(256) k_root_tri(const int64_t* rp, const int32
   }
 }
 
+// What the edges of EDGE_WORK_BLOCK vertices cost the per-edge launches where
+// they have triangles (ns): x and y over the edges to larger ids, z over those
+// to smaller ones; w what the vertices' rows and triangles cost the triangle
+// sums.  A block each: the first vertices of an R-MAT graph are its hubs.
+__global__ void __launch_bounds__(512) k_edge_work(TriArgs a, const int32_t* src, const int32_t* tri, float4* work) {
+  __shared__ float4 s_part[8];
+  const int64_t v = (int64_t)blockIdx.x * EDGE_WORK_BLOCK, ve = min((int64_t)a.nv, v + EDGE_WORK_BLOCK), end = a.rp[ve];
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (v + threadIdx.x < ve) {
+    const int64_t u = v + threadIdx.x;
+    s.w = 0.0035f * (float)(a.rp[u + 1] - a.rp[u]) * (float)(a.drp[u + 1] - a.drp[u]);
+  }
+  for (int64_t e0 = a.rp[v] + threadIdx.x; e0 < end; e0 += 2048) {
+    int32_t te[4];
+    bool up[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t e = min(e0 + 512 * k, end - 1);
+      te[k] = e0 + 512 * k < end ? tri[e] : 0;
+      up[k] = a.ci[e] > src[e];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float t = (float)te[k];
+      if (t == 0.f) continue;
+      const float b = 8.f + 0.6f * t + 0.00045f * t * t;
+      if (up[k]) {
+        s.x += 5.f + 0.001f * t * t;
+        s.y += b;
+      } else {
+        s.z += b;
+        s.w += 0.0087f * t;
+      }
+    }
+  }
+#pragma unroll
+  for (int o = 32; o; o >>= 1) {
+    s.x += __shfl_xor(s.x, o);
+    s.y += __shfl_xor(s.y, o);
+    s.z += __shfl_xor(s.z, o);
+    s.w += __shfl_xor(s.w, o);
+  }
+  if (lane() == 0) s_part[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < 8; ++k) {
+      s.x += s_part[k].x;
+      s.y += s_part[k].y;
+      s.z += s_part[k].z;
+      s.w += s_part[k].w;
+    }
+    work[blockIdx.x] = s;
+  }
+}
+
 // grid of a kernel with a wave per item, 4 waves per block
 unsigned item_grid(int64_t items, int num_cu) {
   const int64_t blocks = (items + 3) / 4;
@@ -867,6 +922,12 @@ hipError_t launch_edge_sum(bool p3, const int64_t* rp, const int32_t* ci, const 
 
 hipError_t launch_root_tri(const int64_t* rp, const int32_t* tri, int32_t nv, int64_t* sum, int num_cu, hipStream_t st) {
   hipLaunchKernelGGL(k_root_tri, dim3(item_grid(nv, num_cu)), dim3(256), 0, st, rp, tri, nv, sum);
+  return hipGetLastError();
+}
+
+hipError_t launch_edge_work(const TriArgs& a, const int32_t* src, const int32_t* tri, float4* work, hipStream_t st) {
+  if (a.nv > 0)
+    hipLaunchKernelGGL(k_edge_work, dim3((unsigned)edge_work_blocks(a.nv)), dim3(512), 0, st, a, src, tri, work);
   return hipGetLastError();
 }
 
