@@ -397,7 +397,7 @@ int enqueue_batch(jgpm_ctx_s* c, const jgpm_query* q, int n, std::vector<jk::BQ>
   jk::P1Args pa;
   rc = plan_batch(c, q, n, hq, cs, max_sym, pa, st);
   if (rc) return rc;
-  if (pa.nq && (rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(pa.roots, pa.edges), st))) return rc;
+  if (pa.nq && (rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(pa.roots, pa.edges), SIZE_MAX, st))) return rc;
   const int grid = batch_grid(c);
   const size_t need = (size_t)grid * jk::BWPB * jk::symd::NLIST * (size_t)max_sym;
   if (c->sscr_ints < need) {

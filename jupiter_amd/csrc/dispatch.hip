@@ -20,12 +20,34 @@ jgpm_ctx_s* exec_ctx(const jgpm_graph_s* g) { return t_exec ? t_exec : g->ctx; }
 ExecScope::ExecScope(jgpm_ctx_s* c) : prev(t_exec) { t_exec = c; }
 ExecScope::~ExecScope() { t_exec = prev; }
 
+size_t ws_held(const jgpm_ctx_s* c) {
+  return c->hub_bytes + c->ego_bytes + c->te_bytes + c->p1_bytes + sizeof(uint64_t) * c->scr_words +
+         sizeof(int32_t) * (c->sscr_ints + 3 * (size_t)c->hcap);
+}
+
+void ws_release(jgpm_ctx_s* c) {
+  void* p[] = {c->d_hub, c->d_ego, c->d_te, c->d_p1, c->d_scr, c->d_sscr, c->d_hlist};
+  for (void* x : p)
+    if (x) (void)hipFree(x);
+  c->d_hub = c->d_ego = c->d_te = c->d_p1 = nullptr;
+  c->d_scr = nullptr;
+  c->d_sscr = c->d_hlist = nullptr;
+  c->hub_bytes = c->ego_bytes = c->te_bytes = c->p1_bytes = c->scr_words = c->sscr_ints = 0;
+  c->hcap = 0;
+}
+
+// Bytes a workspace that holds `have` may take under the context's cap.
+static size_t ws_room(const jgpm_ctx_s* c, size_t have) {
+  const size_t others = ws_held(c) - have;
+  return c->ws_cap > others ? c->ws_cap - others : 0;
+}
+
 // Grows one of the context's scratch buffers to `need` bytes (allocates, never
-// while capturing); its contents are lost.  More than `cap` bytes are
-// JGPM_E_NOMEM, as where the device has no room.
+// while capturing); its contents are lost.  More than `cap` bytes in all the
+// workspaces together are JGPM_E_NOMEM, as where the device has no room.
 static int grow(jgpm_ctx_s* c, void*& p, size_t& have, size_t need, size_t cap, hipStream_t st) {
   if (have >= need) return JGPM_OK;
-  if (need > cap) return JGPM_E_NOMEM;
+  if (cap != SIZE_MAX && ws_held(c) - have + need > cap) return JGPM_E_NOMEM;
   prof_stale(c);
   if (c->capturing) return JGPM_E_STATE;
   if (p) {
@@ -50,9 +72,24 @@ static int64_t tri_hub_bytes(int64_t nnz) {
   return std::max<int64_t>((int64_t)128 << 20, std::min<int64_t>((int64_t)512 << 20, 16 * nnz));
 }
 
+// Scratch of the triangle launches: the hub bitmaps, the task lists, and what
+// the sums keep of a block's root.
+static int64_t tri_hwords(int64_t nv) { return ((nv + 31) / 32 + 3) & ~(int64_t)3; }
+static int32_t tri_hubs(const jgpm_graph_s* g) {
+  return (int32_t)std::min<int64_t>(g->hubs, tri_hub_bytes(g->sym.nnz) / (4 * tri_hwords(g->sym.nv)));
+}
+static size_t tri_list_bytes(const jgpm_graph_s* g) {
+  return (sizeof(int32_t) * 3 * (size_t)g->sym.nv + 15) & ~(size_t)15;
+}
+static size_t tri_root_bytes(const jgpm_graph_s* g, const jgpm_ctx_s* c) {
+  return g->sym.max_deg <= 64 ? 0 : sizeof(int32_t) * 3 * (size_t)std::max(1, g->dag.max_deg) *
+                                        (size_t)(jk::TRI_SMALL_PER_CU * c->num_cu);
+}
+
 // Arguments of the triangle launches on g, their scratch on the executing
-// context (the hub bitmaps still to be made by launch_hub_bitmaps).
-static int tri_args(jgpm_graph_s* g, hipStream_t st, jk::TriArgs& a) {
+// context (the hub bitmaps still to be made by launch_hub_bitmaps).  build:
+// only for the triangle array.
+static int tri_args(jgpm_graph_s* g, hipStream_t st, jk::TriArgs& a, bool build = false) {
   jgpm_ctx_s* c = exec_ctx(g);
   const int32_t nv = g->sym.nv;
   a = jk::TriArgs{};
@@ -67,17 +104,17 @@ static int tri_args(jgpm_graph_s* g, hipStream_t st, jk::TriArgs& a) {
   // a wave works its vertices off one after another: no more per wave than
   // it takes to fill the device (32 waves per CU)
   a.vchunk = std::max(1, std::min(64, nv / (64 * c->num_cu)));
-  a.hwords = (((int64_t)nv + 31) / 32 + 3) & ~(int64_t)3;
-  a.nhub = (int32_t)std::min<int64_t>(g->hubs, tri_hub_bytes(g->sym.nnz) / (4 * a.hwords));
+  a.hwords = tri_hwords(nv);
+  a.nhub = tri_hubs(g);
   a.lstride = std::max(1, g->dag.max_deg);
   size_t hub_b = 4 * (size_t)a.hwords * (size_t)a.nhub;
-  const size_t list_b = (sizeof(int32_t) * 3 * (size_t)nv + 15) & ~(size_t)15;
-  const size_t lscr_b = a.wide ? sizeof(int32_t) * 3 * (size_t)a.lstride * (size_t)(jk::TRI_SMALL_PER_CU * c->num_cu) : 0;
+  const size_t list_b = tri_list_bytes(g), lscr_b = tri_root_bytes(g, c);
   int rc = grow(c, c->d_te, c->te_bytes, 64 + hub_b + list_b + lscr_b, c->ws_cap, st);
   if (rc == JGPM_E_NOMEM) {  // without bitmaps: every row searched for
     a.nhub = 0;
     hub_b = 0;
-    rc = grow(c, c->d_te, c->te_bytes, 64 + list_b + lscr_b, SIZE_MAX, st);
+    rc = grow(c, c->d_te, c->te_bytes, 64 + list_b + lscr_b, c->ws_cap, st);
+    if (rc == JGPM_E_NOMEM && build) rc = grow(c, c->d_te, c->te_bytes, 64 + list_b, c->ws_cap, st);
   }
   if (rc) return rc;
   unsigned char* b = static_cast<unsigned char*>(c->d_te);
@@ -131,7 +168,7 @@ static int build_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStre
   if (need_tri && !g->d_tri) {
     const int64_t nd = g->dag.nnz;
     jk::TriArgs a;
-    int rc = tri_args(g, st, a);
+    int rc = tri_args(g, st, a, true);
     if (rc) return rc;
     int32_t *tri = nullptr, *dtri = nullptr;
     if (hipMalloc(&tri, sizeof(int32_t) * std::max<int64_t>(ne, 1)) != hipSuccess ||
@@ -212,7 +249,9 @@ static int enqueue_tri_sum(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int s
   int gblocks = 0;
   if (widest_rows(g) > 0) {
     a.rstride = g->tri_rows;
-    gblocks = (int)std::max<int64_t>(1, std::min<int64_t>(c->num_cu, ((int64_t)1 << 27) / a.rstride));  // 1 GiB
+    const int64_t room = (int64_t)(ws_room(c, sizeof(uint64_t) * c->scr_words) / sizeof(uint64_t)) / a.rstride;
+    if (room < 1) return JGPM_E_NOMEM;
+    gblocks = (int)std::min(room, std::max<int64_t>(1, std::min<int64_t>(c->num_cu, ((int64_t)1 << 27) / a.rstride)));  // 1 GiB
     if ((rc = ensure_scratch(c, (size_t)a.rstride * (size_t)gblocks))) return rc;
     a.rows = c->d_scr;
   }
@@ -364,6 +403,9 @@ static int over_triangles(jgpm_graph_s* g, int p, int64_t rb, int64_t re, hipStr
 // has a vertex per directed edge of the roots and 2 t entries per edge.  It is
 // built per query, for as many roots at a time as EGO_CAP entries hold.
 constexpr int64_t EGO_CAP = (int64_t)1 << 28;
+// Workspace bytes for an entry and an edge: 28 and 4 of the wedge launches, 8
+// and 8 of the graph, and some to spare.
+constexpr size_t EGO_ENTRY_BYTES = 64;
 
 // Whether the range runs on the induced neighbourhoods: every root fits the
 // cap, for P10, whose triangle part covers all triangles, the range is not a
@@ -383,7 +425,11 @@ static int enqueue_ego(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot,
   uint64_t* const out = c->d_out + slot;
   const int64_t *rp = g->sym_rp_h.data(), *pre = g->tri_pre_h.data();
   // chunks of whole roots, and the scratch of the largest
-  const int64_t cap = std::min<int64_t>(EGO_CAP, (int64_t)(c->ws_cap / 32));
+  const size_t tri_b = std::max(c->te_bytes, 64 + tri_list_bytes(g) + tri_root_bytes(g, c)) +
+                       (p == 10 ? sizeof(uint64_t) * (size_t)widest_rows(g) : 0);
+  const size_t room = ws_room(c, c->te_bytes + c->ego_bytes + c->p1_bytes);
+  const int64_t cap = std::min<int64_t>(EGO_CAP, (int64_t)((room > tri_b ? room - tri_b : 0) / EGO_ENTRY_BYTES));
+  if (cap < 1) return JGPM_E_NOMEM;
   std::vector<int64_t> cut{rb};
   int64_t most_e = 0, most_n = 0;
   for (int64_t r = rb; r < re;) {
@@ -397,7 +443,7 @@ static int enqueue_ego(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot,
   const size_t rp_b = sizeof(int64_t) * (size_t)(most_n + 1), tiles_b = sizeof(int64_t) * (size_t)jk::ego_tiles(most_n);
   const size_t ent_b = sizeof(int32_t) * (size_t)most_e;
   int rc = grow(c, c->d_ego, c->ego_bytes, rp_b + tiles_b + 2 * ent_b + 64, c->ws_cap, st);
-  if (!rc) rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(most_n, most_e), st);
+  if (!rc) rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(most_n, most_e), c->ws_cap, st);
   jk::TriArgs ta;
   if (!rc) rc = tri_args(g, st, ta);
   if (!rc && p == 10) rc = enqueue_tri_sum(g, 10, rb, re, slot, st, &ta);
@@ -475,7 +521,7 @@ static int enqueue_p4(jgpm_graph_s* g, int64_t rb, int64_t re, int slot, hipStre
   a.roots = a.one.nr;
   a.edges = a.one.ne;
   a.out = c->d_out;
-  if ((rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(a.roots, a.edges), st))) return rc;
+  if ((rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(a.roots, a.edges), c->ws_cap, st))) return rc;
   if (!whole && (rc = enqueue_tri_sum(g, 4, rb, re, slot, st))) return rc;  // (nothing is launched when there was no room)
   jk::p1_bind_scratch(a, c->d_p1);
   prof_begin(c, st, "sym_p4_wedge");
@@ -497,8 +543,8 @@ bool edge_route_needs_tri(const jgpm_ctx_s* c, int p) {
   return p == 2 || pattern_uses_tri(p) || heavy_split_on(c, p);
 }
 
-int ensure_p1_scratch(jgpm_ctx_s* c, size_t bytes, hipStream_t st) {
-  return grow(c, c->d_p1, c->p1_bytes, bytes, SIZE_MAX, st);
+int ensure_p1_scratch(jgpm_ctx_s* c, size_t bytes, size_t cap, hipStream_t st) {
+  return grow(c, c->d_p1, c->p1_bytes, bytes, cap, st);
 }
 
 int p1_query(jgpm_graph_s* g, int64_t rb, int64_t re, hipStream_t st, jk::P1Q& q) {
@@ -533,7 +579,7 @@ static int enqueue_p1(jgpm_graph_s* g, int64_t rb, int64_t re, int slot, hipStre
   a.roots = a.one.nr;
   a.edges = a.one.ne;
   a.out = c->d_out;
-  if ((rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(a.roots, a.edges), st))) return rc;
+  if ((rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(a.roots, a.edges), SIZE_MAX, st))) return rc;
   jk::p1_bind_scratch(a, c->d_p1);
   prof_begin(c, st, "sym_p1_wedge");
   hipError_t e = jk::launch_p1(a, c->num_cu, st);
@@ -586,6 +632,10 @@ int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStr
   }
   int rc = ensure_sym_aux(g, edge_route_needs_tri(c, p), false, st);
   if (rc) return rc;
+  const int wpb = jk::sym_waves_per_block();
+  const int grid = grid_for(c, 2);
+  const size_t stride = (size_t)std::max(1, g->sym_mmin);
+  const size_t need = (size_t)grid * wpb * jk::sym_lists_per_wave() * stride;
   // the heavy-edge split needs its three edge lists, each as long as the
   // range's edge count up to 2^26 (grown per context, so not while a launch
   // sequence is being captured; edges beyond a full list run in the
@@ -593,6 +643,14 @@ int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStr
   const int64_t ne_r = g->sym_rp_h[re] - g->sym_rp_h[rb];
   bool heavy = heavy_split_on(c, p) && ne_r < INT32_MAX;
   const int64_t hwant = std::min<int64_t>(std::max<int64_t>(ne_r, 1), (int64_t)1 << 26);
+  // a capped context gives back what another route took before it found no room
+  if (c->ws_cap != SIZE_MAX) {
+    const size_t want = sizeof(int32_t) * (std::max(need, c->sscr_ints) + (heavy ? 3 * (size_t)std::max(hwant, c->hcap) : 0));
+    if (ws_held(c) - sizeof(int32_t) * (c->sscr_ints + 3 * (size_t)c->hcap) + want > c->ws_cap) {
+      if (hipStreamSynchronize(st) != hipSuccess) return JGPM_E_HIP;
+      ws_release(c);
+    }
+  }
   if (heavy && c->hcap < hwant) {
     if (c->capturing) {
       heavy = c->d_hlist != nullptr;  // the lists it has
@@ -608,10 +666,6 @@ int enqueue_sym(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot, hipStr
       if (!c->d_hctr && hipMalloc(&c->d_hctr, sizeof(unsigned long long) * 6) != hipSuccess) return JGPM_E_NOMEM;
     }
   }
-  const int wpb = jk::sym_waves_per_block();
-  const int grid = grid_for(c, 2);
-  const size_t stride = (size_t)std::max(1, g->sym_mmin);
-  const size_t need = (size_t)grid * wpb * jk::sym_lists_per_wave() * stride;
   if (c->sscr_ints < need) {
     if (c->d_sscr) {
       if (hipStreamSynchronize(st) != hipSuccess) return JGPM_E_HIP;
@@ -726,6 +780,53 @@ int enqueue_pattern(jgpm_graph_s* g, int pattern, int64_t rb, int64_t re, int s,
       return enqueue_clique(g, 4, false, rb, re, s + 3, st);
   }
   return JGPM_E_PATTERN;
+}
+
+int64_t query_array_bytes(const jgpm_graph_s* g, const jgpm_ctx_s* c, int p, int64_t rb, int64_t re) {
+  if (clique_k(p)) return 0;
+  const int64_t nv = g->sym.nv, nnz = g->sym.nnz;
+  int64_t b = g->d_src ? 0 : 4 * nnz;
+  // P1: the relabelled graph, and the two key arrays that it is sorted in
+  if (p == JGPM_P1) return rb == 0 && re == nv && !g->rsym.ci ? b + 24 * nv + 24 * nnz : b;
+  if (!g->d_tri) b += 4 * nnz + 4 * g->dag.nnz + (int64_t)(64 + tri_list_bytes(g) + tri_root_bytes(g, c)) +
+                      4 * tri_hwords(nv) * tri_hubs(g);
+  if (p == JGPM_P3 && !g->d_nsum) b += 8 * nv;
+  return b;
+}
+
+int64_t query_ws_bytes(const jgpm_graph_s* g, const jgpm_ctx_s* c, int p, int64_t rb, int64_t re, int64_t most) {
+  if (const int k = clique_k(p)) {
+    // row scratch of the widest tiers: slices of the fused 2048-wide kernel,
+    // for 5- to 7-cliques the row slots of the split one (<= 1 GiB); those of
+    // the split 1024-wide one.  The tiers use one buffer after the other.
+    int64_t b = 0;
+    if (g->dag.max_deg > jk::tier_max_deg(jk::TIER_LDS16)) {
+      const int64_t fused = (int64_t)4 * c->num_cu * (int64_t)jk::tier_scratch_words(jk::TIER_GLB32) * 8;
+      b = k >= 5 ? std::max<int64_t>(fused, (int64_t)1 << 30) : fused;
+    }
+    if (k >= 4)
+      b = std::max<int64_t>(b, std::min<int64_t>((int64_t)1 << 30,
+                                                 8 * (int64_t)jk::split_slot_words() * (int64_t)g->tier_h[jk::TIER_LDS16].size()));
+    return b;
+  }
+  const bool whole = rb == 0 && re == g->sym.nv;
+  const int64_t ne = g->sym_rp_h[re] - g->sym_rp_h[rb];
+  const int64_t wedge = (int64_t)jk::p1_scratch_bytes(re - rb, ne);
+  if (p == JGPM_P1) return wedge;
+  if (p == JGPM_P2 || p == JGPM_P3) return 0;
+  const int64_t tri = (int64_t)(64 + tri_list_bytes(g) + tri_root_bytes(g, c));
+  const int64_t rows = jk::tri_rows_global(g->sym.max_deg, g->dag.max_deg)
+                           ? 8 * jk::tri_row_words(g->sym.max_deg, g->dag.max_deg) : 0;
+  // per edge: list scratch of every wave, and the heavy-edge lists
+  int64_t edge = (int64_t)grid_for(const_cast<jgpm_ctx_s*>(c), 2) * jk::sym_waves_per_block() *
+                 jk::sym_lists_per_wave() * std::max(1, g->sym_mmin) * 4;
+  if (jk::sym_heavy_pattern(p)) edge += 12 * std::min<int64_t>(ne, (int64_t)1 << 26);
+  int64_t b = p == JGPM_P4 ? wedge + (whole ? 0 : tri + rows)
+              : jk::sym_heavy_pattern(p) ? tri + rows
+                                         : tri + (p == JGPM_P10 ? rows : 0) + ((int64_t)EGO_ENTRY_BYTES << 18);
+  if (b > most) return edge;
+  // (a part of a graph, and one with few triangles, may run per edge)
+  return whole && p != JGPM_P6 && p != JGPM_P8 && p != JGPM_P10 ? b : std::max(b, edge);
 }
 
 int prepare_pattern(jgpm_graph_s* g, int pattern, int64_t rb, int64_t re) {

@@ -582,9 +582,10 @@ int enqueue_clique(jgpm_graph_s* g, int k, bool bytes, int64_t rb, int64_t re, i
         // chunks of roots bound the slots to 1 GiB.  Without room for them
         // the roots run fused, like 4- and 5-cliques.
         const size_t slot = jk::rows_slot_words(tier);
-        const size_t words = std::min<size_t>((size_t)1 << 27, c->ws_cap / sizeof(uint64_t));
-        const int64_t cap = std::min<int64_t>(n, std::max<int64_t>(1, (int64_t)(words / slot)));
-        int s2 = ensure_scratch(c, slot * (size_t)cap);
+        const size_t room = c->ws_cap / sizeof(uint64_t), others = ws_held(c) / sizeof(uint64_t) - c->scr_words;
+        const size_t words = std::min<size_t>((size_t)1 << 27, room > others ? room - others : 0);
+        const int64_t cap = std::min<int64_t>(n, (int64_t)(words / slot));
+        int s2 = cap < 1 ? JGPM_E_NOMEM : ensure_scratch(c, slot * (size_t)cap);
         if (s2 && s2 != JGPM_E_NOMEM) return s2;
         for (int64_t b = 0; !s2 && b < n; b += cap) {
           jk::CliqueArgs s = a;

@@ -41,7 +41,7 @@ struct jgpm_ctx_s {
   int32_t* d_hlist = nullptr;  // heavy-edge lists of P5/P7/P9/P11/P12 (3 x hcap ints)
   int64_t hcap = 0;
   unsigned long long* d_hctr = nullptr;  // their append and pop counters (6)
-  size_t ws_cap = SIZE_MAX;    // bytes any one of the workspaces may take that a query can also do without
+  size_t ws_cap = SIZE_MAX;    // bytes all workspaces together may take where a query can also do without (ws_held)
   void* d_hub = nullptr;       // hub rows of the clique engine
   size_t hub_bytes = 0;
   void* d_ego = nullptr;       // the graph of induced neighbourhoods of P6, P8, P10
@@ -145,7 +145,18 @@ int noalloc_setup(int dev, uint64_t** out);
 // relabelling; allocates, never while capturing) and describes it.
 int p1_query(jgpm_graph_s* g, int64_t rb, int64_t re, hipStream_t st, jk::P1Q& q);
 // Grows the context's 4-cycle scratch (allocates, never while capturing).
-int ensure_p1_scratch(jgpm_ctx_s* c, size_t bytes, hipStream_t st);
+// `cap`: bytes the context's workspaces may reach by it, else JGPM_E_NOMEM.
+int ensure_p1_scratch(jgpm_ctx_s* c, size_t bytes, size_t cap, hipStream_t st);
+// Bytes of the context's workspaces that queries grow; ws_release frees them
+// (nothing may be running on the context).
+size_t ws_held(const jgpm_ctx_s* c);
+void ws_release(jgpm_ctx_s* c);
+// Bytes that a query run whole on a context of its own needs beyond the
+// resident graph: the graph's arrays still to be built (with what building
+// them takes), and the workspaces that its route cannot do without, of the
+// per-edge route where the other's exceed `most`.
+int64_t query_array_bytes(const jgpm_graph_s* g, const jgpm_ctx_s* c, int p, int64_t rb, int64_t re);
+int64_t query_ws_bytes(const jgpm_graph_s* g, const jgpm_ctx_s* c, int p, int64_t rb, int64_t re, int64_t most);
 // g->rsym: vertex v becomes d_ord[v] (degree order), lists re-sorted, and its
 // edge sources.  Built once per graph (allocates; never while capturing).
 int ensure_rank_csr(jgpm_graph_s* g, hipStream_t st);

@@ -4,9 +4,9 @@
 // A scheduler thread owns the context's stream while the server runs:
 //  * admission: a submitted request is admitted when the number of requests
 //    on the device is below max_inflight and the HBM its intermediates need
-//    (per-graph auxiliary arrays it would create plus its share of the list
-//    scratch) fits the budget; a request that could never fit is rejected
-//    at submit with JGPM_E_BUDGET;
+//    (per-graph auxiliary arrays it would create, and the workspaces that its
+//    launches cannot do without) fits the budget beside that of the others; a
+//    request that could never fit is rejected at submit with JGPM_E_BUDGET;
 //  * slicing: every admitted request is cut into root slices of bounded work
 //    (edges of the slice times a per-pattern cost weight), so expensive
 //    queries cannot hold the device for long;
@@ -55,7 +55,8 @@ struct Req {
   int pattern;
   int64_t rb, re, cur;
   uint64_t count = 0;
-  int64_t footprint = 0;
+  int64_t ws = 0;           // bytes of workspaces its launches cannot do without (heavy)
+  int64_t footprint = 0;    // ... and of the graph's arrays it creates: what admission counts
   bool heavy = false;       // runs whole, with the single-query kernels (not sliced into batches)
   bool dispatched = false;  // a heavy request handed to a lane
   int status = JGPM_OK;
@@ -68,12 +69,18 @@ struct HeavyDone {
   int status;
 };
 
-// One heavy request at a time, on a context of its own.
+// One heavy request at a time, on a context of its own.  Its workspaces may
+// take the request's `ws` bytes and `extra` more for what launches can do
+// without (hub rows and bitmaps, larger chunks); what they hold afterwards is
+// counted against the budget until it is given back.
 struct Lane {
   jgpm_ctx_s* ctx = nullptr;
   std::thread th;
-  bool busy = false;  // guarded by the server's mutex, as is job
+  bool busy = false;  // guarded by the server's mutex, as is all that follows
   Req job;
+  int64_t extra = 0;  // while busy
+  int64_t held = 0;   // while idle
+  bool trim = false;  // to give its workspaces back before the next job
 };
 
 struct Done {
@@ -131,8 +138,8 @@ struct jgpm_serve_s {
   bool lanes_stop = false;
 };
 
-// HBM the request's intermediates need beyond the resident graph.
-static int64_t footprint(jgpm_graph_s* g, int p, const jgpm_ctx_s* c, int grid) {
+// HBM below which no budget serves the request at all.
+static int64_t least_footprint(jgpm_graph_s* g, int p, const jgpm_ctx_s* c, int grid) {
   int64_t b = 64;  // count slot and queue counters
   if (!is_dag_pattern(p)) {
     if (!g->d_src) b += 4 * g->sym.nnz;
@@ -147,8 +154,25 @@ static int64_t footprint(jgpm_graph_s* g, int p, const jgpm_ctx_s* c, int grid) 
     const int64_t fused = (int64_t)4 * c->num_cu * (int64_t)jk::tier_scratch_words(jk::TIER_GLB32) * 8;
     b += jgpm::clique_k(p) >= 5 ? std::max<int64_t>(fused, (int64_t)1 << 30) : fused;
   }
-  (void)c;
   return b;
+}
+
+// Bytes of workspaces beside the admitted requests' footprints: what busy
+// lanes may take on top, and what idle ones hold.
+static int64_t lane_extra(const jgpm_serve_s* s) {
+  int64_t b = 0;
+  for (const Lane* L : s->lanes) b += L->busy ? L->extra : 0;
+  return b;
+}
+static int64_t idle_held(const jgpm_serve_s* s) {
+  int64_t b = 0;
+  for (const Lane* L : s->lanes) b += L->busy ? 0 : L->held;
+  return b;
+}
+// Whether the oldest waiting request may start (idle lanes can be emptied).
+static bool fits(const jgpm_serve_s* s) {
+  return s->active.empty() ||
+         s->inflight_bytes + lane_extra(s) + s->pending.front().footprint <= s->cfg.hbm_budget_bytes;
 }
 
 // Runs a heavy request whole on lane context lc; the graph's lazy arrays are
@@ -179,17 +203,21 @@ static int run_heavy(jgpm_ctx_s* main, jgpm_ctx_s* lc, const Req& r, uint64_t* c
 static void lane_loop(jgpm_serve_s* s, Lane* L) {
   for (;;) {
     Req r;
+    bool trim;
     {
       std::unique_lock<std::mutex> lk(s->mu);
       s->cv_lane.wait(lk, [&] { return s->lanes_stop || L->busy; });
       if (!L->busy) return;
       r = L->job;
+      trim = L->trim;
     }
+    if (trim && hipSetDevice(L->ctx->dev) == hipSuccess) jgpm::ws_release(L->ctx);
     uint64_t count = 0;
     const int st = run_heavy(s->ctx, L->ctx, r, &count);
     {
       std::lock_guard<std::mutex> lk(s->mu);
       L->busy = false;
+      L->held = (int64_t)jgpm::ws_held(L->ctx);
       s->heavy_done.push_back(HeavyDone{r.ticket, count, st});
     }
     s->cv_work.notify_all();
@@ -209,15 +237,14 @@ static void serve_loop(jgpm_serve_s* s) {
   std::vector<uint64_t> h;
   for (;;) {
     std::vector<size_t> to_lane;  // heavy requests to hand to lanes, oldest first
+    std::vector<Lane*> to_empty;  // idle lanes whose workspaces make room (only this thread gives them work)
     {
       std::unique_lock<std::mutex> lk(s->mu);
       // work: an admissible arrival, lane results, light slices, or a heavy
       // request and a free lane
       auto has_work = [&] {
         if (!s->heavy_done.empty()) return true;
-        if (!s->pending.empty() && (int)s->active.size() < s->cfg.max_inflight &&
-            (s->active.empty() || s->inflight_bytes + s->pending.front().footprint <= s->cfg.hbm_budget_bytes))
-          return true;
+        if (!s->pending.empty() && (int)s->active.size() < s->cfg.max_inflight && fits(s)) return true;
         for (const Req& r : s->active) {
           if (r.cur >= r.re) continue;
           if (!r.heavy || (!r.dispatched && free_lane(s))) return true;
@@ -228,12 +255,18 @@ static void serve_loop(jgpm_serve_s* s) {
       if (s->stop && s->active.empty() && s->pending.empty()) return;
       // admission in arrival order
       while (!s->pending.empty() && (int)s->active.size() < s->cfg.max_inflight) {
+        if (!fits(s)) break;
         Req& r = s->pending.front();
-        if (!s->active.empty() && s->inflight_bytes + r.footprint > s->cfg.hbm_budget_bytes) break;
         s->inflight_bytes += r.footprint;
         s->active.push_back(r);
         s->pending.pop_front();
       }
+      if (s->inflight_bytes + lane_extra(s) + idle_held(s) > s->cfg.hbm_budget_bytes)
+        for (Lane* L : s->lanes)
+          if (!L->busy && L->held > 0) {
+            to_empty.push_back(L);
+            L->held = 0;
+          }
       // results of the lanes
       for (const HeavyDone& d : s->heavy_done)
         for (Req& r : s->active)
@@ -250,6 +283,8 @@ static void serve_loop(jgpm_serve_s* s) {
         if (r.heavy && !r.dispatched && r.cur < r.re) to_lane.push_back(i);
       }
     }
+    if (!to_empty.empty() && hipSetDevice(c->dev) == hipSuccess)
+      for (Lane* L : to_empty) jgpm::ws_release(L->ctx);
     // heavy requests to free lanes (the active list is only touched by this thread)
     for (size_t i : to_lane) {
       Req& r = s->active[i];
@@ -262,6 +297,10 @@ static void serve_loop(jgpm_serve_s* s) {
         continue;
       }
       Lane* L = free_lane(s);  // lanes only turn free meanwhile, so one is
+      const int64_t spare = s->cfg.hbm_budget_bytes - s->inflight_bytes - lane_extra(s) - (idle_held(s) - L->held);
+      L->extra = std::max<int64_t>(0, std::min(spare, s->cfg.hbm_budget_bytes / s->cfg.heavy_lanes));
+      L->trim = L->held > L->extra;
+      L->ctx->ws_cap = (size_t)(r.ws + L->extra);
       L->job = r;
       L->busy = true;
       s->cv_lane.notify_all();
@@ -360,8 +399,6 @@ extern "C" int jgpm_serve_start(jgpm_ctx_t ctx, const jgpm_serve_config* cfg, jg
     }
     L->ctx->tune = ctx->tune;
     L->ctx->prof_on = false;  // nobody can ask a lane's context for its profile
-    // workspaces beyond the footprints that admission counts share the budget
-    L->ctx->ws_cap = (size_t)(s->cfg.hbm_budget_bytes / s->cfg.heavy_lanes);
     s->lanes.push_back(L);
     L->th = std::thread(lane_loop, s, L);
   }
@@ -395,17 +432,24 @@ extern "C" int jgpm_serve_submit(jgpm_serve_t s, jgpm_graph_t g, int pattern, in
   r.rb = rb;
   r.re = re;
   r.cur = rb;
-  r.footprint = footprint(g, pattern, s->ctx, grid);
+  const int64_t least = least_footprint(g, pattern, s->ctx, grid);
   {
     const std::vector<int64_t>& rp = is_dag_pattern(pattern) ? g->dag_rp_h : g->sym_rp_h;
     r.heavy = wide || (double)(rp[re] - rp[rb]) * pattern_weight(pattern) > (double)s->slice_edges ||
               rp[re] - rp[rb] > single_edges(pattern);
   }
+  if (r.heavy) {
+    r.ws = jgpm::query_ws_bytes(g, s->ctx, pattern, rb, re, s->cfg.hbm_budget_bytes);
+    r.footprint = jgpm::query_array_bytes(g, s->ctx, pattern, rb, re) + r.ws;
+  } else {  // in batches: the list scratch of their kernel, or the 4-cycle launches' own
+    r.footprint = std::max(least, jgpm::query_array_bytes(g, s->ctx, pattern, rb, re) +
+                                      (pattern == JGPM_P1 ? jgpm::query_ws_bytes(g, s->ctx, pattern, rb, re, 0) : 0));
+  }
   r.t_submit = clk::now();
   std::lock_guard<std::mutex> lk(s->mu);
   if (s->stop) return JGPM_E_STATE;
   if (s->fatal) return s->fatal;
-  if (r.footprint > s->cfg.hbm_budget_bytes) return JGPM_E_BUDGET;
+  if (least > s->cfg.hbm_budget_bytes) return JGPM_E_BUDGET;
   r.ticket = s->next_ticket++;
   *ticket = r.ticket;
   s->live.insert(r.ticket);

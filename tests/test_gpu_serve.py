@@ -1,6 +1,7 @@
 """Serving loop: concurrently submitted queries of different patterns and
 graphs give the same uint64 count as alone (tolerance 0); admission by the
 HBM budget rejects what cannot fit."""
+import ctypes
 import threading
 
 import numpy as np
@@ -148,3 +149,42 @@ def test_lanes_read_finished_arrays_at_every_tuning(ctx):
             assert got == want
     finally:
         ctx.set_tuning(sym_heavy_min=-1)
+
+
+@pytest.mark.parametrize("lanes", [16, 3])
+def test_device_memory_stays_within_the_budget(ctx, lanes):
+    """What a server takes beyond the resident graphs, the arrays it builds on them included, stays within
+    hbm_budget_bytes with every lane at work: rows beyond LDS (35 MB a lane on K_1000 if it may), clique slots,
+    hub bitmaps, wedge scratch.  32 MiB over it are allowed for the runtime's own scratch and rounding."""
+    hip = ctypes.CDLL([ln.split()[-1] for ln in open("/proc/self/maps") if "libamdhip64" in ln][0])
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    src, dst = np.triu_indices(1000, 1)
+    csrs = [J.CSR.from_edges(1000, src, dst), J.rmat(12, 16, seed=32)]
+    spec = [(i, p) for p in ("P5", "P1", "P7", "P9", "P13", "P12", "P11", "TC", "P2", "P3", "P5", "P9") for i in (0, 1)]
+    spec += [(1, p) for p in ("P4", "P15", "P6", "P8", "P10")]
+    gs = [ctx.upload(c) for c in csrs]
+    alone = {(i, p): gs[i].count(p)[0] for i, p in spec}
+    with J.Server(ctx, heavy_lanes=lanes) as srv:  # the runtime's scratch of every queue
+        for t in [srv.submit(gs[i], p) for i, p in spec]:
+            srv.wait(t)
+    for G in gs:
+        G.free()
+    gs = [ctx.upload(c) for c in csrs]
+    budget = 96 << 20
+    with J.Server(ctx, heavy_lanes=lanes, hbm_budget_bytes=budget) as srv:
+        free0 = least = free_bytes()
+        tickets = [srv.submit(gs[i], p) for i, p in spec]
+        got = []
+        for t in tickets:
+            got.append(srv.wait(t)[0])
+            least = min(least, free_bytes())
+    for G in gs:
+        G.free()
+    assert got == [alone[x] for x in spec]
+    print(f"[case] {lanes} lanes: {(free0 - least) >> 20} MiB of {budget >> 20}", flush=True)
+    assert free0 - least <= budget + (32 << 20)
