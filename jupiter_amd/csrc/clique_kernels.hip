@@ -127,7 +127,7 @@ clique_kernel(CliqueArgs a) {
   constexpr size_t ARENA = SMALL && sizeof(SmallRoots) > LY::SLOT ? sizeof(SmallRoots) : LY::SLOT;
   __shared__ __attribute__((aligned(16))) unsigned char s_arena[WPB][ARENA];
   __shared__ int32_t s_wtot[G + 1];
-  __shared__ int64_t s_task;
+  __shared__ uint32_t s_task;
   const int slot = (G == 1) ? (int)(threadIdx.x >> 6) : 0;
   unsigned char* ar = s_arena[slot];
   uint64_t* rowp = LROWS ? reinterpret_cast<uint64_t*>(ar + LY::R_OFF)
@@ -193,10 +193,9 @@ clique_kernel(CliqueArgs a) {
                                                __builtin_amdgcn_readlane(ld, l), a.ratio, ar, rowp, s_wtot, acc,
                                                nullptr, hub);
       }
-      // (64 bits: near 2^31 roots the sum passes 31)
-      if (threadIdx.x == 0) s_task = (int64_t)gridDim.x * a.chunk + atomicAdd(a.qctr, (uint32_t)a.chunk);
+      if (threadIdx.x == 0) s_task = atomicAdd(a.qctr, (uint32_t)a.chunk);
       __syncthreads();
-      base = s_task;
+      base = (int64_t)gridDim.x * a.chunk + s_task;  // (near 2^31 roots it passes 31 bits)
       __syncthreads();
     }
   } else {
@@ -205,7 +204,7 @@ clique_kernel(CliqueArgs a) {
     for (bool first = true;; first = false) {
       int32_t task = (int32_t)blockIdx.x;  // (ids of roots wider than a wave's: far below 2^31 of them)
       if (!first) {
-        if (threadIdx.x == 0) s_task = (int64_t)gridDim.x + atomicAdd(a.qctr, 1u);
+        if (threadIdx.x == 0) s_task = gridDim.x + atomicAdd(a.qctr, 1u);
         __syncthreads();
         task = (int32_t)s_task;
         __syncthreads();
