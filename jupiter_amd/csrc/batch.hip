@@ -110,7 +110,7 @@ __global__ void __launch_bounds__(64 * BWPB) __attribute__((amdgpu_waves_per_eu(
     int64_t u1 = min(Q.ntasks, (kq - a.cstart[lo]) * Q.chunk);
     k = kq;
     uint64_t acc = 0;
-    if (Q.kind == 102 && Q.tri) {
+    if (Q.kind == 102) {
       // diamonds from the per-edge triangle array: lanes over the edges
       for (int64_t u = u0 + ln; u < u1; u += 64) {
         const int64_t e = Q.base + u;
@@ -160,7 +160,6 @@ __global__ void __launch_bounds__(64 * BWPB) __attribute__((amdgpu_waves_per_eu(
         const int32_t v0 = Q.src[e], v1 = Q.ci[e];
         int64_t v = 0;
         switch (Q.kind - 100) {
-          case 2: v = batch_edge<2>(Q, w, v0, v1, lds_lists, glist, a.scr_stride); break;
           case 3: v = batch_edge<3>(Q, w, v0, v1, lds_lists, glist, a.scr_stride); break;
           case 4: v = batch_edge<4>(Q, w, v0, v1, lds_lists, glist, a.scr_stride); break;
           case 5: v = batch_edge<5>(Q, w, v0, v1, lds_lists, glist, a.scr_stride); break;
@@ -276,7 +275,6 @@ static int plan_batch(jgpm_ctx_s* c, const jgpm_query* q, int n, std::vector<jk:
       w.roff = pa.roots;
       pa.edges += w.ne;
       pa.roots += w.nr;
-      pa.max_nv = std::max(pa.max_nv, g->sym.nv);
       p1.push_back(w);
     } else {
       const int p = kind - 100;
@@ -349,7 +347,7 @@ static int launch_batch(jgpm_ctx_s* c, const jgpm_query* q, int n, const std::ve
   // every 4-cycle query in one sequence of wedge launches
   if (pa.nq > 0) {
     prof_begin(c, st, "batch_p1_wedge");
-    hipError_t e = jk::launch_p1(pa, c->num_cu, st);
+    hipError_t e = jk::launch_wedge(jk::WEDGE_P1, pa, c->num_cu, st);
     prof_end(c, st);
     if (e != hipSuccess) return JGPM_E_HIP;
   }

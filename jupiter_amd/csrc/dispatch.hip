@@ -483,7 +483,6 @@ static int enqueue_ego(jgpm_graph_s* g, int p, int64_t rb, int64_t re, int slot,
     }
     if (p == 10) a.one.scale = -4;
     a.nq = 1;
-    a.max_nv = (int32_t)ea.n;
     a.tiles = (ents + 255) / 256;
     a.roots = ea.n;
     a.edges = ents;
@@ -516,7 +515,6 @@ static int enqueue_p4(jgpm_graph_s* g, int64_t rb, int64_t re, int slot, hipStre
   a.one.weight = g->d_tri;
   a.one.xend = g->sym.nv;
   a.nq = 1;
-  a.max_nv = g->sym.nv;
   a.tiles = (a.one.ne + 255) / 256;
   a.roots = a.one.nr;
   a.edges = a.one.ne;
@@ -574,7 +572,6 @@ static int enqueue_p1(jgpm_graph_s* g, int64_t rb, int64_t re, int slot, hipStre
   if (rc) return rc;
   a.one.slot = slot;
   a.nq = 1;
-  a.max_nv = g->sym.nv;
   a.tiles = (a.one.ne + 255) / 256;
   a.roots = a.one.nr;
   a.edges = a.one.ne;
@@ -582,7 +579,7 @@ static int enqueue_p1(jgpm_graph_s* g, int64_t rb, int64_t re, int slot, hipStre
   if ((rc = ensure_p1_scratch(c, jk::p1_scratch_bytes(a.roots, a.edges), SIZE_MAX, st))) return rc;
   jk::p1_bind_scratch(a, c->d_p1);
   prof_begin(c, st, "sym_p1_wedge");
-  hipError_t e = jk::launch_p1(a, c->num_cu, st);
+  hipError_t e = jk::launch_wedge(jk::WEDGE_P1, a, c->num_cu, st);
   prof_end(c, st);
   return e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
 }

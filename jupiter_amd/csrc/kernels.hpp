@@ -145,7 +145,6 @@ struct P1Args {
   P1Q one;               // the query, when q is null
   const P1Q* q;          // device table of nq queries
   int nq;
-  int32_t max_nv;        // largest vertex count of the queries
   const int64_t* tcs;    // prefix of the queries' 256-edge tiles (nq + 1)
   const int64_t* rcs;    // prefix of the queries' roots (nq + 1)
   int64_t tiles, roots, edges;  // totals
@@ -159,8 +158,7 @@ struct P1Args {
 };
 size_t p1_scratch_bytes(int64_t roots, int64_t edges);
 void p1_bind_scratch(P1Args& a, void* p);  // a.roots and a.edges set
-hipError_t launch_p1(const P1Args& a, int num_cu, hipStream_t st);
-hipError_t launch_wedge(int mode, const P1Args& a, int num_cu, hipStream_t st);  // one query
+hipError_t launch_wedge(int mode, const P1Args& a, int num_cu, hipStream_t st);  // P4, P6: one query
 
 // One wave per root vertex v_0 of [rb, re) on the symmetric CSR.
 struct PlanArgs {

@@ -244,11 +244,8 @@ __device__ int64_t edge_value(const Ctx& g, Wave& w, int32_t v0, int32_t v1, int
   int32_t* T = L[3];
   int32_t* pT = L[4];
   const int ln = lane();
-  static_assert(P >= 2 && P <= 12, "P1 runs as wedge counting (wedge.hip)");
-  if constexpr (P == 2) {
-    if (v1 >= v0) return 0;
-    return C2(w_icount(w, N0, d0, N1, d1, INT32_MAX));
-  } else if constexpr (P == 3) {
+  static_assert(P >= 3 && P <= 12, "P1 runs as wedge counting (wedge.hip), P2 from the triangle array");
+  if constexpr (P == 3) {
     const int n = w_imat(w, N0, d0, N1, d1, INT32_MAX, S, p0, nullptr);
     int64_t sp = 0, sd = 0, st = 0;
     for (int k = ln; k < n; k += 64) {

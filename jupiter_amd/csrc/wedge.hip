@@ -578,8 +578,6 @@ static hipError_t launch_wedge_m(const P1Args& a, int num_cu, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_p1(const P1Args& a, int num_cu, hipStream_t st) { return launch_wedge_m<W_P1>(a, num_cu, st); }
-
 hipError_t launch_wedge(int mode, const P1Args& a, int num_cu, hipStream_t st) {
   switch (mode) {
     case WEDGE_P1: return launch_wedge_m<W_P1>(a, num_cu, st);
