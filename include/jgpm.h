@@ -175,8 +175,8 @@ typedef struct {
                                which only reads the triangle array, 256x)                  */
   int32_t batch_blocks_per_cu; /* persistent batched grid = this * num_cu, capped by the
                                   kernel's occupancy                                       */
-  int32_t sym_heavy_min;    /* P5, P7, P9, P11, P12 (single queries over small root ranges;
-                               larger ones run over triangles): directed edges with more
+  int32_t sym_heavy_min;    /* P5, P7, P9, P11, P12 (single queries over root ranges that take less
+                               time per edge than over triangles): directed edges with more
                                than this many common neighbours (up to 8192) run one block
                                per edge, S in an LDS hash (default 32; 8192 turns it off)  */
 } jgpm_tuning;

@@ -5,9 +5,10 @@
 // and the delegation producer/extend pairs of src/delegation_gpu_kernels.cuh.
 // Single queries over large ranges run elsewhere: P1, P4, P6, P8 and P10 as wedge
 // counts (wedge.hip), P5, P7, P9, P11 and P12 as sums over triangles, P3 as a sum
-// over edges (tri_engine.hip).  What is here runs their small root ranges,
-// graphs too small to pay for those launches, and calls without room for their
-// scratch; the device routines also run batches.
+// over edges (tri_engine.hip).  What is here runs the root ranges that take
+// less time per edge (over_triangles), graphs too small to pay for those
+// launches, and calls without room for their scratch; the device routines also
+// run batches.
 // One wave owns one directed edge (v0, v1) of the root range, exactly the
 // edge loop of the reference (eid over the local COO list, :22 etc.), and adds
 // that edge's contribution to the count, so any root range gives the same

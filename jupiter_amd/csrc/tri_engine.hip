@@ -25,12 +25,14 @@
 // tri_hub_bytes), and a binary search in the short list of any other x.  So a
 // directed edge costs d(a) / 64 such steps, a being its end of less degree.
 //
-// What bounds it: the latency of the M and bitmap loads (L2), several in
-// flight per wave.  Per edge, with q(v2) counted by streaming N(v2) or by
-// binary searches, the same counts cost R-MAT 18: P5 296 -> 10.1 ms, P7 349 ->
-// 10.1, P9 121 -> 8.8, P11 163 -> 10.0, P12 350 -> 10.1; R-MAT 16 P5 28 -> 2.1;
-// the triangle array (one intersection per edge by binary searches before)
-// R-MAT 18 20.2 -> 7.4 ms, 3.8M-vertex Chung-Lu 16 -> 6.5.
+// What bounds it: the M and bitmap loads, past L2 with hubs enough (R-MAT 18
+// P5: the small block tier reads 16.6 GB in 2.7 ms, 6.2 TB/s, the large one 15.9
+// GB in 3.65 ms, which also waits for its pairs' LDS rows; the array's block
+// launch 25.9 GB in 3.4 ms), several in flight per wave.  Per edge, with q(v2)
+// counted by streaming N(v2) or by binary searches, the same counts cost R-MAT
+// 18: P5 296 -> 7.9 ms, P7 349 -> 7.8, P9 121 -> 6.6, P11 163 -> 7.8, P12 350 ->
+// 7.8; R-MAT 16 P5 28 -> 1.6; the triangle array (one intersection per edge by
+// binary searches before) R-MAT 18 20.2 -> 4.6 ms, 3.8M-vertex Chung-Lu 16 -> 8.8.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

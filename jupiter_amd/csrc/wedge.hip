@@ -41,9 +41,10 @@
 //
 // What bounds it: the latency of the list loads behind the LDS segment cursor
 // and the LDS atomics; every list is read once (R-MAT 18 P1: 8.6e8 wedges, 3.5
-// GB of list elements in 3.1 ms, 1.1 TB/s).  One wave per root with a 32 KB
+// GB of list elements in 3.2 ms, 1.1 TB/s, 7.7 GB past L2 as whole lines; a
+// bank conflict in two of three LDS cycles).  One wave per root with a 32 KB
 // table of its own held a CU to 4 waves, and roots above 16384 wedges counted
-// in global memory, twice: P1 on R-MAT 18 149 -> 3.1 ms, R-MAT 20 785 -> 17.5
+// in global memory, twice: P1 on R-MAT 18 149 -> 3.2 ms, R-MAT 20 785 -> 17.6
 // ms, 3.8M-vertex Chung-Lu 178 -> 6.2 ms.  With an intersection per pair of the
 // nest: P4 on R-MAT 14 152 -> 1.1 ms, P6 on R-MAT 11 282 -> 0.59, P8 on R-MAT 12
 // 384 -> 0.88, P10 on R-MAT 10 173 -> 0.46.
@@ -62,9 +63,9 @@ using symd::lb;
 namespace {
 
 // Waves per block, the CU's LDS holding 16 / P1_WAVES blocks: one block waits at
-// its barriers while the others work.  16 / 8 / 4 waves: R-MAT 18 3.9 / 3.1 /
-// 4.8 ms, R-MAT 20 20.9 / 17.5 / 29.2, Chung-Lu 11.4 / 10.0 / 9.8 (narrower
-// dense windows and the last split roots' tail cost the 4-wave form).
+// its barriers while the others work.  16 / 8 / 4 waves: R-MAT 18 3.8 / 3.2 /
+// 4.4 ms, R-MAT 20 20.9 / 17.6 / 29.9, 3.8M-vertex Chung-Lu 7.0 / 6.2 / 5.7
+// (narrower dense windows and the last split roots' tail cost the 4-wave form).
 constexpr int P1_WAVES = 8;
 constexpr int P1_SLICE = 2048;         // 32-bit words of LDS counters per wave task (8 KB)
 constexpr int P1_TAB = P1_SLICE * P1_WAVES;  // ... per block task
