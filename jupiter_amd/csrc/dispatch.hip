@@ -199,9 +199,9 @@ static int build_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStre
   return JGPM_OK;
 }
 
-// Makes sure of a graph's lazy arrays.  They are built on
-// the graph's own context: its stream orders the build before every later
-// reader there, and g->aux_built before the readers on other streams.  A
+// Makes sure of a graph's lazy arrays.  They are built on the graph's own
+// context: its stream orders the build before every later reader there, and
+// g->aux_pending says that a reader on another stream has to wait for it.  A
 // context that runs a query of another's graph (a serving lane) would publish
 // an array that its stream is still filling, so where one is missing it gets
 // JGPM_E_NOMEM and does without, like a query that found no room.
@@ -210,10 +210,8 @@ int ensure_sym_aux(jgpm_graph_s* g, bool need_tri, bool need_nsum, hipStream_t s
   if (g->d_src && (!need_tri || g->d_tri) && (!need_nsum || g->d_nsum)) return JGPM_OK;
   if (c != g->ctx) return JGPM_E_NOMEM;
   prof_stale(c);
-  if (!g->aux_built && hipEventCreateWithFlags(&g->aux_built, hipEventDisableTiming) != hipSuccess) return JGPM_E_HIP;
-  const int rc = build_sym_aux(g, need_tri, need_nsum, st);
-  const hipError_t e = hipEventRecord(g->aux_built, st);
-  return rc ? rc : e == hipSuccess ? JGPM_OK : JGPM_E_HIP;
+  g->aux_pending = true;
+  return build_sym_aux(g, need_tri, need_nsum, st);
 }
 
 bool pattern_uses_tri(int p) { return p == 3 || p == 4 || p == 7 || p == 10 || p == 11; }
@@ -852,7 +850,8 @@ int prepare_pattern(jgpm_graph_s* g, int pattern, int64_t rb, int64_t re) {
       }
     }
   }
-  if (hipStreamSynchronize(c->st) != hipSuccess && !rc) rc = JGPM_E_HIP;
+  if (hipStreamSynchronize(c->st) == hipSuccess) g->aux_pending = false;
+  else if (!rc) rc = JGPM_E_HIP;
   return rc;
 }
 

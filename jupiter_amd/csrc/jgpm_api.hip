@@ -434,7 +434,6 @@ extern "C" int jgpm_graph_free(jgpm_graph_t g) {
   if (g->d_tri) (void)hipFree(g->d_tri);
   if (g->d_dtri) (void)hipFree(g->d_dtri);
   if (g->d_nsum) (void)hipFree(g->d_nsum);
-  if (g->aux_built) (void)hipEventDestroy(g->aux_built);
   if (g->d_ord) (void)hipFree(g->d_ord);
   if (g->huge_d) (void)hipFree(g->huge_d);
   free_csr(g->rsym);

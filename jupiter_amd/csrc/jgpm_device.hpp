@@ -102,7 +102,7 @@ struct jgpm_graph_s {
   int32_t hubs = 0;                            // vertices of at least HUB_MIN_DEG neighbours
   int64_t tri_rows = -1;                       // widest rows of the triangle sums beyond LDS, words (-1: not known yet)
   int64_t* d_nsum = nullptr;                   // neighbour-degree sums (lazy)
-  hipEvent_t aux_built = nullptr;              // after the last build of d_src, d_tri, d_dtri or d_nsum
+  bool aux_pending = false;                    // a build of one of these may still be on the context's stream
   DevCSR rsym;                                 // symmetric CSR relabelled by d_ord (lazy, 4-cycle totals)
   int32_t* d_rsrc = nullptr;                   // ... and the source of each of its edges
   int32_t rank_min2 = 0;                       // vertices with at most one neighbour: the first ranks

@@ -186,7 +186,9 @@ static int run_heavy(jgpm_ctx_s* main, jgpm_ctx_s* lc, const Req& r, uint64_t* c
     std::lock_guard<std::mutex> gl(main->mu);
     if (!st) st = jgpm::ctx_reset_counters(lc, lc->st);
     // an array that a batch built since may still be under way on its stream
-    if (!st && r.g->aux_built && hipStreamWaitEvent(lc->st, r.g->aux_built, 0) != hipSuccess) st = JGPM_E_HIP;
+    if (!st && r.g->aux_pending &&
+        (hipEventRecord(lc->e0, main->st) != hipSuccess || hipStreamWaitEvent(lc->st, lc->e0, 0) != hipSuccess))
+      st = JGPM_E_HIP;
     if (!st) {
       jgpm::prof_reset(lc, nullptr);
       st = jgpm::enqueue_pattern(r.g, r.pattern, r.rb, r.re, 0, lc->st);
