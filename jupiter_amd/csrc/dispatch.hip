@@ -358,9 +358,9 @@ int ensure_edge_work(jgpm_graph_s* g, hipStream_t st) {
 // 1.6 ms per edge (6.5 over triangles), the first eighth 64.  P4 per edge waits
 // for one intersection after the other at an edge to a hub, about 3 us each.
 // Over ranges of 1/2 to 1/2048 of the edges at both ends and in the middle, on
-// those graphs, the route taken was at most 1.2 times slower than per edge,
-// and than the better one 2 times (a range of R-MAT 12's first roots 2.8: 0.35
-// and 0.13 ms).  A share of the edges as the line (1/8 for P9, P11, P12, 1/32 for P5,
+// those graphs, the route taken was at most 1.23 times slower than per edge
+// (P4 1.33 at 0.08 ms), and than the better one 2 times (a range of R-MAT 12's
+// first roots 2.8: 0.35 and 0.13 ms).  A share of the edges as the line (1/8 for P9, P11, P12, 1/32 for P5,
 // P7, 1/1024 for P4) was up to 4.7, 3.9 and 16 times slower than per edge.
 static int over_triangles(jgpm_graph_s* g, int p, int64_t rb, int64_t re, hipStream_t st, bool& yes) {
   const int64_t ne = g->sym_rp_h[re] - g->sym_rp_h[rb];
